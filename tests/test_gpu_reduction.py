@@ -1,0 +1,53 @@
+"""The bucket reduction (tree of joins by lane groups) at the edges of its
+shapes, through the MSM entry points, bit for bit against the oracle: windows
+whose bucket sets take one, two or three tree launches, sets of exactly one
+tile, and sets large enough for the level-1 segments. Equal and opposite points
+in neighbouring buckets make the joins meet equal operands (doubling), opposite
+ones (infinity) and infinity on either side."""
+import numpy as np
+import pytest
+
+import zyklop_amd as zk
+from tests import pyref
+from tests.test_gpu_parity import mont_pts_g1, mont_pts_g2, oracle_msm_g1, oracle_msm_g2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = zk.Context(0)
+    yield c
+    c.close()
+
+
+def scalars(vals):
+    return np.array([[(v >> (64 * i)) & (2**64 - 1) for i in range(4)] for v in vals], dtype=np.uint64)
+
+
+def cases(n):
+    """(point multiples, scalars): one point in n neighbouring buckets; the
+    same with alternating signs; full-size scalars over few points."""
+    rng = np.random.default_rng(7)
+    full = [int.from_bytes(rng.bytes(32), "little") % pyref.R for _ in range(n)]
+    yield [1] * n, list(range(1, n + 1))
+    yield [1 if i % 4 < 2 else pyref.R - 1 for i in range(n)], list(range(1, n + 1))
+    yield [1 + i % 3 for i in range(n)], full
+
+
+@pytest.mark.parametrize("window", [4, 8, 9, 15, 16, 19])
+def test_reduction_g1(ctx, window):
+    for ks, vals in cases(300):
+        pts, sc = mont_pts_g1(ks), scalars(vals)
+        expect, expect_inf = oracle_msm_g1(pts, sc)
+        got, inf = ctx.msm_g1(pts, sc, window)
+        assert inf == expect_inf and (inf or np.array_equal(got, expect))
+
+
+@pytest.mark.parametrize("window", [4, 7, 8, 13, 16, 19])
+def test_reduction_g2(ctx, window):
+    for ks, vals in cases(150):
+        pts, sc = mont_pts_g2(ks), scalars(vals)
+        expect, expect_inf = oracle_msm_g2(pts, sc)
+        got, inf = ctx.msm_g2(pts, sc, window)
+        assert inf == expect_inf and (inf or np.array_equal(got, expect))

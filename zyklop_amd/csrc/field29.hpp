@@ -18,7 +18,7 @@
 //
 // Points enter this form once per circuit (from the standard 8 x 32-bit,
 // R = 2^256 Montgomery form); the buckets stay in it through the reduction
-// and only the level-2 partials leave it, so every other kernel keeps the
+// and only the reduction's last points leave it, so every other kernel keeps the
 // standard form.
 #pragma once
 #include <stdint.h>

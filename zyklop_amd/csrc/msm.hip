@@ -1,6 +1,5 @@
 // Pippenger MSM kernels for G1/G2 on gfx950 (see msm.hpp for the design).
 #include <algorithm>
-#include <future>
 #include <mutex>
 #include <type_traits>
 
@@ -43,15 +42,48 @@ MsmGeom msm_geom(size_t n, int c, bool g2, bool merged) {
     g.merged = merged;
     g.Wr = merged ? 1 : g.W;
     g.K = 1u << (c - 1);
-    // level-1 segments: 4 G1 buckets up to 2^18 buckets in all (their
-    // chains, split-fold longer, set the reduction's latency), else 8, which
-    // keeps the level-2 partials the host combines to a few dozen per set
-    const uint32_t l1 = (!g2 && (size_t)g.Wr * g.K <= (1u << 18)) ? 4u : L1_MAX;
-    g.l1 = std::min<uint32_t>(l1, g.K);
-    g.nseg = g.K / g.l1;
-    uint32_t per_blk = (uint32_t)(g2 ? RedBlk<Fq2>::V : RedBlk<Fp>::V) * L2;
-    g.nblk = (g.nseg + per_blk - 1) / per_blk;
     return g;
+}
+
+MsmTree msm_tree(const MsmGeom& g, bool g2, int split) {
+    MsmTree t{};
+    // Level 1 first where the additions, not their depth, take the time: a
+    // group of lanes spends about 1.6 times the work of one thread on an
+    // addition. G1, 7 sets of 2^18 buckets: tree alone 0.91 ms, segments of 4
+    // 0.95 ms, of 8 0.60 ms. One set of 2^18 in batched proofs of 2^20
+    // constraints (10.5 ms each): segments of 4 1.5 % faster than the tree
+    // alone or segments of 8. Below that the tree alone: G1 2^15 buckets 45 us
+    // against 0.44 ms for segments of 4 and a block scan, G2 2^10 0.14 against
+    // 1.4 ms.
+    const size_t nb = (size_t)g.Wr * g.K;
+    t.l1 = nb >= (1u << 20) ? std::min(8u, g.K) : nb >= (1u << 18) ? std::min(4u, g.K) : 1u;
+    uint32_t C = 1;
+    t.parts = 1;
+    if (t.l1 > 1) {
+        t.nodes = g.K / t.l1;
+        t.seg = 2 * nb / t.l1;
+        C = 2;
+    } else if ((split & (split - 1)) == 0) {
+        t.plain = ilog2(split);
+        t.nodes = g.K * (uint32_t)split;
+    } else {
+        t.parts = (uint32_t)split;
+        t.nodes = g.K;
+    }
+    const int qmax = g2 ? TREE_LOG<Fq2> : TREE_LOG<Fp>;
+    int rem = ilog2(t.nodes), plain = t.plain;
+    do {   // at least one launch: it converts the points for the host
+        const int q = std::min(rem, qmax);
+        t.q[t.levels] = q;
+        C += (uint32_t)std::max(0, q - plain);
+        plain = std::max(0, plain - q);
+        rem -= q;
+        size_t& buf = t.levels & 1 ? t.node1 : t.node0;
+        buf = std::max(buf, ((size_t)g.Wr * C) << rem);
+        t.levels++;
+    } while (rem > 0);
+    t.nout = C;
+    return t;
 }
 
 int msm_table_c(size_t n) {
@@ -525,8 +557,8 @@ void MsmSort::run(const void* d_scalars, size_t n_, int c, hipStream_t st, bool 
     ZK_HIP(hipGetLastError());
 }
 
-void msm_reserve_partials(MsmPartials& out, const MsmGeom& g, bool g2) {
-    out.host.ensure(2 * (size_t)g.Wr * g.nblk * (g2 ? 256 : 128));
+void msm_reserve_partials(MsmPartials& out, const MsmGeom& g, bool g2, int split) {
+    out.host.ensure((size_t)g.Wr * msm_tree(g, g2, split).nout * (g2 ? 256 : 128));
 }
 
 void msm_points_to29(const void* d_points, size_t n, void* d_out, bool g2, hipStream_t st) {
@@ -563,10 +595,10 @@ static void scratch_buffers(S& q, const MsmGeom& g, size_t max_chunks, bool g2, 
     const size_t xb = g2 ? 256 : 128;
     const size_t nb = (size_t)g.Wr * g.K;
     f(q.buckets, nb * split * xb);
-    f(q.r1, (size_t)g.Wr * g.nseg * xb);
-    f(q.t1, (size_t)g.Wr * g.nseg * xb);
-    f(q.r2, (size_t)g.Wr * g.nblk * xb);
-    f(q.t2, (size_t)g.Wr * g.nblk * xb);
+    const MsmTree t = msm_tree(g, g2, split);
+    f(q.seg, t.seg * xb);
+    f(q.node0, t.node0 * xb);
+    f(q.node1, t.node1 * xb);
     f(q.partials, max_chunks * xb);
 }
 
@@ -609,7 +641,7 @@ static __device__ __align__(256) uint8_t scratch[MSM_NOALLOC_SCRATCH_BYTES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static std::mutex g_noalloc_mu;
 static void* g_noalloc_ptr[NOALLOC_MAX_DEVICES] = {};
-// host partials of the fixed-scratch MSM: [W][nblk] R then T, XYZZ (128 B) each
+// host partials of the fixed-scratch MSM: at most W*(c + 2) XYZZ points of 128 B
 static uint64_t g_noalloc_host[16384];
 
 void msm_noalloc_setup(int device) {
@@ -646,7 +678,7 @@ zkh::Xyzz<zkh::Fp> msm_g1_noalloc(int device, const void* d_points, const void* 
                "MSM of " + std::to_string(n) + " points at window " + std::to_string(g.c) + " needs " +
                    std::to_string(need) + " bytes of workspace; the fixed scratch holds " +
                    std::to_string(MSM_NOALLOC_SCRATCH_BYTES) + " (65536 points at the default window)");
-    const size_t host_need = 2 * (size_t)g.Wr * g.nblk * 128;
+    const size_t host_need = (size_t)g.Wr * msm_tree(g, false, split).nout * 128;
     ZK_REQUIRE(host_need <= sizeof g_noalloc_host, ZK_E_ARG, "MSM window too large for the fixed host partials");
     size_t used = 0;
     auto take = [&](DevBuf& b, size_t bytes) {
@@ -675,58 +707,34 @@ zkh::Fp load_h<zkh::Fp>(const uint64_t* p) { return zkh::Fp::from_raw(p); }
 template <>
 zkh::Fp2 load_h<zkh::Fp2>(const uint64_t* p) { return {zkh::Fp::from_raw(p), zkh::Fp::from_raw(p + 4)}; }
 
-// value of bucket set w from its level-2 partials: sum_blk (T_blk +
-// blk*U*R_blk) with U = 2^logU, by running sums over the blocks
+// The points of every set by their power of two (offset of the set's window
+// plus the bit of the bucket index), then one Horner chain from the top.
 template <class HT>
-static zkh::Xyzz<HT> window_value(const MsmPartials& p, int w) {
+static zkh::Xyzz<HT> finish_t(const MsmPartials& p) {
     const MsmGeom& g = p.g;
-    const int lw = sizeof(HT) / 8;  // u64 words per coordinate
-    const uint64_t* R = p.data();
-    const uint64_t* Tt = R + (size_t)g.Wr * g.nblk * 4 * lw;
-    const int logU = ilog2(g.l1) + ilog2(L2) + ilog2(p.g2 ? RedBlk<Fq2>::V : RedBlk<Fp>::V);
-    auto ld = [&](const uint64_t* base, size_t i) {
-        const uint64_t* q = base + i * 4 * lw;
+    const size_t lw = sizeof(HT) / 8;  // u64 words per coordinate
+    auto ld = [&](size_t i) {
+        const uint64_t* q = p.data() + i * 4 * lw;
         return zkh::Xyzz<HT>{load_h<HT>(q), load_h<HT>(q + lw), load_h<HT>(q + 2 * lw), load_h<HT>(q + 3 * lw)};
     };
-    zkh::Xyzz<HT> run = zkh::Xyzz<HT>::infinity(), acc = run, tsum = run;
-    for (int b = (int)g.nblk - 1; b >= 0; b--) {
-        acc = zkh::xyzz_add(acc, run);
-        run = zkh::xyzz_add(run, ld(R, (size_t)w * g.nblk + b));
-        tsum = zkh::xyzz_add(tsum, ld(Tt, (size_t)w * g.nblk + b));
+    const uint32_t first = p.bit0 ? 1 : 0;   // the constant's channel, the O_t after it
+    std::vector<std::vector<size_t>> at(GLV_BITS + 1);
+    int off = 0;
+    for (int w = 0; w < g.Wr; w++) {
+        at[off].push_back((size_t)w * p.nout + first);
+        for (uint32_t t = first + 1; t < p.nout; t++)
+            at[off + p.bit0 + (int)(t - first - 1)].push_back((size_t)w * p.nout + t);
+        off += w < g.nlo ? g.c - 1 : g.c;   // widths of the windows
     }
-    for (int d = 0; d < logU; d++) acc = zkh::xyzz_dbl(acc);
-    return zkh::xyzz_add(tsum, acc);
-}
-
-// window values (on `tasks` threads when > 1), then Horner across windows;
-// over window tables the one bucket set is the whole MSM
-template <class HT>
-static zkh::Xyzz<HT> finish_t(const MsmPartials& p, int tasks) {
-    const MsmGeom& g = p.g;
-    if (g.merged) return window_value<HT>(p, 0);
-    std::vector<zkh::Xyzz<HT>> S(g.W);
-    if (tasks <= 1 || g.W < 2) {
-        for (int w = 0; w < g.W; w++) S[w] = window_value<HT>(p, w);
-    } else {
-        std::vector<std::future<void>> fs;
-        for (int t = 0; t < tasks; t++)
-            fs.push_back(std::async(std::launch::async, [&, t] {
-                for (int w = t; w < g.W; w += tasks) S[w] = window_value<HT>(p, w);
-            }));
-        for (auto& f : fs) f.get();
-    }
-    // total = sum_w 2^(offset of w) S_w; window w is c - 1 bits wide below nlo
     zkh::Xyzz<HT> total = zkh::Xyzz<HT>::infinity();
-    for (int w = g.W - 1; w >= 0; w--) {
-        const int width = w < g.nlo ? g.c - 1 : g.c;
-        for (int d = 0; d < width; d++) total = zkh::xyzz_dbl(total);
-        total = zkh::xyzz_add(total, S[w]);
+    for (int b = GLV_BITS; b >= 0; b--) {
+        total = zkh::xyzz_dbl(total);
+        for (size_t i : at[b]) total = zkh::xyzz_add(total, ld(i));
     }
     return total;
 }
 
-zkh::Xyzz<zkh::Fp> msm_finish_g1(const MsmPartials& p) { return finish_t<zkh::Fp>(p, 1); }
-// G2 window values cost about 4x those of G1: spread them over 4 threads
-zkh::Xyzz<zkh::Fp2> msm_finish_g2(const MsmPartials& p) { return finish_t<zkh::Fp2>(p, 4); }
+zkh::Xyzz<zkh::Fp> msm_finish_g1(const MsmPartials& p) { return finish_t<zkh::Fp>(p); }
+zkh::Xyzz<zkh::Fp2> msm_finish_g2(const MsmPartials& p) { return finish_t<zkh::Fp2>(p); }
 
 }  // namespace zk

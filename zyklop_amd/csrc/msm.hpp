@@ -16,9 +16,10 @@
 //     9 x 29-bit-limb Montgomery form (field29.hpp) over a converted copy of
 //     the bases; oversized buckets are split into fixed chunks reduced by
 //     whole workgroups (device-side work lists, no host round trip);
-//   * bucket reduction: thread-level running sums over segments, then an LDS
-//     suffix-scan combine per workgroup; the host finishes a few points per
-//     window and runs Horner across windows;
+//   * bucket reduction: a tree of joins whose additions are all independent,
+//     each done by a group of lanes (coop29.hpp), after running sums per
+//     segment where the buckets are many; the host weighs the c points it
+//     leaves per set by powers of two, one Horner chain over all sets;
 //   * window tables for bases that stay resident (a circuit's CRS): table w
 //     holds 2^(offset of window w) * P_i for every base, so the digits of all
 //     windows go to ONE set of buckets (sum_w d_w 2^off_w P = sum_w d_w T_w).
@@ -44,10 +45,21 @@ struct MsmGeom {
     bool merged;    // all windows share one set of buckets (bases from window tables)
     int Wr;         // bucket sets: W, or 1 when merged
     uint32_t K;     // buckets per set = 2^(c-1)
-    uint32_t l1;    // buckets per level-1 reduction thread
-    uint32_t nseg;  // level-1 segments per bucket set = K / l1
-    uint32_t nblk;  // level-2 blocks per bucket set
 };
+
+// Reduction of the bucket sets (k_msm_tree, msm_kernels.hpp): what each launch
+// joins. A set ends in nout points: the tree's channels.
+struct MsmTree {
+    uint32_t l1;        // buckets per level-1 thread (k_msm_reduce1), 1: no level 1
+    uint32_t nodes;     // nodes per set that the first tree launch reads (2^any)
+    uint32_t parts;     // points per node there (a split that is no power of two)
+    int plain;          // joins that add parts of one bucket (log2 of a power-of-two split)
+    int levels;         // tree launches
+    int q[8];           // log2 of the nodes each joins
+    uint32_t nout;      // points per set at the end
+    size_t seg, node0, node1;   // points that the launches' buffers hold
+};
+MsmTree msm_tree(const MsmGeom& g, bool g2, int split);
 
 int msm_default_c(size_t n);
 // The geometry depends on the window count only: every c with the same
@@ -110,11 +122,16 @@ struct MsmSort {
              const uint8_t* cls = nullptr);
 };
 
-// Result of the device part of one MSM: level-2 partials per window, on the host.
+// Result of the device part of one MSM: the tree's last points per bucket set,
+// on the host. Set w is worth c_w + sum_t 2^(bit0 + t) O_t: after a level 1
+// (bit0 > 0) its points are R (unused), T = c_w, O_0, O_1, ..., else S = c_w,
+// O_0, O_1, ...
 struct MsmPartials {
     MsmGeom g{};
     bool g2 = false;
-    HostBuf host;       // [Wr][nblk] R then [Wr][nblk] T, XYZZ each
+    int bit0 = 0;
+    uint32_t nout = 0;
+    HostBuf host;       // [Wr][nout], XYZZ each
     // caller-owned host memory used instead of `host` when set (ext_bytes long)
     void* ext = nullptr;
     size_t ext_bytes = 0;
@@ -123,7 +140,7 @@ struct MsmPartials {
 
 // Device scratch for the bucket phase of one MSM.
 struct MsmScratch {
-    DevBuf buckets, r1, t1, r2, t2, partials;
+    DevBuf buckets, seg, node0, node1, partials;
     int split = 0;     // threads per bucket of the queued MSM (set by msm_launch_pre)
     size_t cap_buckets = 0;
     // optional events around the bucket-accumulation kernel (profiling)
@@ -169,7 +186,7 @@ void msm_points_to29(const void* d_points, size_t n, void* d_out, bool g2, hipSt
 void msm_points_table(const void* d_points, size_t n, int c, void* d_out, bool g2, hipStream_t st);
 
 // size out's host buffer for an MSM of geometry g (no launch)
-void msm_reserve_partials(MsmPartials& out, const MsmGeom& g, bool g2);
+void msm_reserve_partials(MsmPartials& out, const MsmGeom& g, bool g2, int split);
 
 // G1 MSM whose whole device workspace (29-bit base copies, digit sort,
 // buckets, reductions) lives in a fixed per-device array allocated at load

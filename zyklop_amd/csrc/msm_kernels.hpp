@@ -1,12 +1,13 @@
 // Device code shared by the per-curve MSM translation units (msm_g1.hip,
 // msm_g2.hip): constants of the bucket phase, the oversized-bucket chunk path,
-// the two reduction levels, and the launch sequence of one MSM's bucket phase,
+// the bucket reduction, and the launch sequence of one MSM's bucket phase,
 // templated on the coordinate field. msm.hip holds the digit sort and the
 // host finish.
 #pragma once
 #include <algorithm>
 #include <type_traits>
 
+#include "coop29.hpp"
 #include "curve.hpp"
 #include "field29.hpp"
 #include "glv.hpp"
@@ -16,23 +17,23 @@ namespace zk {
 
 constexpr uint32_t L_MIN_LARGE = 64;  // floor of the oversized-bucket threshold
 constexpr uint32_t CHUNK = 256 * 16;  // entries per chunk of an oversized bucket
-constexpr uint32_t L1_MAX = 8;        // buckets per level-1 reduction thread (fewer if K is smaller)
-constexpr int L2 = 4;                 // level-1 segments per level-2 thread
-constexpr int LOG_L2 = 2;
-template <class T> struct RedBlk;
-template <> struct RedBlk<Fp> { static constexpr int V = 256; };
-template <> struct RedBlk<Fq2> { static constexpr int V = 128; };
+// the tree reduction (k_msm_tree): threads per workgroup, nodes per workgroup
+// (18 KiB of LDS; one join per lane group in its first step)
+constexpr int TREE_THREADS = 256;
+template <class T> inline constexpr int TREE_LOG = 7;   // G1: 64 groups of 4 lanes
+template <> inline constexpr int TREE_LOG<Fq2> = 6;     // 32 groups of 8 lanes
+template <class T> inline constexpr int TREE_NODES = 1 << TREE_LOG<T>;
 
 struct ChunkRec { uint32_t bucket, start, len, pad; };
 struct LargeRec { uint32_t bucket, first, count, pad; };
 
-// oversized-bucket threshold floor, chunk size and level sizes are shared with
-// the sort (msm.hip), which builds the chunk lists
+// oversized-bucket threshold floor and chunk size are shared with the sort
+// (msm.hip), which builds the chunk lists
 
 // ---------------------------------------------------------------- point forms
-// Buckets, level-1 results and the level-2 working set are in the 29-bit form
-// (field29.hpp), in which the accumulation leaves its buckets; the level-2
-// partials go to the host in the standard form.
+// Buckets and the tree's nodes are in the 29-bit form (field29.hpp), in which
+// the accumulation leaves its buckets; the tree's last points go to the host in
+// the standard form.
 template <class T> struct Red;
 template <>
 struct Red<Fp> {
@@ -40,7 +41,6 @@ struct Red<Fp> {
     static constexpr int WORDS = 32;  // packed words per point (xyzz29_pack)
     ZK_DEV static Pt inf() { return xyzz29_inf(); }
     ZK_DEV static Pt add(const Pt& a, const Pt& b) { return f29_xyzz_add(a, b); }
-    ZK_DEV static Pt dbl(const Pt& a) { return f29_xyzz_dbl(a); }
     ZK_DEV static void pack(const Pt& p, uint32_t* w) { xyzz29_pack(p, w); }
     ZK_DEV static Pt unpack(const uint32_t* w) { return xyzz29_unpack(w); }
     ZK_DEV static Pt from_std(const Xyzz<Fp>& s) {
@@ -53,10 +53,6 @@ struct Red<Fp> {
         r.inf = false;
         return r;
     }
-    ZK_DEV static Xyzz<Fp> to_std(const Pt& p) {
-        if (p.inf) return xyzz_inf<Fp>();
-        return {f29_to_std(p.X), f29_to_std(p.Y), f29_to_std(p.ZZ), f29_to_std(p.ZZZ)};
-    }
 };
 template <>
 struct Red<Fq2> {
@@ -64,7 +60,6 @@ struct Red<Fq2> {
     static constexpr int WORDS = 64;  // packed words per point (xyzz29q_pack)
     ZK_DEV static Pt inf() { return xyzz29q_inf(); }
     ZK_DEV static Pt add(const Pt& a, const Pt& b) { return f29q_xyzz_add(a, b); }
-    ZK_DEV static Pt dbl(const Pt& a) { return f29q_xyzz_dbl(a); }
     ZK_DEV static void pack(const Pt& p, uint32_t* w) { xyzz29q_pack(p, w); }
     ZK_DEV static Pt unpack(const uint32_t* w) { return xyzz29q_unpack(w); }
     ZK_DEV static Pt from_std(const Xyzz<Fq2>& s) {
@@ -76,10 +71,6 @@ struct Red<Fq2> {
         r.ZZZ = f29q_from_std(s.ZZZ);
         r.inf = false;
         return r;
-    }
-    ZK_DEV static Xyzz<Fq2> to_std(const Pt& p) {
-        if (p.inf) return xyzz_inf<Fq2>();
-        return {f29q_to_std(p.X), f29q_to_std(p.Y), f29q_to_std(p.ZZ), f29q_to_std(p.ZZZ)};
     }
 };
 
@@ -242,18 +233,18 @@ __global__ void __launch_bounds__(CHUNK_THREADS) k_msm_merge(const uint32_t* __r
 }
 
 // ---------------------------------------------------------------- reduction
-// Arithmetic in the 29-bit form (Red<T>). The point additions are inlined,
-// each loop body holding one or two addition sites (level 2 selects its operands per step; the step index is
-// uniform across the wave): out-of-line calls would pass the 128/256-byte
-// operands through scratch memory on every step of these latency-bound chains.
+// Arithmetic in the 29-bit form. The point additions are inlined, each loop
+// body holding one or two addition sites: out-of-line calls would pass the
+// operands through scratch memory on every step of these chains.
 //
-// Level 1: thread j owns buckets [j*L1, (j+1)*L1) of one window; with bucket
-// b holding digit b+1: R_j = sum B_b, T_j = sum (b - j*L1 + 1) B_b, so the
-// window value is sum_j (T_j + j*L1*R_j). B_b is the sum of the bucket's
-// `split` slots from the accumulation.
+// Level 1 of large bucket sets: thread j owns buckets [j*L1, (j+1)*L1) of one
+// window; with bucket b holding digit b+1: R_j = sum B_b, T_j = sum (b - j*L1
+// + 1) B_b, so the window value is sum_j (T_j + j*L1*R_j). B_b is the sum of
+// the bucket's `split` slots from the accumulation. out: [W][R, T][K/L1], the
+// two channels of the tree's nodes.
 template <class T>
 __global__ void __launch_bounds__(128) k_msm_reduce1(const void* __restrict__ buckets, uint32_t K, int W, uint32_t L1,
-                                                     uint32_t split, void* __restrict__ R, void* __restrict__ Tt) {
+                                                     uint32_t split, void* __restrict__ out) {
     using P = Red<T>;
     uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t nseg = K / L1;
@@ -267,77 +258,94 @@ __global__ void __launch_bounds__(128) k_msm_reduce1(const void* __restrict__ bu
         for (uint32_t h = 0; h < split; h++) run = P::add(run, red_load<T>(buckets, (base + b) * split + h));
         acc = P::add(acc, run);
     }
-    red_store<T>(R, j, run);
-    red_store<T>(Tt, j, acc);
+    red_store<T>(out, (size_t)w * 2 * nseg + jj, run);
+    red_store<T>(out, ((size_t)w * 2 + 1) * nseg + jj, acc);
 }
 
-// Level 2: input per window is M pairs (R_j, T_j) worth sum_j (T_j + j*U*R_j),
-// U = 2^logU. Block blk covers j in [blk*BLK*L2, (blk+1)*BLK*L2); thread t owns
-// L2 consecutive j. Per thread: run = sum R_j, acc = sum (j - j0) R_j,
-// tsum = sum T_j. With S_t = sum_{t' >= t} run_t' (suffix scan over the block),
-// sum_t t*run_t = sum_{t >= 1} S_t, so the block's value relative to j_blk is
-// sum_t V_t with V_t = tsum_t + U*(acc_t + L2*[t >= 1]*S_t): one tree sum.
-// Output per block: R'' = S_0 and T'' = sum_t V_t, so the window value is
-// sum_blk (T''_blk + blk * (U*L2*BLK) * R''_blk).
-template <class T, int BLK>
-__global__ void __launch_bounds__(BLK) k_msm_reduce2(const void* __restrict__ Rin, const void* __restrict__ Tin, uint32_t M,
-                                                     int logU, uint32_t nblk, void* __restrict__ Rout,
-                                                     void* __restrict__ Tout) {
-    using P = Red<T>;
-    using Pt = typename P::Pt;
-    __shared__ Pt sh[BLK];
-    const int t = threadIdx.x;
-    const uint32_t w = blockIdx.x / nblk, blk = blockIdx.x - w * nblk;
-    const uint32_t j0 = (blk * BLK + t) * L2;
-    Pt run = P::inf(), acc = P::inf(), tsum = P::inf();
-    // per item, highest j first: acc += run; run += R_j; tsum += T_j
+// Tree over the nodes of every bucket set, in groups of lanes (coop29.hpp).
+// A node covers 2^j consecutive buckets and holds points by channel: 0 its
+// plain sum S, then sums that only add up, among them O_t, the sum of its
+// buckets whose index has bit t set. Joining a left and a right node adds
+// channel by channel, and S of the right node is the new O_j: nothing but
+// independent additions, 2K of them for K buckets in a depth of log2 K (a
+// running sum per segment takes as many, two dependent ones per bucket), and
+// no doubling on the device: the host weighs the O_t by 2^t.
+//
+// The workgroup (x, y) takes the 2^q nodes x * 2^q.. of channel c = y mod C of
+// set y / C (input [set][c][N]), joins them in LDS and writes one node to
+// [set][c][N >> q]; channel 0 also makes the O_t of the joins' bits, `plain`
+// joins first being parts of one bucket (they make none), as channels C, C +
+// 1, ... of the Cout output channels. Every entry may come in `parts`
+// consecutive points. O_t of the node at i lies where S of its right half was
+// joined, at i + 2^t. last: to the standard form, for the host.
+//
+// Bound by the depth of the additions (2.3 us each for a lone wave, G2 about
+// 4.5 us) up to about 2^16 buckets, by instruction issue above. Measured alone,
+// all launches: G1 2^15 buckets 45 us, 2^17 100 us, 2^18 in 3 parts 243 us; G2
+// 10 sets of 2^12 138 us, 2^12 in 3 parts 0.14 ms. The level-1 segments with a
+// suffix scan and a tree sum over one workgroup per 1024 segments that this
+// replaced took 0.43, 0.52, 0.56, 1.31 and 1.42 ms.
+template <class T>
+__global__ void __launch_bounds__(TREE_THREADS) k_msm_tree(const void* __restrict__ in, uint32_t N, uint32_t C,
+                                                           uint32_t parts, int plain, int q, int last, uint32_t Cout,
+                                                           void* __restrict__ out) {
+    constexpr int L = Coop<T>::LANES, G = TREE_THREADS / L;
+    __shared__ uint32_t sh[TREE_NODES<T> * L * 9];
+    const uint32_t lane = threadIdx.x % L, grp = threadIdx.x / L;
+    const Coop<T> k(lane);
+    // place of this lane's coordinate in a packed point: c0 before c1
+    const uint32_t word4 = 2 * ((lane & 3) * (L / 4) + (lane >> 2));
+    const uint32_t set = blockIdx.y / C, c = blockIdx.y - set * C, nodes = 1u << q;
+    const uint4* src = reinterpret_cast<const uint4*>(in) + word4 +
+                       (size_t)(Red<T>::WORDS / 4) * parts * ((size_t)blockIdx.y * N + ((size_t)blockIdx.x << q));
+    auto ld = [&](uint32_t i) {
+        F29 v;
+#pragma unroll
+        for (int l = 0; l < 9; l++) v.l[l] = sh[(i * L + lane) * 9 + l];
+        return v;
+    };
+    auto st = [&](uint32_t i, const F29& v) {
+#pragma unroll
+        for (int l = 0; l < 9; l++) sh[(i * L + lane) * 9 + l] = v.l[l];
+    };
+    for (uint32_t i = grp; i < nodes; i += G) {
+        F29 v = f29_load_packed(src + (size_t)(Red<T>::WORDS / 4) * parts * i);
 #pragma unroll 1
-    for (int step = 0; step < 3 * L2; step++) {
-        const int q = L2 - 1 - step / 3, k = step % 3;
-        const uint32_t j = j0 + q;
-        if (j >= M) continue;
-        Pt x = k == 0 ? acc : (k == 1 ? run : tsum);
-        Pt y = k == 0 ? run : red_load<T>(k == 1 ? Rin : Tin, (size_t)w * M + j);
-        Pt r = P::add(x, y);
-        if (k == 0) acc = r;
-        else if (k == 1) run = r;
-        else tsum = r;
+        for (uint32_t h = 1; h < parts; h++)
+            v = coop_add<T>(k, v, f29_load_packed(src + (size_t)(Red<T>::WORDS / 4) * (parts * i + h)));
+        st(i, v);
     }
-    // suffix scan of run across the block: S_t = sum_{t' >= t} run_t'
-    sh[t] = run;
 #pragma unroll 1
-    for (int d = 1; d < BLK; d <<= 1) {
+    for (int j = 0; j < q; j++) {
         __syncthreads();
-        Pt mine = sh[t];
-        Pt other = (t + d < BLK) ? sh[t + d] : P::inf();
-        __syncthreads();
-        sh[t] = P::add(mine, other);
-    }
-    __syncthreads();
-    const Pt S = sh[t], total_r = sh[0];
-    __syncthreads();
-    // V_t = tsum + U * (acc + L2 * [t >= 1] * S_t): doublings and additions
-    // through one site each
-    Pt v = t >= 1 ? S : P::inf();
+        const int lp = q - 1 - j;   // 2^lp joins
+        const uint32_t bits = c == 0 && j > plain ? (uint32_t)(j - plain) : 0u;
+        const uint32_t tasks = (1u + bits) << lp;
 #pragma unroll 1
-    for (int step = 0; step < LOG_L2 + 1 + logU + 1; step++) {
-        if (step < LOG_L2 || (step > LOG_L2 && step <= LOG_L2 + logU)) {
-            v = P::dbl(v);
-        } else {
-            v = P::add(v, step == LOG_L2 ? acc : tsum);
+        for (uint32_t t = grp; t < tasks; t += G) {
+            const uint32_t b = t >> lp;   // 0: S; b >= 1: O of the join plain + b - 1
+            const uint32_t l = ((t & ((1u << lp) - 1)) << (j + 1)) + (b ? 1u << (plain + b - 1) : 0u);
+            st(l, coop_add<T>(k, ld(l), ld(l + (1u << j))));
         }
     }
-    // tree sum of V over the block
-    sh[t] = v;
-#pragma unroll 1
-    for (int h = BLK >> 1; h >= 1; h >>= 1) {
-        __syncthreads();
-        if (t < h) sh[t] = P::add(sh[t], sh[t + h]);
-    }
     __syncthreads();
-    if (t == 0) {
-        PointIO<T>::store_xyzz(Rout, blockIdx.x, P::to_std(total_r));
-        PointIO<T>::store_xyzz(Tout, blockIdx.x, P::to_std(sh[0]));
+    // outputs: the channel itself, and for channel 0 the new O_t
+    const uint32_t nout = 1u + (c == 0 && q > plain ? (uint32_t)(q - plain) : 0u);
+    for (uint32_t o = grp; o < nout; o += G) {
+        const F29 v = ld(o ? 1u << (plain + o - 1) : 0u);
+        uint32_t w[8];
+        if (last) {
+            const Fp s = f29_to_std(v);
+#pragma unroll
+            for (int i = 0; i < 8; i++) w[i] = s.v[i];
+        } else {
+            f29_pack(f29_reduce(v), w);   // X may be above 2^256
+        }
+        uint4* dst = reinterpret_cast<uint4*>(out) + word4 +
+                     (size_t)(Red<T>::WORDS / 4) *
+                         (((size_t)set * Cout + (o ? C + o - 1 : c)) * (N >> q) + blockIdx.x);
+        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
     }
 }
 
@@ -386,27 +394,43 @@ static void launch_main_t(const MsmSort& sort, const void* d_points29, MsmScratc
     launch_accum<T>(sort, nb, split, d_points29, scr.buckets.p, st, range);
     ZK_HIP(hipGetLastError());
     if (scr.ev_acc1) ZK_HIP(hipEventRecord(scr.ev_acc1, st));
-    uint32_t nseg_all = (uint32_t)g.Wr * g.nseg;
-    k_msm_reduce1<T><<<cdiv(nseg_all, 128), 128, 0, st>>>(scr.buckets.p, g.K, g.Wr, g.l1, (uint32_t)split, scr.r1.p,
-                                                           scr.t1.p);
-    ZK_HIP(hipGetLastError());
-    constexpr int BLK = RedBlk<T>::V;
-    k_msm_reduce2<T, BLK><<<(unsigned)(g.Wr * g.nblk), BLK, 0, st>>>(scr.r1.p, scr.t1.p, g.nseg, ilog2(g.l1), g.nblk,
-                                                                      scr.r2.p, scr.t2.p);
-    ZK_HIP(hipGetLastError());
-    size_t xb = g2 ? 256 : 128;
-    size_t half = (size_t)g.Wr * g.nblk * xb;
+    const MsmTree t = msm_tree(g, g2, split);
+    const void* in = scr.buckets.p;
+    if (t.l1 > 1) {
+        k_msm_reduce1<T><<<cdiv((size_t)g.Wr * (g.K / t.l1), 128), 128, 0, st>>>(scr.buckets.p, g.K, g.Wr, t.l1,
+                                                                                 (uint32_t)split, scr.seg.p);
+        ZK_HIP(hipGetLastError());
+        in = scr.seg.p;
+    }
+    uint32_t N = t.nodes, C = t.l1 > 1 ? 2 : 1, parts = t.parts;
+    int plain = t.plain;
+    DevBuf* dst[2] = {&scr.node0, &scr.node1};
+    for (int lev = 0; lev < t.levels; lev++) {
+        const int q = t.q[lev];
+        const uint32_t Cout = C + (uint32_t)std::max(0, q - plain);
+        k_msm_tree<T><<<dim3(N >> q, (unsigned)g.Wr * C), TREE_THREADS, 0, st>>>(in, N, C, parts, plain, q,
+                                                                               lev == t.levels - 1, Cout,
+                                                                               dst[lev & 1]->p);
+        ZK_HIP(hipGetLastError());
+        in = dst[lev & 1]->p;
+        N >>= q;
+        C = Cout;
+        parts = 1;
+        plain = std::max(0, plain - q);
+    }
+    const size_t bytes = (size_t)g.Wr * t.nout * (g2 ? 256 : 128);
     out.g = g;
     out.g2 = g2;
-    void* dst = out.ext;
-    if (dst) {
-        ZK_REQUIRE(out.ext_bytes >= 2 * half, ZK_E_INTERNAL, "MSM partials exceed the caller's host buffer");
+    out.bit0 = ilog2(t.l1);
+    out.nout = t.nout;
+    void* to = out.ext;
+    if (to) {
+        ZK_REQUIRE(out.ext_bytes >= bytes, ZK_E_INTERNAL, "MSM partials exceed the caller's host buffer");
     } else {
-        out.host.ensure(2 * half);
-        dst = out.host.p;
+        out.host.ensure(bytes);
+        to = out.host.p;
     }
-    ZK_HIP(hipMemcpyAsync(dst, scr.r2.p, half, hipMemcpyDeviceToHost, st));
-    ZK_HIP(hipMemcpyAsync((char*)dst + half, scr.t2.p, half, hipMemcpyDeviceToHost, st));
+    ZK_HIP(hipMemcpyAsync(to, in, bytes, hipMemcpyDeviceToHost, st));
     if (scr.ev_end) ZK_HIP(hipEventRecord(scr.ev_end, st));
 }
 

@@ -380,7 +380,7 @@ size_t ProveSlot::device_bytes() const {
              q->order.bytes + q->lkeys.bytes + q->chunks.bytes + q->large.bytes + q->counters.bytes + q->cls_off.bytes +
              q->order_a.bytes + q->order_b.bytes + q->okeys.bytes;
     for (const MsmScratch* s : {&scrA, &scrB1, &scrC, &scrB2, &scrH})
-        b += s->buckets.bytes + s->r1.bytes + s->t1.bytes + s->r2.bytes + s->t2.bytes + s->partials.bytes;
+        b += s->buckets.bytes + s->seg.bytes + s->node0.bytes + s->node1.bytes + s->partials.bytes;
     return b;
 }
 
@@ -414,9 +414,9 @@ void ProveSlot::reserve(Context& ctx, const Circuit& c, bool host_witness) {
     for (MsmScratch* q : {&scrA, &scrB1, &scrC}) q->ensure(gw1, kw, false, pl.sp_w1);
     scrB2.ensure(gw2, kw, true, pl.sp_w2);
     scrH.ensure(gh, kh, false, pl.sp_h);
-    for (MsmPartials* q : {&parts.a, &parts.b1, &parts.c}) msm_reserve_partials(*q, gw1, false);
-    msm_reserve_partials(parts.b2, gw2, true);
-    msm_reserve_partials(parts.h, gh, false);
+    for (MsmPartials* q : {&parts.a, &parts.b1, &parts.c}) msm_reserve_partials(*q, gw1, false, pl.sp_w1);
+    msm_reserve_partials(parts.b2, gw2, true, pl.sp_w2);
+    msm_reserve_partials(parts.h, gh, false, pl.sp_h);
 }
 
 void ProveSlot::enqueue(Context& ctx, const Circuit& c, const uint64_t* witness, bool on_dev, const uint64_t r_[4],

@@ -71,7 +71,7 @@ struct Circuit {
 // first: no proof of c may be in flight.
 void circuit_set_tables(Circuit& c, int mode);
 
-// Device results of one proof's five MSMs (level-2 partials, host memory).
+// Device results of one proof's five MSMs (the reduction's last points, host memory).
 struct ProofParts {
     MsmPartials a, b1, c, b2, h;
 };
