@@ -23,6 +23,7 @@ struct zk_server;
 struct zk_ctx {
     zk::Context impl;
     std::vector<std::unique_ptr<zk::ProveSlot>> batch_slots;
+    zk::MsmWorkspace msm_ws;   // of the MSM entry points, which hold impl.mu
     // servers created on this context: destroying the context finishes and
     // detaches them first (their worker threads use the context)
     std::mutex servers_mu;
@@ -144,6 +145,27 @@ void put_result(const zkh::Xyzz<HT>& p, uint64_t* out, int* is_inf) {
     memcpy(out + lw, &a.y, 8 * lw);
 }
 
+// the context's workspace for one call, or one of the call's own while another
+// thread takes the context's back
+struct WorkspaceUse {
+    std::unique_ptr<zk::MsmWorkspace> own;
+    zk::MsmWorkspace* w;
+    hipStream_t st;
+    WorkspaceUse(zk::MsmWorkspace& kept, hipStream_t s) : w(&kept), st(s) {
+        if (kept.busy.exchange(true)) {
+            own = std::make_unique<zk::MsmWorkspace>();
+            w = own.get();
+            w->busy = true;
+        }
+    }
+    ~WorkspaceUse() {
+        // a call that failed may have left work queued on the buffers
+        if (std::uncaught_exceptions()) (void)hipStreamSynchronize(st);
+        if (w->bytes() > zk::MSM_KEEP_BYTES || std::uncaught_exceptions()) w->release();
+        w->busy = false;
+    }
+};
+
 // MSM over device points; slots29, when given, are the points' 29-bit slots
 // already made (a circuit's resident arrays, W window tables when merged)
 // cls / range: scalar classes and the part of every bucket to read, as a
@@ -154,12 +176,13 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
                 int range = zk::MSM_RANGE_ALL, int split = 0) {
     zk::Context& C = ctx->impl;
     hipStream_t st = C.stream;
-    zk::MsmSort sort;
-    zk::MsmScratch scr;
-    zk::MsmPartials part;
+    WorkspaceUse use(ctx->msm_ws, st);
+    zk::MsmSort& sort = use.w->sort;
+    zk::MsmScratch& scr = use.w->scr;
+    zk::MsmPartials& part = use.w->part;
     scr.enable_timing();
     // buckets are accumulated in the 29-bit-limb form: convert the points first
-    zk::DevBuf p29;
+    zk::DevBuf& p29 = use.w->p29;
     if (n && !slots29) {
         p29.ensure(n * (g2 ? zk::PT29Q_BYTES : zk::PT29_BYTES));
         zk::msm_points_to29(d_points, n, p29.p, g2, st);
@@ -171,15 +194,16 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
     zk::msm_launch_pre(sort, pts, g2, scr, st, split > 0 ? split : zk::msm_default_split(n, sort.g.c, g2, merged));
     zk::msm_launch_main(sort, g2, scr, part, st, pts, range);
     ZK_HIP(hipEventRecord(ctx->ev2, st));
+    const size_t nb = (size_t)sort.g.Wr * sort.g.K;
+    use.w->entries.ensure(4);
+    ZK_HIP(hipMemcpyAsync(use.w->entries.p, sort.offsets.as<uint32_t>() + nb, 4, hipMemcpyDeviceToHost, st));
     ZK_HIP(hipStreamSynchronize(st));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[0], ctx->ev0, ctx->ev2));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[1], ctx->ev0, ctx->ev1));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[2], scr.ev_acc0, scr.ev_acc1));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[4], scr.ev_acc1, scr.ev_end));
     // entries the accumulation read: the sort's, or the parts of the range
-    const size_t nb = (size_t)sort.g.Wr * sort.g.K;
-    uint32_t entries = 0;
-    ZK_HIP(hipMemcpy(&entries, sort.offsets.as<uint32_t>() + nb, 4, hipMemcpyDeviceToHost));
+    uint32_t entries = *use.w->entries.as<uint32_t>();
     if (sort.classes && range != zk::MSM_RANGE_ALL) {
         std::vector<uint32_t> off(nb + 1), co(3 * nb);
         ZK_HIP(hipMemcpy(off.data(), sort.offsets.p, 4 * (nb + 1), hipMemcpyDeviceToHost));
@@ -846,7 +870,7 @@ int zk_dev_alloc(zk_ctx* ctx, size_t bytes, void** out) {
         need(ctx && out, "NULL argument");
         ZK_HIP(hipSetDevice(ctx->impl.device));
         void* p = nullptr;
-        hipError_t e = hipMalloc(&p, bytes ? bytes : 256);
+        hipError_t e = zk::device_malloc(&p, bytes ? bytes : 256);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             throw zk::Error(ZK_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));

@@ -32,6 +32,26 @@ struct Error : std::runtime_error {
         if (!(cond)) throw ::zk::Error((code), (msg));      \
     } while (0)
 
+// Gives back the idle MSM workspaces that contexts keep (MsmWorkspace,
+// msm.hpp): they count as free memory. Called where an allocation failed,
+// before it is tried again, and by free_device_bytes().
+void release_idle_workspaces();
+
+// hipMalloc that takes back idle workspaces before it gives up
+inline hipError_t device_malloc(void** p, size_t n) {
+    hipError_t e = hipMalloc(p, n);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    release_idle_workspaces();
+    return hipMalloc(p, n);
+}
+
+// free and total bytes of the current device
+inline void free_device_bytes(size_t* free_b, size_t* total_b) {
+    release_idle_workspaces();
+    ZK_HIP(hipMemGetInfo(free_b, total_b));
+}
+
 // Device allocation: owning (hipMalloc), or borrowed from memory the caller
 // manages (borrow()), which never grows and is never freed here.
 struct DevBuf {
@@ -62,7 +82,7 @@ struct DevBuf {
         if (borrowed) throw Error(ZK_E_INTERNAL, "a borrowed device buffer cannot grow");
         release();
         if (n == 0) n = 256;
-        hipError_t e = hipMalloc(&p, n);
+        hipError_t e = device_malloc(&p, n);
         if (e != hipSuccess) {
             p = nullptr;
             (void)hipGetLastError();

@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
+#include <vector>
 
 #include "msm_kernels.hpp"
 #include "qap.hpp"
@@ -588,6 +589,58 @@ MsmScratch::~MsmScratch() {
     if (ev_acc0) (void)hipEventDestroy(ev_acc0);
     if (ev_acc1) (void)hipEventDestroy(ev_acc1);
     if (ev_end) (void)hipEventDestroy(ev_end);
+}
+
+static DevBuf MsmSort::* const SORT_BUFS[] = {
+    &MsmSort::half, &MsmSort::matrix, &MsmSort::mscan, &MsmSort::pairs, &MsmSort::offsets, &MsmSort::entries,
+    &MsmSort::order, &MsmSort::lkeys, &MsmSort::cls_off, &MsmSort::order_a, &MsmSort::order_b, &MsmSort::okeys,
+    &MsmSort::chunks, &MsmSort::large, &MsmSort::counters};
+static DevBuf MsmScratch::* const SCRATCH_BUFS[] = {&MsmScratch::buckets, &MsmScratch::seg, &MsmScratch::node0,
+                                                          &MsmScratch::node1, &MsmScratch::partials};
+
+size_t MsmSort::bytes() const {
+    size_t b = 0;
+    for (auto m : SORT_BUFS) b += (this->*m).bytes;
+    return b;
+}
+
+size_t MsmScratch::bytes() const {
+    size_t b = 0;
+    for (auto m : SCRATCH_BUFS) b += (this->*m).bytes;
+    return b;
+}
+
+// ---------------------------------------------------------------- workspaces
+static std::mutex g_ws_mu;
+static std::vector<MsmWorkspace*>& workspaces() {
+    static std::vector<MsmWorkspace*> v;
+    return v;
+}
+
+MsmWorkspace::MsmWorkspace() {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    workspaces().push_back(this);
+}
+
+MsmWorkspace::~MsmWorkspace() {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    auto& v = workspaces();
+    v.erase(std::find(v.begin(), v.end(), this));
+}
+
+void MsmWorkspace::release() {
+    for (auto m : SORT_BUFS) (sort.*m).release();
+    for (auto m : SCRATCH_BUFS) (scr.*m).release();
+    p29.release();
+}
+
+void release_idle_workspaces() {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    for (MsmWorkspace* w : workspaces()) {
+        if (w->busy.exchange(true)) continue;
+        w->release();
+        w->busy = false;
+    }
 }
 
 template <class S, class F>

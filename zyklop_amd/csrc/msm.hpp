@@ -29,6 +29,7 @@
 #pragma once
 #include <stdint.h>
 
+#include <atomic>
 #include <vector>
 
 #include "common.hpp"
@@ -120,6 +121,7 @@ struct MsmSort {
     // classes (optional)
     void run(const void* d_scalars, size_t n, int c, hipStream_t st, bool merged = false,
              const uint8_t* cls = nullptr);
+    size_t bytes() const;   // device bytes held
 };
 
 // Result of the device part of one MSM: the tree's last points per bucket set,
@@ -150,6 +152,29 @@ struct MsmScratch {
     void ensure(const MsmGeom& g, size_t max_chunks, bool g2, int split);
     // the device bytes ensure() would add now (into gc)
     void count_ensure(const MsmGeom& g, size_t max_chunks, bool g2, int split, GrowCount& gc) const;
+    size_t bytes() const;   // device bytes held
+};
+
+// What one MSM over caller-owned points works in, kept by a context from one
+// call to the next: allocating and freeing it took up to as long as the MSM (G1
+// calls of 2^22 points 8.5 -> 6.2 ms, of 700001 4.4 -> 1.9, of 1000 0.61 ->
+// 0.54; G2 of 200003 2.9 -> 1.9). A
+// context keeps at most MSM_KEEP_BYTES of device memory (enough for 2^22 G1
+// points); a larger workspace is freed when its call ends, an idle one when an
+// allocation of the library fails, when free memory is asked for, and with its
+// context. busy: in use by a call, or being released.
+constexpr size_t MSM_KEEP_BYTES = (size_t)2 << 30;
+struct MsmWorkspace {
+    MsmSort sort;
+    MsmScratch scr;
+    MsmPartials part;
+    DevBuf p29;         // the points' 29-bit slots
+    HostBuf entries;    // the sort's entry count
+    std::atomic<bool> busy{false};
+    MsmWorkspace();
+    ~MsmWorkspace();
+    size_t bytes() const { return sort.bytes() + scr.bytes() + p29.bytes; }
+    void release();     // frees the device buffers
 };
 
 // Launch bucket accumulation + GPU reduction against a finished sort; queue

@@ -189,7 +189,7 @@ void circuit_set_tables(Circuit& c, int mode) {
     if (mode < 0) {
         const size_t extra = (size_t)(Ww - 1) * ne * (3 * PT29_BYTES + PT29Q_BYTES) + (size_t)(Wh - 1) * n * PT29_BYTES;
         size_t free_b = 0, total_b = 0;
-        ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+        free_device_bytes(&free_b, &total_b);
         // tables the circuit holds now are freed before the new ones are made
         const size_t held = c.A29.bytes + c.B1_29.bytes + c.C29.bytes + c.B2_29.bytes + c.H29.bytes;
         const size_t base = ne * (3 * PT29_BYTES + PT29Q_BYTES) + n * PT29_BYTES;
@@ -375,12 +375,8 @@ ProveSlot::~ProveSlot() {
 
 size_t ProveSlot::device_bytes() const {
     size_t b = scal.bytes + aw.bytes + bw.bytes + cw.bytes + t0.bytes + t1.bytes + t2.bytes + h.bytes;
-    for (const MsmSort* q : {&sortW, &sortH})
-        b += q->half.bytes + q->matrix.bytes + q->mscan.bytes + q->pairs.bytes + q->offsets.bytes + q->entries.bytes +
-             q->order.bytes + q->lkeys.bytes + q->chunks.bytes + q->large.bytes + q->counters.bytes + q->cls_off.bytes +
-             q->order_a.bytes + q->order_b.bytes + q->okeys.bytes;
-    for (const MsmScratch* s : {&scrA, &scrB1, &scrC, &scrB2, &scrH})
-        b += s->buckets.bytes + s->seg.bytes + s->node0.bytes + s->node1.bytes + s->partials.bytes;
+    for (const MsmSort* q : {&sortW, &sortH}) b += q->bytes();
+    for (const MsmScratch* q : {&scrA, &scrB1, &scrC, &scrB2, &scrH}) b += q->bytes();
     return b;
 }
 

@@ -50,7 +50,7 @@ uint64_t Server::admit_request(std::shared_ptr<ServerRequest> req, const Circuit
     if (s) memcpy(req->s, s, 32);
     ZK_REQUIRE(zkh::Fr::is_canonical(req->r) && zkh::Fr::is_canonical(req->s), ZK_E_ARG, "blinding must be canonical");
     size_t free_b = 0, total_b = 0;
-    ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_device_bytes(&free_b, &total_b);
     size_t need;
     {
         std::lock_guard<std::mutex> g(ctx_.mu);
@@ -97,14 +97,14 @@ int Server::prepare(const Circuit* const* cs, int count) {
             size_t need = 0;
             for (const Circuit* c : order) need = std::max(need, ProveSlot::bytes_needed(ctx_, *c));
             size_t free_b = 0, total_b = 0;
-            ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+            free_device_bytes(&free_b, &total_b);
             if (k > 0 && free_b < need + reserve_) break;
             slots_.push_back(std::make_unique<ProveSlot>());
             running_.push_back(nullptr);
         }
         for (const Circuit* c : order) {
             size_t free_b = 0, total_b = 0;
-            ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+            free_device_bytes(&free_b, &total_b);
             ZK_REQUIRE(free_b >= slots_[k]->grow_bytes(ctx_, *c) + reserve_, ZK_E_NOMEM,
                        "not enough free device memory to prepare a slot above the reserve");
             slots_[k]->reserve(ctx_, *c, true);
@@ -211,7 +211,7 @@ bool Server::try_admit(std::unique_lock<std::mutex>& lk) {
             if (!running_[i] && grow(i) == 0) pick = (int)i;
         if (pick < 0) {
             size_t free_b = 0, total_b = 0;
-            ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+            free_device_bytes(&free_b, &total_b);
             size_t need;
             {
                 std::lock_guard<std::mutex> g(ctx_.mu);
