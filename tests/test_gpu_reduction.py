@@ -51,3 +51,15 @@ def test_reduction_g2(ctx, window):
         expect, expect_inf = oracle_msm_g2(pts, sc)
         got, inf = ctx.msm_g2(pts, sc, window)
         assert inf == expect_inf and (inf or np.array_equal(got, expect))
+
+
+@pytest.mark.parametrize("g2,n", [(False, 40), (False, 1500), (True, 40), (True, 600)])
+def test_many_parts_per_bucket(ctx, g2, n):
+    """Few buckets, so that each is accumulated in 2 to 64 parts (joined before
+    any bit of the bucket index): the smallest window, all scalars full size."""
+    three = (mont_pts_g2 if g2 else mont_pts_g1)([1, 2, pyref.R - 3])
+    pts, sc = np.ascontiguousarray(three[np.arange(n) % 3]), zk.synth_uniform(5, n)
+    expect, expect_inf = (oracle_msm_g2 if g2 else oracle_msm_g1)(pts, sc)
+    for window in (4, 5):
+        got, inf = (ctx.msm_g2 if g2 else ctx.msm_g1)(pts, sc, window)
+        assert inf == expect_inf and np.array_equal(got, expect)

@@ -191,7 +191,7 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
     sort.run(d_scalars, n, window, st, merged, cls);
     ZK_HIP(hipEventRecord(ctx->ev1, st));
     const void* pts = slots29 ? slots29 : p29.p;
-    zk::msm_launch_pre(sort, pts, g2, scr, st, split > 0 ? split : zk::msm_default_split(n, sort.g.c, g2, merged));
+    zk::msm_launch_pre(sort, pts, g2, scr, st, split > 0 ? split : zk::msm_alone_split(n, sort.g.c, g2));
     zk::msm_launch_main(sort, g2, scr, part, st, pts, range);
     ZK_HIP(hipEventRecord(ctx->ev2, st));
     const size_t nb = (size_t)sort.g.Wr * sort.g.K;

@@ -30,6 +30,24 @@ int msm_default_split(size_t n, int c, bool g2, bool merged) {
     return (int)std::max<size_t>(1, std::min<size_t>(3, target / nb));
 }
 
+// Nothing else runs beside an MSM of its own, so its accumulation takes up to
+// half a million threads (two rounds of the resident waves for G1, four for G2)
+// while every part keeps about two entries: the chain of entries per thread,
+// about 10 us each in a GPU that is not full, gets shorter, and more rounds of
+// waves even out their lengths. Each part costs one addition in the tree.
+// Against at most 3 threads per bucket (other limits in brackets): G1 1000 points 0.52 -> 0.33 ms, 20000 0.48 -> 0.37, 100000 0.61 -> 0.51
+// (2^17 0.61, 2^20 0.57), 400000 and more unchanged; G2 1000 1.10 -> 0.57,
+// 200003 1.88 -> 1.41 (2^18 1.62, 2^20 1.58). In proofs, where five MSMs share
+// the GPU, the extra additions cost more than they give (8 proofs of 50021
+// constraints 6.6 ms at 3 threads, 7.1 at 8, 8.4 at 16).
+int msm_alone_split(size_t n, int c, bool g2) {
+    const MsmGeom g = msm_geom(n, c, g2);
+    const size_t nb = (size_t)g.Wr * g.K, load = 2 * n * (size_t)g.W / nb;
+    int s = 1;
+    while (s < MSM_SPLIT_MAX && nb * s * 2 <= (1u << 19) && load >= (size_t)s * 4) s *= 2;
+    return s >= 4 ? s : msm_default_split(n, c, g2);
+}
+
 MsmGeom msm_geom(size_t n, int c, bool g2, bool merged) {
     if (c <= 0) c = msm_default_c(n);
     ZK_REQUIRE(c >= 4 && c <= 22, ZK_E_ARG, "MSM window must be in [4, 22]");
@@ -664,7 +682,7 @@ void MsmScratch::count_ensure(const MsmGeom& g, size_t max_chunks, bool g2, int 
 }
 
 void msm_launch_pre(const MsmSort& sort, const void* d_points29, bool g2, MsmScratch& scr, hipStream_t st, int split) {
-    ZK_REQUIRE(split >= 1 && split <= MSM_SPLIT_MAX, ZK_E_ARG, "bucket split must be in [1, 4]");
+    ZK_REQUIRE(split >= 1 && split <= MSM_SPLIT_MAX, ZK_E_ARG, "bucket split out of range");
     ZK_REQUIRE(sort.n == 0 || d_points29, ZK_E_INTERNAL, "MSM launch without the 29-bit copy of its points");
     if (g2) msm_launch_pre_g2(sort, d_points29, scr, st, split);
     else msm_launch_pre_g1(sort, d_points29, scr, st, split);
@@ -717,16 +735,21 @@ zkh::Xyzz<zkh::Fp> msm_g1_noalloc(int device, const void* d_points, const void* 
     ZK_REQUIRE(base != nullptr, ZK_E_STATE, "fixed MSM scratch not set up on this device");
     const SortShape z = sort_shape(n, window, false);
     const MsmGeom& g = z.g;
-    const int split = msm_default_split(n, g.c, false);
-    // the same buffers the allocating path sizes, laid out in the array
+    // the same buffers the allocating path sizes, laid out in the array; fewer
+    // threads per bucket where that makes them fit
     MsmSort sort;
     MsmScratch scr;
     DevBuf p29;
     size_t need = 0;
     auto count = [&](const DevBuf&, size_t b) { need = ((need + 255) & ~(size_t)255) + b; };
-    sort_buffers(sort, z, count);
-    scratch_buffers(scr, g, z.max_chunks, false, split, count);
-    count(p29, std::max<size_t>(n, 1) * PT29_BYTES);
+    int split = msm_alone_split(n, g.c, false);
+    for (;; split = split > 4 ? split / 2 : split - 1) {
+        need = 0;
+        sort_buffers(sort, z, count);
+        scratch_buffers(scr, g, z.max_chunks, false, split, count);
+        count(p29, std::max<size_t>(n, 1) * PT29_BYTES);
+        if (need <= MSM_NOALLOC_SCRATCH_BYTES || split == 1) break;
+    }
     ZK_REQUIRE(need <= MSM_NOALLOC_SCRATCH_BYTES, ZK_E_ARG,
                "MSM of " + std::to_string(n) + " points at window " + std::to_string(g.c) + " needs " +
                    std::to_string(need) + " bytes of workspace; the fixed scratch holds " +

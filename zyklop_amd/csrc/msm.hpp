@@ -183,11 +183,15 @@ struct MsmWorkspace {
 // sort, the W window tables of msm_points_table, table w at slot w*n); may be
 // null only for n = 0.
 // split: threads per bucket in the accumulation (1..MSM_SPLIT_MAX), each over
-// a consecutive part of the bucket's entries; the level-1 reduction adds the
-// parts. More threads than buckets fill the GPU when the buckets are few.
-constexpr int MSM_SPLIT_MAX = 4;
-// split that gives about two rounds of resident waves on a 256-CU GPU
+// a consecutive part of the bucket's entries; the reduction adds the parts.
+// More threads than buckets fill the GPU when the buckets are few.
+constexpr int MSM_SPLIT_MAX = 64;
+constexpr int MSM_SPLIT_TUNE = 4;   // largest split of a proof's MSMs (autotuner, tables)
+// of a proof's MSMs: about two rounds of resident waves on a 256-CU GPU
 int msm_default_split(size_t n, int c, bool g2, bool merged = false);
+// of an MSM that has the GPU to itself (the MSM entry points over caller-owned
+// points)
+int msm_alone_split(size_t n, int c, bool g2);
 void msm_launch(const MsmSort& sort, bool g2, MsmScratch& scr, MsmPartials& out, hipStream_t st,
                 const void* d_points29, int split = 1);
 // msm_launch in two parts: the chunked path of the oversized buckets, then

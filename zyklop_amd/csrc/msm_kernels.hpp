@@ -112,7 +112,7 @@ ZK_DEV void store_bucket(void* buckets, size_t slot, const Xyzz<T>& p) {
 // reduction.
 // Thread tid of an accumulation launch over nb buckets, each split into
 // `split` parts of consecutive entries (bucket b's parts go to slots
-// b*split + h, summed by the level-1 reduction). Returns false when the thread
+// b*split + h, summed by the reduction). Returns false when the thread
 // has nothing to accumulate: past the end, or a bucket above lmax entries.
 // Such a bucket is summed by the chunked path before this launch
 // (k_msm_chunks, k_msm_merge into slot b*split); its other parts store

@@ -111,10 +111,10 @@ float elapsed(TuneBufs& tb) {
 }
 
 // Device ms at window c, mean over reps after one warm-up: the sort, and each
-// MSM of `kind` at each split 1..MSM_SPLIT_MAX (msm[m][split-1]; splits that
+// MSM of `kind` at each split 1..MSM_SPLIT_TUNE (msm[m][split-1]; splits that
 // would start more than 2^21 threads are skipped and left at -1).
 void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged, const void* d_sc, size_t n,
-                 int reps, TuneBufs& tb, float& sort_ms, float msm[4][MSM_SPLIT_MAX]) {
+                 int reps, TuneBufs& tb, float& sort_ms, float msm[4][MSM_SPLIT_TUNE]) {
     hipStream_t st = ctx.stream;
     // the witness MSMs as a proof runs them: with the circuit's wire classes,
     // A and B1, B2 read their parts of the buckets
@@ -128,7 +128,7 @@ void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged
     const MsmGeom g = msm_geom(n, c, false, merged);
     sort_ms = 0;
     for (int m = 0; m < 4; m++)
-        for (int s = 0; s < MSM_SPLIT_MAX; s++) msm[m][s] = -1;
+        for (int s = 0; s < MSM_SPLIT_TUNE; s++) msm[m][s] = -1;
     for (int it = 0; it <= reps; it++) {
         ZK_HIP(hipEventRecord(tb.e0, st));
         tb.sort.run(d_sc, n, c, st, merged, cls);
@@ -136,7 +136,7 @@ void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged
         const float t_sort = elapsed(tb);
         if (it > 0) sort_ms += t_sort / reps;
         for (int m = 0; m < nm; m++)
-            for (int s = 1; s <= MSM_SPLIT_MAX; s++) {
+            for (int s = 1; s <= MSM_SPLIT_TUNE; s++) {
                 if ((size_t)g.Wr * g.K * s > ((size_t)1 << 21) && s > 1) continue;
                 ZK_HIP(hipEventRecord(tb.e0, st));
                 MsmScratch& scr = ms[m].g2 ? tb.g2 : tb.g1;
@@ -188,15 +188,15 @@ void Context::autotune(const Circuit& circ, bool force, int reps, int chosen[2])
             }
         }
         for (int c : cands) {
-            float sort_ms, msm[4][MSM_SPLIT_MAX];
+            float sort_ms, msm[4][MSM_SPLIT_TUNE];
             time_window(*this, circ, kind, c, tc != 0, d_sc.p, n, reps, tb, sort_ms, msm);
             float total = sort_ms;
             int sp[4] = {1, 1, 1, 1};
-            // a larger split adds level-1 work (one addition per extra part
+            // a larger split adds reduction work (one addition per extra part
             // and bucket) that a GPU shared with other proofs pays in full:
             // it must beat the smaller split alone by SPLIT_MARGIN
             for (int m = 0; m < (kind == 0 ? 4 : 1); m++) {
-                for (int s = 2; s <= MSM_SPLIT_MAX; s++)
+                for (int s = 2; s <= MSM_SPLIT_TUNE; s++)
                     if (msm[m][s - 1] >= 0 && msm[m][s - 1] < SPLIT_MARGIN * msm[m][sp[m] - 1]) sp[m] = s;
                 total += msm[m][sp[m] - 1];
             }
@@ -230,7 +230,7 @@ int Context::tune_load(const std::string& path) {
         ZK_REQUIRE(bool(is >> a >> kind >> cls >> c), ZK_E_FORMAT, "bad tuning table line: " + line);
         if (is >> s1) ZK_REQUIRE(bool(is >> s2), ZK_E_FORMAT, "bad tuning table line: " + line);
         ZK_REQUIRE(kind >= 0 && kind <= 3 && cls >= 0 && cls <= 40 && c >= 4 && c <= 22 && s1 >= 0 &&
-                       s1 <= MSM_SPLIT_MAX && s2 >= 0 && s2 <= MSM_SPLIT_MAX,
+                       s1 <= MSM_SPLIT_TUNE && s2 >= 0 && s2 <= MSM_SPLIT_TUNE,
                    ZK_E_FORMAT, "bad tuning table entry: " + line);
         if (a != me) continue;
         tuned[{kind, cls}] = {c, s1, s2};
