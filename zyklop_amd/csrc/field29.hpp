@@ -309,11 +309,8 @@ ZK_DEV F29 f29_unpack(const uint32_t w[8]) {
 ZK_DEV void f29_pack(const F29& a, uint32_t w[8]) {
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-        const int bit = 32 * k, i = bit / 29, sh = bit % 29;
-        uint64_t v = (uint64_t)a.l[i] >> sh;
-        if (i + 1 < 9) v |= (uint64_t)a.l[i + 1] << (29 - sh);
-        if (i + 2 < 9 && 58 - sh < 64) v |= (uint64_t)a.l[i + 2] << (58 - sh);
-        w[k] = (uint32_t)v;
+        const int bit = 32 * k, i = bit / 29, sh = bit % 29;   // sh = 3k: two limbs make a word
+        w[k] = a.l[i] >> sh | a.l[i + 1] << (29 - sh);
     }
 }
 
@@ -530,22 +527,15 @@ namespace fr29c {
 constexpr uint32_t R[9] = {0x10000001u, 0x1f0fac9fu, 0x0e5c2450u, 0x07d090f3u, 0x1585d283u,
                            0x02db40c0u, 0x00a6e141u, 0x0e5c2634u, 0x0030644eu};
 constexpr uint32_t NR = 0x0fffffffu;   // -r^-1 mod 2^29
-// 2^k r with every limb but the top one in [2^29, 2^30) (borrowed from the
-// next limb), so that 2^k r - b never borrows for normalized b < 2^k r
+// 2r with every limb but the top one in [2^29, 2^30) (borrowed from the next
+// limb), so that 2r - b never borrows for normalized b < 2r
 constexpr uint32_t R2[9] = {0x20000002u, 0x3e1f593eu, 0x3cb848a0u, 0x2fa121e5u, 0x2b0ba505u,
                             0x25b68180u, 0x214dc281u, 0x3cb84c67u, 0x0060c89bu};
-constexpr uint32_t R4[9] = {0x20000004u, 0x3c3eb27du, 0x39709142u, 0x3f4243ccu, 0x36174a0bu,
-                            0x2b6d0301u, 0x229b8503u, 0x397098cfu, 0x00c19138u};
-constexpr uint32_t R8[9] = {0x20000008u, 0x387d64fbu, 0x32e12286u, 0x3e84879au, 0x2c2e9418u,
-                            0x36da0604u, 0x25370a07u, 0x32e1319fu, 0x01832272u};
-constexpr uint32_t R16[9] = {0x20000010u, 0x30fac9f7u, 0x25c2450eu, 0x3d090f36u, 0x385d2832u,
-                             0x2db40c09u, 0x2a6e1410u, 0x25c2633fu, 0x030644e6u};
+// 4r with every limb but the top one in [2^30 - 2, 2^31) (2 borrowed): 4r - a - b
+// never borrows for normalized a + b < 4r
+constexpr uint32_t R4B[9] = {0x40000004u, 0x5c3eb27cu, 0x59709141u, 0x5f4243cbu, 0x56174a0au,
+                             0x4b6d0300u, 0x429b8502u, 0x597098ceu, 0x00c19137u};
 constexpr uint32_t RTOP1 = 3171407u;   // (r >> 232) + 1
-template <int K> struct ROff;          // 2^K r, borrowed
-template <> struct ROff<1> { static constexpr const uint32_t* L = R2; };
-template <> struct ROff<2> { static constexpr const uint32_t* L = R4; };
-template <> struct ROff<3> { static constexpr const uint32_t* L = R8; };
-template <> struct ROff<4> { static constexpr const uint32_t* L = R16; };
 }  // namespace fr29c
 
 struct F29ModR {
@@ -555,13 +545,12 @@ struct F29ModR {
 
 ZK_DEV F29 fr29_mul(const F29& a, const F29& b) { return f29_mul_mod<F29ModR>(a, b); }
 
-// a - b + 2^K r limb-wise, for normalized b < 2^K r: limbs below 2^31 (the
-// top one wraps below zero only when a carry from below makes it up)
-template <int K>
+// a - b + 2r limb-wise, for normalized b < 2r: limbs grow by less than 2^30
+// (the top one wraps below zero only when a carry from below makes it up)
 ZK_DEV F29 fr29_sub(const F29& a, const F29& b) {
     F29 r;
 #pragma unroll
-    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + fr29c::ROff<K>::L[i] - b.l[i];
+    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + fr29c::R2[i] - b.l[i];
     return r;
 }
 

@@ -1,9 +1,9 @@
-// Fr NTT kernels (design in ntt.hpp): register-radix passes of the four-step
-// recursion. Each thread owns one column of R = 2^lr points (lr <= 4), does
-// the whole radix-R DFT in registers, applies the inter-pass twiddle and
+// Fr NTT kernels (design in ntt.hpp): a pass transforms units of R = 2^q points
+// by a group of lanes of one wave, multiplies by the inter-pass twiddle and
 // writes back; the last pass writes the digit-reversed (natural) order.
 #include <vector>
 
+#include "coop29.hpp"
 #include "field.hpp"
 #include "field29.hpp"
 #include "host_field.hpp"
@@ -19,22 +19,10 @@ struct NttPtrs {
     void* out[NTT_MAX_BATCH];
 };
 
-// w_R^i for i < R/2 (standard form, prescaled by 2^5: field29.hpp "Fr"),
-// passed by value so they live in SGPRs
-struct RootsR {
-    Fr w[8];
-};
-
 struct NttDigits {
     int np;
     int lr[NTT_MAX_PASSES];
 };
-
-constexpr int bitrev_c(int x, int bits) {
-    int r = 0;
-    for (int i = 0; i < bits; i++) r |= ((x >> i) & 1) << (bits - 1 - i);
-    return r;
-}
 
 // ---- elements: 9 x 29-bit limbs in registers, 8 canonical words in memory ----
 // A product by a prescaled table value keeps the standard form (field29.hpp).
@@ -52,183 +40,270 @@ ZK_DEV void st29(void* base, size_t i, const F29& x) {
     p[0] = make_uint4(w[0], w[1], w[2], w[3]);
     p[1] = make_uint4(w[4], w[5], w[6], w[7]);
 }
-// limbs below 2^31, value below 2^261 -> normalized, below r + 2^240
+// x normalized and below 5r, not made canonical: between the passes of one
+// transform, whose loads take any value that fits 8 words
+ZK_DEV void st29_lazy(void* base, size_t i, const F29& x) {
+    uint32_t w[8];
+    f29_pack(x, w);
+    uint4* p = reinterpret_cast<uint4*>(base) + 2 * i;
+    p[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    p[1] = make_uint4(w[4], w[5], w[6], w[7]);
+}
+// limbs below 2^32, value below 2^261 -> normalized, below r + 2^240
 ZK_DEV F29 settle29(const F29& x) { return fr29_reduce(f29_norm(x)); }
 
-// one radix-2 DIT stage (span 2^(S-1)) of a 2^LR-point DFT held in registers;
-// every loop has a constant trip count so the whole DFT unrolls to registers.
-// Bounds (worst cases followed stage by stage in an exact model): the DFT's
-// inputs are below 1.2r (canonical loads, products by a prescaled table
-// value, below 1.01r, or settled values, below r + 2^240); stage S then
-// sees b below 2^S r with a top limb below that of the borrowed 2^S r, so
-// a - b + 2^S r has no negative limb; outputs stay below 32r (radix 16),
-// limbs below 2^31. Between stages the limbs are normalized; the last
-// stage's outputs go straight to a product (limbs below 2^31 are fine
-// there) or to settle29.
-template <int LR, int S>
-struct DftStage {
-    ZK_DEV static void run(F29 (&x)[1 << LR], const F29 (&w)[8]) {
-        constexpr int R = 1 << LR, half = 1 << (S - 1);
+// root i of the DFTs inside a unit, w_256^i in limbs, 12 words apart
+constexpr int ROOT_WORDS = 12;
+ZK_DEV F29 ld_root(const void* roots, uint32_t i) {
+    const uint4* p = reinterpret_cast<const uint4*>(roots) + ROOT_WORDS / 4 * i;
+    const uint4 a = p[0], b = p[1];
+    return F29{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, reinterpret_cast<const uint32_t*>(p + 2)[0]}};
+}
+
+// what a pass reads and writes: unit u of 2^q points. Passes 0..np-2, in place
+// over blocks of M = R*S elements: u is the column c of block beta, points
+// beta*M + b*S + c. The last pass: points of row r (unrev of u), r*R + b, to
+// out[u + k*O], O = n/R.
+struct NttShape {
+    NttDigits dg;
+    int logS;     // of a pass that is not the last
+    int last;
+    size_t n;
+    const void* roots;   // w_256^i, i < 256 (ld_root)
+    const void* tw;      // w_M^(c k), [k][c], passes but the last
+    const void* pre;     // first pass: multiplies input i
+    const void* post;    // last pass: multiplies output i
+};
+struct NttUnit {
+    size_t in, in_step, out, out_step, col;
+};
+template <int Q>
+ZK_DEV NttUnit ntt_unit(const NttShape& z, size_t u) {
+    if (!z.last) {
+        const size_t c = u & (((size_t)1 << z.logS) - 1), base = ((u >> z.logS) << (z.logS + Q)) + c;
+        return {base, (size_t)1 << z.logS, base, (size_t)1 << z.logS, c};
+    }
+    size_t r = u, row = 0;
+    for (int d = 0; d < z.dg.np - 1; d++) {
+        const size_t digit = r & (((size_t)1 << z.dg.lr[d]) - 1);
+        r >>= z.dg.lr[d];
+        row = (row << z.dg.lr[d]) | digit;
+    }
+    return {row << Q, 1, u, z.n >> Q, 0};
+}
+// output k of a unit, x with limbs below 1.5 * 2^30 and value below 20r: scaled,
+// then stored. Apart, so that the scaling loads of all outputs come before any
+// store, which they could not pass.
+ZK_DEV F29 ntt_scale(const NttShape& z, const NttUnit& t, uint32_t k, const F29& x) {
+    if (!z.last) return fr29_mul(x, ld29(z.tw, ((size_t)k << z.logS) + t.col));
+    if (z.post) return fr29_mul(x, ld29(z.post, t.out + k * t.out_step));
+    return settle29(x);
+}
+ZK_DEV void ntt_store(const NttShape& z, const NttUnit& t, void* out, uint32_t k, const F29& x) {
+    if (!z.last) st29_lazy(out, t.out + k * t.out_step, x);
+    else st29(out, t.out + k * t.out_step, x);
+}
+
+// ---- two points per lane
+// A unit's 2^q points on 2^(q-1) lanes, radix-2 DIT stages in registers; before
+// stage s the lanes swap one point with lane ^ 2^(s-2), so that every lane holds
+// both points of its butterfly: position bit s-1 is then the slot, bits below
+// are lane bits 0..s-2. About 20 % more instructions per point than four points
+// per lane (below), but half the chain per launch and twice the waves: for
+// transforms that do not fill the GPU, where the chain sets the time. 2^12
+// points: two launches of 9 and 7 us, against 26 + 13 + 9 us for radix-8 threads
+// whose pass pairs went through 36 KiB of LDS (77 -> 45 us for the call); three
+// arrays of 2^17 142 -> 89 us.
+// Bounds: after stage 1 values below 3.2r, each later stage adds at most 2r
+// (its b is a product, below 1.1r): below 16r after 7. Limbs grow by at most
+// 2^30 a stage from 2^29; normalized after every second stage, so a product's
+// operand stays below 1.5 * 2^30.
+template <int BIT>
+ZK_DEV void lane_swap(F29& x0, F29& x1) {
+    if (BIT == 4 || BIT == 5) {
 #pragma unroll
-        for (int q = 0; q < R / 2; q++) {
-            const int p = q & (half - 1);
-            const int i0 = (q >> (S - 1)) * 2 * half + p, i1 = i0 + half;
-            const F29 a = x[i0];
-            F29 b = x[i1];
-            if (p) b = fr29_mul(b, w[p * (R >> S)]);
-            x[i0] = f29_add(a, b);
-            x[i1] = fr29_sub<S>(a, b);
+        for (int i = 0; i < 9; i++) {
+            // odd rows (halves) of x0 against even ones of x1
+            const auto r = BIT == 4 ? __builtin_amdgcn_permlane16_swap(x0.l[i], x1.l[i], false, false)
+                                    : __builtin_amdgcn_permlane32_swap(x0.l[i], x1.l[i], false, false);
+            x0.l[i] = r[0];
+            x1.l[i] = r[1];
         }
-        if (S < LR) {
+        return;
+    }
+    const uint32_t m = 0u - (threadIdx.x >> BIT & 1u);   // lanes with the bit keep x1
+    const F29 give = f29_sel(m, x0, x1);
+    F29 got;
 #pragma unroll
-            for (int i = 0; i < R; i++) x[i] = f29_norm(x[i]);
+    for (int i = 0; i < 9; i++) {
+        if (BIT == 0) got.l[i] = u32_quad<1, 0, 3, 2>(give.l[i]);
+        if (BIT == 1) got.l[i] = u32_quad<2, 3, 0, 1>(give.l[i]);
+        if (BIT == 2) got.l[i] = u32_xor4(give.l[i]);
+        if (BIT == 3) got.l[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give.l[i], 0x128, 0xf, 0xf, true);   // row_ror:8
+    }
+    x0 = f29_sel(m, got, x0);
+    x1 = f29_sel(m, x1, got);
+}
+template <int Q, int S>
+struct LaneStage {
+    ZK_DEV static void run(F29& x0, F29& x1, uint32_t lane, const void* roots) {
+        lane_swap<S - 2>(x0, x1);
+        const uint32_t p = lane & ((1u << (S - 1)) - 1);
+        const F29 b = fr29_mul(x1, ld_root(roots, p << (8 - S)));
+        x1 = fr29_sub(x0, b);
+        x0 = f29_add(x0, b);
+        if (S % 2 == 0) {
+            x0 = f29_norm(x0);
+            x1 = f29_norm(x1);
         }
-        DftStage<LR, S + 1>::run(x, w);
+        LaneStage<Q, S + 1>::run(x0, x1, lane, roots);
     }
 };
-template <int LR>
-struct DftStage<LR, LR + 1> {
-    ZK_DEV static void run(F29 (&)[1 << LR], const F29 (&)[8]) {}
+template <int Q> struct LaneEnd {
+    ZK_DEV static void run(F29&, F29&, uint32_t, const void*) {}
 };
+template <> struct LaneStage<1, 2> : LaneEnd<1> {};
+template <> struct LaneStage<2, 3> : LaneEnd<2> {};
+template <> struct LaneStage<3, 4> : LaneEnd<3> {};
+template <> struct LaneStage<4, 5> : LaneEnd<4> {};
+template <> struct LaneStage<5, 6> : LaneEnd<5> {};
+template <> struct LaneStage<6, 7> : LaneEnd<6> {};
+template <> struct LaneStage<7, 8> : LaneEnd<7> {};
 
-// radix-2^LR DFT in registers, X_k = sum_b x_b w_R^(b k); the caller loads
-// input b into x[bitrev(b)] and gets natural-order output
-template <int LR>
-ZK_DEV void dft_reg(F29 (&x)[1 << LR], const RootsR& rt) {
-    F29 w[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) w[i] = f29_unpack(rt.w[i].v);
-    DftStage<LR, 1>::run(x, w);
-}
-
-// In-place pass j < np-1 over blocks of M = R*S elements: thread (beta, c)
-// transforms x[beta*M + b*S + c], b < R, then multiplies output k by w_M^(c k)
-// (the table holds w_M^0 for c = 0, so every output k >= 1 is a product).
-template <int LR>
-__global__ void __launch_bounds__(NTT_THREADS) k_ntt_pass(NttPtrs ptrs, int logM, size_t n, RootsR rt,
-                                                          const void* __restrict__ tw, const void* __restrict__ pre) {
-    constexpr int R = 1 << LR;
-    size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= (n >> LR)) return;
-    void* data = ptrs.in[blockIdx.y];
-    const int logS = logM - LR;
-    const size_t c = tid & (((size_t)1 << logS) - 1);
-    const size_t base = (tid >> logS) << logM;
-    F29 x[R];
-#pragma unroll
-    for (int b = 0; b < R; b++) {
-        const size_t i = base + ((size_t)b << logS) + c;
-        F29 v = ld29(data, i);
-        if (pre) v = fr29_mul(v, ld29(pre, i));
-        x[bitrev_c(b, LR)] = v;
-    }
-    dft_reg<LR>(x, rt);
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-        const F29 y = k ? fr29_mul(x[k], ld29(tw, ((size_t)k << logS) + c)) : settle29(x[k]);
-        st29(data, base + ((size_t)k << logS) + c, y);
-    }
-}
-
-// Two consecutive passes j, j+1 (radix R1 = 2^LR1, then R2 = 2^LR2) in one
-// kernel, the intermediate result staged in LDS. With M = R1*S (pass j),
-// S = R2*S' (pass j+1), the R1*R2 points x[beta*M + b*S + b2*S' + c2]
-// (b < R1, b2 < R2) of one unit u = (beta, c2) touch no other unit in either
-// pass. A workgroup takes U consecutive units:
-//   step 1: thread (b2, u) runs pass j's DFT over b for column c = b2*S' + c2,
-//           multiplies output k by w_M^(c k) and writes LDS[k][b2][u];
-//   step 2: thread (k, u) runs pass j+1's DFT over b2 for sub-block (beta, k),
-//           multiplies output k2 by w_S^(c2 k2) and stores x[beta*M + k*S +
-//           k2*S' + c2].
-// Consecutive lanes take consecutive units, so global accesses stay coalesced
-// (runs of min(S', U) elements). The LDS holds the 9 limbs of each staged
-// element (normalized, below 1.2r), limb-major.
-template <int LR1, int LR2, int U>
-__global__ void __launch_bounds__((1 << LR2) * U) k_ntt_pass2(NttPtrs ptrs, int logM, size_t n, RootsR rt1, RootsR rt2,
-                                                              const void* __restrict__ tw1, const void* __restrict__ tw2,
-                                                              const void* __restrict__ pre) {
-    constexpr int R1 = 1 << LR1, R2 = 1 << LR2, NS = R1 * R2 * U;
-    static_assert(R1 == R2, "one task per thread in both steps");
-    __shared__ uint32_t lds[9 * NS];
-    void* data = ptrs.in[blockIdx.y];
-    const int logS = logM - LR1, logS2 = logS - LR2;
-    const size_t S2 = (size_t)1 << logS2;
-    const int ul = threadIdx.x % U, q = threadIdx.x / U;   // unit lane, digit (b2 in step 1, k in step 2)
-    const size_t u = (size_t)blockIdx.x * U + ul;
-    const size_t beta = u >> logS2, c2 = u & (S2 - 1);
-    const size_t base = beta << logM;
-    const bool live = u < (n >> (LR1 + LR2));
-    if (live) {
-        // step 1: pass j over b for column c = q*S' + c2
-        const size_t c = ((size_t)q << logS2) + c2;
-        F29 x[R1];
-#pragma unroll
-        for (int b = 0; b < R1; b++) {
-            const size_t i = base + ((size_t)b << logS) + c;
-            F29 v = ld29(data, i);
-            if (pre) v = fr29_mul(v, ld29(pre, i));
-            x[bitrev_c(b, LR1)] = v;
-        }
-        dft_reg<LR1>(x, rt1);
-#pragma unroll
-        for (int k = 0; k < R1; k++) {
-            const F29 y = k ? fr29_mul(x[k], ld29(tw1, ((size_t)k << logS) + c)) : settle29(x[k]);
-#pragma unroll
-            for (int l = 0; l < 9; l++) lds[l * NS + (k * R2 + q) * U + ul] = y.l[l];
-        }
-    }
-    __syncthreads();
-    if (!live) return;
-    // step 2: pass j+1 over b2 for sub-block (beta, k = q), column c2
-    F29 x[R2];
-#pragma unroll
-    for (int b2 = 0; b2 < R2; b2++) {
-        F29 v;
-#pragma unroll
-        for (int l = 0; l < 9; l++) v.l[l] = lds[l * NS + (q * R2 + b2) * U + ul];
-        x[bitrev_c(b2, LR2)] = v;
-    }
-    dft_reg<LR2>(x, rt2);
-    const size_t sub = base + ((size_t)q << logS);
-#pragma unroll
-    for (int k2 = 0; k2 < R2; k2++) {
-        const F29 y = k2 ? fr29_mul(x[k2], ld29(tw2, ((size_t)k2 << logS2) + c2)) : settle29(x[k2]);
-        st29(data, sub + ((size_t)k2 << logS2) + c2, y);
-    }
-}
-
-// Last pass: thread = output column rv (digit-reversed row index); the row of
-// R contiguous points at unrev(rv)*R gives out[rv + O*k], k < R.
-template <int LR>
-__global__ void __launch_bounds__(NTT_THREADS) k_ntt_final(NttPtrs ptrs, NttDigits dg, size_t n, RootsR rt,
-                                                           const void* __restrict__ pre, const void* __restrict__ post) {
-    constexpr int R = 1 << LR;
-    const size_t O = n >> LR;
-    size_t rv = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (rv >= O) return;
+template <int Q>
+__global__ void __launch_bounds__(NTT_THREADS) k_ntt_lane(NttPtrs ptrs, NttShape z) {
+    constexpr uint32_t LANES = 1u << (Q - 1);
+    const size_t tid = (size_t)blockIdx.x * NTT_THREADS + threadIdx.x, u = tid >> (Q - 1);
+    if (u >= z.n >> Q) return;   // whole units
+    const uint32_t lane = (uint32_t)tid & (LANES - 1);
     const void* in = ptrs.in[blockIdx.y];
-    void* out = ptrs.out[blockIdx.y];
-    size_t r = rv, row = 0;
-    for (int d = 0; d < dg.np - 1; d++) {
-        size_t digit = r & (((size_t)1 << dg.lr[d]) - 1);
-        r >>= dg.lr[d];
-        row = (row << dg.lr[d]) | digit;
+    const NttUnit t = ntt_unit<Q>(z, u);
+    const uint32_t b = Q > 1 ? __brev(lane) >> (33 - Q) : 0u;
+    const size_t i0 = t.in + b * t.in_step, i1 = i0 + LANES * t.in_step;
+    F29 x0 = ld29(in, i0), x1 = ld29(in, i1);
+    if (z.pre) {
+        x0 = fr29_mul(x0, ld29(z.pre, i0));
+        x1 = fr29_mul(x1, ld29(z.pre, i1));
     }
-    F29 x[R];
+    const F29 a = x0;
+    x0 = f29_add(a, x1);
+    x1 = fr29_sub(a, x1);
+    LaneStage<Q, 2>::run(x0, x1, lane, z.roots);
+    void* out = z.last ? ptrs.out[blockIdx.y] : ptrs.in[blockIdx.y];
+    x0 = ntt_scale(z, t, lane, x0);
+    x1 = ntt_scale(z, t, lane + LANES, x1);
+    ntt_store(z, t, out, lane, x0);
+    ntt_store(z, t, out, lane + LANES, x1);
+}
+
+// ---- four points per lane
+// A unit's 2^Q points on 2^(Q-2) lanes, radix-4 steps in registers (a radix-2
+// one last when Q is odd). Step t transforms the top digit left, which the
+// lane's four slots hold, multiplies output k_t by w^(k_t * rest) and swaps the
+// slots with the two lane bits that hold the next digit. In the end the lane
+// bits hold k_1, k_2, ... from the top and the slots the last digit, of output k
+// = k_1 + 4 k_2 + 16 k_3 + ...
+// Which lane bits: the first swap on bits 5, 4 (v_permlane32/16_swap, one
+// instruction per limb for both points), then 1, 0 (DPP in a quad); 3, 2 only
+// in units of 2^7 points and more. The bits left over number the wave's units.
+// Bound by instruction issue: 5044 VALU instructions per lane for 2^8 points per
+// unit (3336 for 2^6), 60 % of them v_mad_u64_u32; the 2^22 transform is three
+// launches of 165, 165 and 110 us and its instructions alone take 0.38 ms. Four
+// waves per SIMD (five are the same, six spill 12 %). The radix-8 threads before
+// took four launches, 0.56 ms (call 617 -> 522 us); eight points per lane with
+// the same exchange held three waves per SIMD and 563 us.
+constexpr int quad_bit(int Q, int i) {   // lane bit of the i-th bit from the top of the unit's lane
+    return Q == 8 ? 5 - i : Q == 7 ? (i < 2 ? 5 - i : i < 4 ? 3 - i : 3) : (i < 2 ? 5 - i : 3 - i);
+}
+template <int BIT_HI, int BIT_LO>
+ZK_DEV void quad_swap(F29 (&x)[4]) {
+    lane_swap<BIT_HI>(x[0], x[2]);
+    lane_swap<BIT_HI>(x[1], x[3]);
+    lane_swap<BIT_LO>(x[0], x[1]);
+    lane_swap<BIT_LO>(x[2], x[3]);
+}
+// Four-point DFT, natural order in and out. Inputs normalized and below 1.2r;
+// outputs below 7r, limbs below 2.5 * 2^30 (a product takes them as they are: 9
+// * 2.5 * 2^59 + 9 * 2^58 and the carry stay below 2^64). The difference of two
+// sums takes 4r borrowed twice (R4B).
+ZK_DEV void dft4(F29 (&x)[4], const F29& w4) {
+    const F29 a = f29_add(x[0], x[2]), b = f29_add(x[1], x[3]);
+    const F29 c = fr29_sub(x[0], x[2]), d = fr29_mul(fr29_sub(x[1], x[3]), w4);
+    x[0] = f29_add(a, b);
 #pragma unroll
-    for (int b = 0; b < R; b++) {
-        const size_t i = (row << LR) + b;
-        F29 v = ld29(in, i);
-        if (pre && dg.np == 1) v = fr29_mul(v, ld29(pre, i));
-        x[bitrev_c(b, LR)] = v;
-    }
-    dft_reg<LR>(x, rt);
+    for (int i = 0; i < 9; i++) x[2].l[i] = a.l[i] + fr29c::R4B[i] - b.l[i];
+    x[1] = f29_add(c, d);
+    x[3] = fr29_sub(c, d);
+}
+// step T of a unit of 2^Q points, the digit over what lies below it in the lane
+template <int Q, int T>
+struct QuadStep {
+    ZK_DEV static void run(F29 (&x)[4], uint32_t lane, const void* roots, const F29& w4) {
+        constexpr int LEFT = Q - 2 * T;   // bits below this step's digit
+        dft4(x, w4);
+        if constexpr (LEFT > 0) {
+            const uint32_t rest = lane & ((1u << LEFT) - 1);   // of the unit's lane, its low LEFT bits
+            x[0] = settle29(x[0]);
 #pragma unroll
-    for (int k = 0; k < R; k++) {
-        const size_t o = rv + (size_t)k * O;
-        const F29 y = post ? fr29_mul(x[k], ld29(post, o)) : settle29(x[k]);
-        st29(out, o, y);
+            for (uint32_t k = 1; k < 4; k++)   // w_{2^(LEFT + 2)}^(rest * k)
+                x[k] = fr29_mul(x[k], ld_root(roots, (rest * k) << (8 - LEFT - 2)));
+            if constexpr (LEFT == 1) {
+                lane_swap<quad_bit(Q, Q - 3)>(x[0], x[2]);
+                lane_swap<quad_bit(Q, Q - 3)>(x[1], x[3]);
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const F29 a = x[i], b = x[i + 2];
+                    x[i] = f29_add(a, b);
+                    x[i + 2] = fr29_sub(a, b);
+                }
+            } else {
+                quad_swap<quad_bit(Q, 2 * T - 2), quad_bit(Q, 2 * T - 1)>(x);
+                QuadStep<Q, T + 1>::run(x, lane, roots, w4);
+            }
+        }
     }
+};
+
+template <int Q>
+__global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_ntt_quad(NttPtrs ptrs, NttShape z) {
+    constexpr int LB = Q - 2;            // lane bits of a unit
+    const uint32_t hw = threadIdx.x & 63;
+    uint32_t lane = 0, used = 0, sub = 0;   // the unit's lane; the unit in the wave
+#pragma unroll
+    for (int i = 0; i < LB; i++) {
+        lane |= (hw >> quad_bit(Q, i) & 1u) << (LB - 1 - i);
+        used |= 1u << quad_bit(Q, i);
+    }
+#pragma unroll
+    for (int i = 0, k = 0; i < 6; i++)
+        if (!(used >> i & 1u)) sub |= (hw >> i & 1u) << k++;
+    const size_t u = (((size_t)blockIdx.x * (NTT_THREADS / 64) + threadIdx.x / 64) << (6 - LB)) + sub;
+    if (u >= z.n >> Q) return;   // whole units
+    const void* in = ptrs.in[blockIdx.y];
+    const NttUnit t = ntt_unit<Q>(z, u);
+    F29 x[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) x[i] = ld29(in, t.in + (lane + (i << LB)) * t.in_step);
+    if (z.pre) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) x[i] = fr29_mul(x[i], ld29(z.pre, t.in + (lane + (i << LB)) * t.in_step));
+    }
+    QuadStep<Q, 1>::run(x, lane, z.roots, ld_root(z.roots, 64));
+    // output of slot s: digits k_1.. from the lane's top bits, the last from the slot
+    uint32_t k0 = 0;
+#pragma unroll
+    for (int d = 0; 2 * d + 1 < LB; d++) k0 |= (lane >> (LB - 2 - 2 * d) & 3u) << (2 * d);
+    // an odd Q's radix-2 step left the low bit of its radix-4 neighbour's digit
+    // in slot bit 0, its high bit in the lane's last bit, its own digit in slot bit 1
+    uint32_t k[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++)
+        k[i] = Q % 2 ? k0 | (2 * (lane & 1u) + (i & 1u)) << (Q - 3) | (i >> 1) << (Q - 1) : k0 | i << LB;
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = ntt_scale(z, t, k[i], x[i]);
+    void* out = z.last ? ptrs.out[blockIdx.y] : ptrs.in[blockIdx.y];
+#pragma unroll
+    for (int i = 0; i < 4; i++) ntt_store(z, t, out, k[i], x[i]);
 }
 
 // table[i] = lo[e & 4095] * hi[e >> 12] for e = exponent(i)
@@ -272,18 +347,29 @@ static zkh::Fr root_of_unity(int log_n) {
     return zkh::Fr::from_u64(5).pow(e);
 }
 
-// pass radices of a size-2^ln transform: radix-8 passes; a radix-16 pass
-// absorbs one leftover bit, radix-4/2 the rest. Returns the pass count.
+// Pass radices of a size-2^ln transform; returns the pass count. Up to 2^17, two
+// points per lane: radices up to 2^7 of even sizes. Above, four points per lane:
+// up to 2^8, even powers (radix-4 steps only) but for an odd ln's last pass.
+constexpr int NTT_LANE_LOG = 17;
 static int ntt_layout(int ln, int lr[NTT_MAX_PASSES]) {
-    int np = 0, rem = ln;
-    while (rem > 0) {
-        int take = rem >= 3 ? 3 : rem;
-        lr[np++] = take;
-        rem -= take;
+    const int most = ln <= NTT_LANE_LOG ? 7 : 8, np = (ln + most - 1) / most;
+    for (int j = 0; j < NTT_MAX_PASSES; j++) lr[j] = 0;
+    if (ln <= NTT_LANE_LOG) {
+        for (int j = 0; j < np; j++) lr[j] = ln / np + (j < ln % np);
+        return np;
     }
-    if (np >= 2 && lr[np - 1] == 1) { lr[np - 2] += 1; np--; }  // ...3,1 -> ...4
-    for (int j = np; j < NTT_MAX_PASSES; j++) lr[j] = 0;
+    int rem = ln;
+    for (int j = 0; j < np; j++) rem -= lr[j] = ln / (2 * np) * 2;
+    for (int j = 0; rem >= 2; j++, rem -= 2) lr[j] += 2;
+    lr[np - 1] += rem;
     return np;
+}
+// Two points per lane below 2^20 points in all, where four leave less than four
+// waves per SIMD: three arrays of 2^18 125 against 130 us, one of 2^19 101
+// against 107, three of 2^17 89 against 103; from 2^20 on four are faster (three
+// of 2^20 395 against 415, one of 2^22 522 against 569).
+static bool ntt_two_points(int ln, size_t points) {
+    return ln <= NTT_LANE_LOG || (ln <= 19 && points < ((size_t)1 << 20));   // 2^20 and up have 2^8 passes
 }
 
 // entries of the concatenated pass twiddle tables (passes 0..np-2), and each pass's offset
@@ -302,7 +388,7 @@ size_t NttPlan::bytes_for(int ln) {
     int lr_[NTT_MAX_PASSES];
     const int np_ = ntt_layout(ln, lr_);
     const size_t tot = ntt_tw_entries(ln, np_, lr_, nullptr);
-    return 2 * std::max<size_t>(tot, 1) * 32 + 4 * ((size_t)1 << ln) * 32;
+    return 2 * std::max<size_t>(tot, 1) * 32 + 2 * 256 * ROOT_WORDS * 4 + 4 * ((size_t)1 << ln) * 32;
 }
 
 void NttPlan::build(int ln, hipStream_t st) {
@@ -330,15 +416,22 @@ void NttPlan::build(int ln, hipStream_t st) {
     ZK_HIP(hipMemcpyAsync(d_s32.p, &s32, 32, hipMemcpyHostToDevice, st));
     const uint64_t mask2n = (2 * (uint64_t)n) - 1;
 
-    // radix roots w_R^i = w_2n^(i * 2n / R), forward and inverse, on the host
-    for (int j = 0; j < np; j++) {
-        int R = 1 << lr[j];
-        for (int i = 0; i < 8; i++) {
-            uint64_t e = i < R / 2 ? ((uint64_t)i * ((2 * (uint64_t)n) >> lr[j])) & mask2n : 0;
-            zkh::Fr f = lo_f[e & 4095] * hi_f[e >> 12] * s32, v = lo_i[e & 4095] * hi_i[e >> 12] * s32;
-            memcpy(roots_fwd[j] + 4 * i, f.v, 32);  // 4 words per element
-            memcpy(roots_inv[j] + 4 * i, v.v, 32);
-        }
+    // w_256^i for the DFTs inside a unit, forward and inverse, in limbs
+    std::vector<uint32_t> limbs[2];
+    for (int d = 0; d < 2; d++) {
+        const zkh::Fr g = d ? root_of_unity(8).inv() : root_of_unity(8);
+        zkh::Fr f = s32;
+        limbs[d].assign(256 * ROOT_WORDS, 0);
+        for (int i = 0; i < 256; i++, f = f * g)
+            for (int l = 0; l < 9; l++) {
+                const int k = 29 * l / 64, sh = 29 * l % 64;
+                uint64_t v = f.v[k] >> sh;
+                if (sh > 35 && k < 3) v |= f.v[k + 1] << (64 - sh);
+                limbs[d][ROOT_WORDS * i + l] = (uint32_t)v & f29c::MASK;
+            }
+        DevBuf& dst = d ? roots_inv : roots_fwd;
+        dst.ensure(256 * ROOT_WORDS * 4);
+        ZK_HIP(hipMemcpyAsync(dst.p, limbs[d].data(), 256 * ROOT_WORDS * 4, hipMemcpyHostToDevice, st));
     }
     // pass twiddle tables w_M^(c k), layout [k][c], for passes 0..np-2
     const size_t tot = ntt_tw_entries(ln, np, lr, tw_off);
@@ -369,26 +462,13 @@ void NttPlan::build(int ln, hipStream_t st) {
     ZK_HIP(hipStreamSynchronize(st));  // the temporaries above are freed on return
 }
 
-template <int LR>
-static void launch_pass(const NttPtrs& ptrs, int batch, int logM, size_t n, const RootsR& rt, const void* tw,
-                        const void* pre, hipStream_t st) {
-    unsigned grid = cdiv(n >> LR, NTT_THREADS);
-    k_ntt_pass<LR><<<dim3(grid, batch), NTT_THREADS, 0, st>>>(ptrs, logM, n, rt, tw, pre);
+template <int Q>
+static void launch_lane(const NttPtrs& ptrs, int batch, const NttShape& z, hipStream_t st) {
+    k_ntt_lane<Q><<<dim3(cdiv(z.n / 2, NTT_THREADS), batch), NTT_THREADS, 0, st>>>(ptrs, z);
 }
-
-constexpr int NTT2_UNITS = 16;   // 36 KiB of LDS per workgroup (9 limbs x 64 points x 16 units)
-
-static void launch_pass2(const NttPtrs& ptrs, int batch, int logM, size_t n, const RootsR& rt1, const RootsR& rt2,
-                         const void* tw1, const void* tw2, const void* pre, hipStream_t st) {
-    unsigned grid = cdiv(n >> 6, NTT2_UNITS);
-    k_ntt_pass2<3, 3, NTT2_UNITS><<<dim3(grid, batch), 8 * NTT2_UNITS, 0, st>>>(ptrs, logM, n, rt1, rt2, tw1, tw2, pre);
-}
-
-template <int LR>
-static void launch_final(const NttPtrs& ptrs, int batch, const NttDigits& dg, size_t n, const RootsR& rt, const void* pre,
-                         const void* post, hipStream_t st) {
-    unsigned grid = cdiv(n >> LR, NTT_THREADS);
-    k_ntt_final<LR><<<dim3(grid, batch), NTT_THREADS, 0, st>>>(ptrs, dg, n, rt, pre, post);
+template <int Q>
+static void launch_quad(const NttPtrs& ptrs, int batch, const NttShape& z, hipStream_t st) {
+    k_ntt_quad<Q><<<dim3(cdiv(z.n / 4, NTT_THREADS), batch), NTT_THREADS, 0, st>>>(ptrs, z);
 }
 
 void ntt_run(const NttPlan& p, void* const* in, void* const* out, int batch, bool inverse, const void* pre, const void* post,
@@ -398,47 +478,42 @@ void ntt_run(const NttPlan& p, void* const* in, void* const* out, int batch, boo
     for (int b = 0; b < NTT_MAX_BATCH; b++) {
         ptrs.in[b] = b < batch ? in[b] : nullptr;
         ptrs.out[b] = b < batch ? out[b] : nullptr;
-        if (b < batch && p.np > 1) ZK_REQUIRE(in[b] != out[b], ZK_E_ARG, "multi-pass NTT needs distinct in/out");
+        if (b < batch && p.log_n > 4) ZK_REQUIRE(in[b] != out[b], ZK_E_ARG, "NTT of more than 16 points needs distinct in/out");
     }
-    NttDigits dg;
-    dg.np = p.np;
-    for (int j = 0; j < NTT_MAX_PASSES; j++) dg.lr[j] = p.lr[j];
+    NttShape z;
+    z.dg.np = p.np;
+    for (int j = 0; j < NTT_MAX_PASSES; j++) z.dg.lr[j] = p.lr[j];
+    z.n = p.n;
+    z.roots = (inverse ? p.roots_inv : p.roots_fwd).p;
     const char* tw = (const char*)(inverse ? p.tw_inv.p : p.tw_fwd.p);
+    const bool lanes = ntt_two_points(p.log_n, p.n * batch);
     int consumed = 0;
     for (int j = 0; j < p.np; j++) {
-        RootsR rt;
-        memcpy(&rt, inverse ? p.roots_inv[j] : p.roots_fwd[j], sizeof rt);
-        const int lrj = p.lr[j];
-        if (j < p.np - 1) {
-            const int logM = p.log_n - consumed;
-            const void* pj = j == 0 ? pre : nullptr;
-            const void* twj = tw + p.tw_off[j] * 32;
-            // two radix-8 passes through LDS when both are regular passes
-            if (lrj == 3 && j + 1 < p.np - 1 && p.lr[j + 1] == 3) {
-                RootsR rt2;
-                memcpy(&rt2, inverse ? p.roots_inv[j + 1] : p.roots_fwd[j + 1], sizeof rt2);
-                launch_pass2(ptrs, batch, logM, p.n, rt, rt2, twj, tw + p.tw_off[j + 1] * 32, pj, st);
-                ZK_HIP(hipGetLastError());
-                consumed += 6;
-                j++;
-                continue;
-            }
-            switch (lrj) {
-                case 1: launch_pass<1>(ptrs, batch, logM, p.n, rt, twj, pj, st); break;
-                case 2: launch_pass<2>(ptrs, batch, logM, p.n, rt, twj, pj, st); break;
-                case 3: launch_pass<3>(ptrs, batch, logM, p.n, rt, twj, pj, st); break;
-                default: launch_pass<4>(ptrs, batch, logM, p.n, rt, twj, pj, st); break;
+        const int q = p.lr[j];
+        consumed += q;
+        z.last = j == p.np - 1;
+        z.logS = p.log_n - consumed;
+        z.tw = tw + p.tw_off[j] * 32;
+        z.pre = j == 0 ? pre : nullptr;
+        z.post = post;
+        if (lanes) {
+            switch (q) {
+                case 1: launch_lane<1>(ptrs, batch, z, st); break;
+                case 2: launch_lane<2>(ptrs, batch, z, st); break;
+                case 3: launch_lane<3>(ptrs, batch, z, st); break;
+                case 4: launch_lane<4>(ptrs, batch, z, st); break;
+                case 5: launch_lane<5>(ptrs, batch, z, st); break;
+                case 6: launch_lane<6>(ptrs, batch, z, st); break;
+                default: launch_lane<7>(ptrs, batch, z, st); break;
             }
         } else {
-            switch (lrj) {
-                case 1: launch_final<1>(ptrs, batch, dg, p.n, rt, pre, post, st); break;
-                case 2: launch_final<2>(ptrs, batch, dg, p.n, rt, pre, post, st); break;
-                case 3: launch_final<3>(ptrs, batch, dg, p.n, rt, pre, post, st); break;
-                default: launch_final<4>(ptrs, batch, dg, p.n, rt, pre, post, st); break;
+            switch (q) {
+                case 6: launch_quad<6>(ptrs, batch, z, st); break;
+                case 7: launch_quad<7>(ptrs, batch, z, st); break;
+                default: launch_quad<8>(ptrs, batch, z, st); break;
             }
         }
         ZK_HIP(hipGetLastError());
-        consumed += lrj;
     }
 }
 
