@@ -63,3 +63,31 @@ def test_many_parts_per_bucket(ctx, g2, n):
     for window in (4, 5):
         got, inf = (ctx.msm_g2 if g2 else ctx.msm_g1)(pts, sc, window)
         assert inf == expect_inf and np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("g2,n", [(False, 65), (False, 512), (False, 513), (False, 1100), (True, 65), (True, 513)])
+def test_oversized_bucket_chunks(ctx, g2, n):
+    """One bucket far above the mean load, at the edges of its chunks: equal,
+    opposite and infinite bases in every lane's sum, and bases that cancel."""
+    four = (mont_pts_g2 if g2 else mont_pts_g1)([1, pyref.R - 1, 0, 5])
+    for pattern in ([0], [0, 1], [3, 2, 0, 1, 0]):
+        pts = np.ascontiguousarray(four[np.resize(pattern, n)])
+        sc = scalars([1] * (n - 1) + [pyref.R - 1])
+        expect, expect_inf = (oracle_msm_g2 if g2 else oracle_msm_g1)(pts, sc)
+        got, inf = (ctx.msm_g2 if g2 else ctx.msm_g1)(pts, sc)
+        assert inf == expect_inf and (inf or np.array_equal(got, expect))
+
+
+def test_oversized_bucket_most_chunks(ctx):
+    """A bucket whose chunks grow because their number is bounded (above 2^19
+    entries), beside two light ones; sums of known multiples of the generator."""
+    n = 600001
+    three = mont_pts_g1([1, 2, 7])
+    pts = np.ascontiguousarray(three[np.arange(n) % 3])
+    vals = np.zeros((n, 4), np.uint64)
+    vals[:, 0] = 1
+    vals[:5, 0] = [9, 12, 0, 9, 3]
+    total = sum(int(v) * [1, 2, 7][i % 3] for i, v in enumerate(vals[:, 0]))
+    expect = mont_pts_g1([total])[0]
+    got, inf = ctx.msm_g1(pts, vals)
+    assert not inf and np.array_equal(got, expect)

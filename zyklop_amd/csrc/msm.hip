@@ -242,6 +242,30 @@ __global__ void __launch_bounds__(1024) k_sort_tile_scatter(const uint32_t* __re
     }
 }
 
+// Adds 1 to cnt[key] for every active lane; returns the count before it. Lanes
+// that share the first lane's key, and then the next one's, take one atomic
+// together where that saves many: the atomics of one address go one lane at a
+// time, and a bit-heavy witness sends a third of all entries to one bucket.
+ZK_DEV uint32_t lds_count(uint32_t* cnt, uint32_t key) {
+    uint32_t pos = 0;
+    bool todo = true;
+#pragma unroll
+    for (int round = 0; round < 2; round++) {
+        if (!todo) continue;
+        const uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)key);
+        const uint64_t same = __ballot(key == k0);
+        if (__popcll(same) < 8) break;
+        if (key == k0) {
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+            uint32_t base = 0;
+            if (rank == 0) base = atomicAdd(&cnt[k0], (uint32_t)__popcll(same));
+            pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + rank;
+            todo = false;
+        }
+    }
+    return todo ? atomicAdd(&cnt[key], 1u) : pos;
+}
+
 // Entries of a group go to their final positions through an LDS stage of
 // `stage_cap` words when the group fits (then the block writes its whole
 // range with coalesced stores), else straight to global memory: scattered
@@ -253,6 +277,10 @@ constexpr uint32_t SORT_GROUP_LDS_MAX = 160 * 1024 - 1024;
 // 16 waves per group: the LDS stage often leaves room for one workgroup per
 // CU, whose waves then carry the pass's LDS atomics and loads alone
 constexpr int SORT_GROUP_THREADS = 1024;
+// pairs each thread has in flight: a heavy group has one workgroup, whose loads
+// wait one after the other (245000 entries in one bucket 416 -> 179 us with
+// lds_count and 4; uniform 2^22 points' pass 344 -> 320 us, 8 no better)
+constexpr uint32_t SORT_UNROLL = 4;
 //
 // With scalar classes (cls_off non-null; the class is in bits 30..31 of a
 // pair's bucket word) the entries go out class by class: one pass over the
@@ -268,7 +296,14 @@ __global__ void __launch_bounds__(1024) k_sort_group(const uint2* __restrict__ p
     const uint32_t start = mscan[(size_t)g * nt], end = mscan[(size_t)(g + 1) * nt];
     for (uint32_t f = threadIdx.x; f < F; f += blockDim.x) cnt[f] = 0;
     __syncthreads();
-    for (uint32_t e = start + threadIdx.x; e < end; e += blockDim.x) atomicAdd(&cnt[pairs[e].y & mask], 1u);
+    for (uint32_t e = start + threadIdx.x; e < end; e += SORT_UNROLL * blockDim.x) {
+        uint32_t b[SORT_UNROLL];
+#pragma unroll
+        for (uint32_t j = 0; j < SORT_UNROLL; j++) b[j] = e + j * blockDim.x < end ? pairs[e + j * blockDim.x].y & mask : ~0u;
+#pragma unroll
+        for (uint32_t j = 0; j < SORT_UNROLL; j++)
+            if (b[j] != ~0u) lds_count(cnt, b[j]);
+    }
     __syncthreads();
     // exclusive scan of the counters: per-thread chunks, then the block scan
     const uint32_t q = (F + blockDim.x - 1) / blockDim.x, f0 = threadIdx.x * q;
@@ -302,12 +337,18 @@ __global__ void __launch_bounds__(1024) k_sort_group(const uint2* __restrict__ p
             }
             __syncthreads();
         }
-        for (uint32_t e = start + threadIdx.x; e < end; e += blockDim.x) {
-            const uint2 p = pairs[e];
-            if (cls_off && (int)(p.y >> 30) != k) continue;
-            const uint32_t pos = atomicAdd(&cnt[p.y & mask], 1u);
-            if (staged) stage[pos - start] = p.x;
-            else entries[pos] = p.x;
+        for (uint32_t e = start + threadIdx.x; e < end; e += SORT_UNROLL * blockDim.x) {
+            uint2 p[SORT_UNROLL];
+#pragma unroll
+            for (uint32_t j = 0; j < SORT_UNROLL; j++)
+                if (e + j * blockDim.x < end) p[j] = pairs[e + j * blockDim.x];
+#pragma unroll
+            for (uint32_t j = 0; j < SORT_UNROLL; j++) {
+                if (e + j * blockDim.x >= end || (cls_off && (int)(p[j].y >> 30) != k)) continue;
+                const uint32_t pos = lds_count(cnt, p[j].y & mask);
+                if (staged) stage[pos - start] = p[j].x;
+                else entries[pos] = p[j].x;
+            }
         }
     }
     if (staged) {
@@ -392,11 +433,12 @@ __global__ void __launch_bounds__(256) k_chunk_list(const uint32_t* __restrict__
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_over; i += gridDim.x * blockDim.x) {
         const uint32_t b = order[i];
         const uint32_t s0 = off[b], e0 = off[b + 1];
-        const uint32_t nch = (e0 - s0 + CHUNK - 1) / CHUNK;
+        const uint32_t parts = min((e0 - s0 + CHUNK - 1) / CHUNK, CHUNK_PARTS);
+        const uint32_t len = (e0 - s0 + parts - 1) / parts, nch = (e0 - s0 + len - 1) / len;
         const uint32_t first = atomicAdd(&counters[0], nch);
         for (uint32_t j = 0; j < nch; j++) {
-            const uint32_t c0 = s0 + j * CHUNK;
-            chunks[first + j] = {b, c0, min(CHUNK, e0 - c0), 0u};
+            const uint32_t c0 = s0 + j * len;
+            chunks[first + j] = {b, c0, min(len, e0 - c0), 0u};
         }
         const uint32_t li = atomicAdd(&counters[1], 1u);
         large[li] = {b, first, nch, 0u};
@@ -438,7 +480,9 @@ static SortShape sort_shape(size_t n, int c, bool merged) {
     z.qs = 0;
     while ((z.lmax >> z.qs) + 2 > 4096) z.qs++;
     z.nkey = (z.lmax >> z.qs) + 2;
-    z.max_chunks = z.ne / CHUNK + z.ne / L_MIN_LARGE + 2;
+    // ceil(len / CHUNK) <= len / L_MIN_LARGE for the len > L_MIN_LARGE entries of
+    // an oversized bucket
+    z.max_chunks = z.ne / L_MIN_LARGE + 2;
     z.max_large = z.ne / L_MIN_LARGE + 2;
     // a window of width wd spreads the 2n digits of its halves over 2^(wd-1)
     // magnitudes; the lowest buckets carry the most: those of the narrower

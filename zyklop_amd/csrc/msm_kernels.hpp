@@ -16,7 +16,8 @@
 namespace zk {
 
 constexpr uint32_t L_MIN_LARGE = 64;  // floor of the oversized-bucket threshold
-constexpr uint32_t CHUNK = 256 * 16;  // entries per chunk of an oversized bucket
+constexpr uint32_t CHUNK = 512;       // entries per chunk of an oversized bucket, or more:
+constexpr uint32_t CHUNK_PARTS = 1024;   // chunks per bucket at most
 // the tree reduction (k_msm_tree): threads per workgroup, nodes per workgroup
 // (18 KiB of LDS; one join per lane group in its first step)
 constexpr int TREE_THREADS = 256;
@@ -43,16 +44,6 @@ struct Red<Fp> {
     ZK_DEV static Pt add(const Pt& a, const Pt& b) { return f29_xyzz_add(a, b); }
     ZK_DEV static void pack(const Pt& p, uint32_t* w) { xyzz29_pack(p, w); }
     ZK_DEV static Pt unpack(const uint32_t* w) { return xyzz29_unpack(w); }
-    ZK_DEV static Pt from_std(const Xyzz<Fp>& s) {
-        if (xyzz_is_inf(s)) return xyzz29_inf();
-        Xyzz29 r;
-        r.X = f29_from_std(s.X);
-        r.Y = f29_from_std(s.Y);
-        r.ZZ = f29_from_std(s.ZZ);
-        r.ZZZ = f29_from_std(s.ZZZ);
-        r.inf = false;
-        return r;
-    }
 };
 template <>
 struct Red<Fq2> {
@@ -62,16 +53,6 @@ struct Red<Fq2> {
     ZK_DEV static Pt add(const Pt& a, const Pt& b) { return f29q_xyzz_add(a, b); }
     ZK_DEV static void pack(const Pt& p, uint32_t* w) { xyzz29q_pack(p, w); }
     ZK_DEV static Pt unpack(const uint32_t* w) { return xyzz29q_unpack(w); }
-    ZK_DEV static Pt from_std(const Xyzz<Fq2>& s) {
-        if (xyzz_is_inf(s)) return xyzz29q_inf();
-        Xyzz29q r;
-        r.X = f29q_from_std(s.X);
-        r.Y = f29q_from_std(s.Y);
-        r.ZZ = f29q_from_std(s.ZZ);
-        r.ZZZ = f29q_from_std(s.ZZZ);
-        r.inf = false;
-        return r;
-    }
 };
 
 // points of this form in memory: WORDS words each, 16-byte aligned
@@ -97,12 +78,6 @@ ZK_DEV void red_store(void* base, size_t i, const typename Red<T>::Pt& p) {
 #pragma unroll
     for (int k = 0; k < Red<T>::WORDS / 4; k++) o[k] = make_uint4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
 }
-// a bucket slot written from the standard form (oversized buckets, empty parts)
-template <class T>
-ZK_DEV void store_bucket(void* buckets, size_t slot, const Xyzz<T>& p) {
-    red_store<T>(buckets, slot, Red<T>::from_std(p));
-}
-
 // ---------------------------------------------------------------- buckets
 // Bucket accumulation, G1. One thread per bucket, in the sort's accumulation
 // order (longest first, so a wave's lanes carry near-equal loads and the
@@ -130,7 +105,7 @@ ZK_DEV bool acc_range(uint32_t tid, uint32_t nb, uint32_t split, const uint32_t*
     uint32_t s0 = offsets[b], e0 = offsets[b + 1];
     slot = b * split + h;
     if (e0 - s0 > lmax) {
-        if (h != 0) store_bucket<T>(buckets, slot, xyzz_inf<T>());
+        if (h != 0) red_store<T>(buckets, slot, Red<T>::inf());
         return false;
     }
     if (cls_off && range == MSM_RANGE_A) {
@@ -153,82 +128,150 @@ ZK_DEV Fp beta_mont(const uint32_t* c) {
     return b;
 }
 
-// the base an entry names (slot | half << 30, field29.hpp), read from the
-// 29-bit slots and returned in the standard form; an all-zero slot is the
-// point at infinity (0, 0)
-template <class T>
-ZK_DEV Aff<T> load_base(const void* pts29, uint32_t ref);
+// ---------------------------------------------------------------- oversized buckets
+// A lane's sum over entries of the 29-bit slots, by mixed additions: G1 in
+// registers, G2 with three coordinates in LDS (AccLds) as in the accumulation.
+// coord: coordinate q (X, Y, ZZ, ZZZ), component c, of the sum.
+template <class T> struct LaneSum;
 template <>
-ZK_DEV Aff<Fp> load_base<Fp>(const void* pts29, uint32_t ref) {
-    F29 x, y;
-    f29_load_point(pts29, ref, x, y);
-    return {f29_to_std(x), f29_to_std(y)};
-}
+struct LaneSum<Fp> {
+    static constexpr int LDS_WORDS = 1;
+    Xyzz29 a;
+    ZK_DEV explicit LaneSum(uint32_t*) { a = xyzz29_inf(); }
+    ZK_DEV void add(const void* pts, uint32_t ref) {
+        F29 x, y;
+        f29_load_point(pts, ref, x, y);
+        if (f29_is_zero(x) && f29_is_zero(y)) return;   // infinity
+        f29_madd(a, x, ref >> 31 ? f29_neg_lazy2(y) : y);
+    }
+    ZK_DEV bool inf() const { return a.inf; }
+    ZK_DEV F29 coord(int q, int) const { return q == 0 ? a.X : q == 1 ? a.Y : q == 2 ? a.ZZ : a.ZZZ; }
+};
 template <>
-ZK_DEV Aff<Fq2> load_base<Fq2>(const void* pts29, uint32_t ref) {
-    F29q x, y;
-    f29q_load_point(pts29, ref, x, y);
-    return {f29q_to_std(x), f29q_to_std(y)};
-}
+struct LaneSum<Fq2> {
+    static constexpr int LDS_WORDS = AccLds<64>::LDS_WORDS;
+    AccLds<64> a;
+    bool empty = true;
+    ZK_DEV explicit LaneSum(uint32_t* lds) : a{lds + threadIdx.x, {}} {}
+    ZK_DEV void add(const void* pts, uint32_t ref) {
+        F29q x, y;
+        f29q_load_point(pts, ref, x, y);
+        if (f29_is_zero(x.c0) && f29_is_zero(x.c1) && f29_is_zero(y.c0) && f29_is_zero(y.c1)) return;
+        if (ref >> 31) y = {f29_neg_lazy2(y.c0), f29_neg_lazy2(y.c1)};
+        f29q_madd(a, empty, x, y);
+    }
+    ZK_DEV bool inf() const { return empty; }
+    ZK_DEV F29 coord(int q, int c) const {
+        using L = AccLds<64>;
+        const F29q v = a.ld(q == 0 ? L::X : q == 1 ? L::Y : q == 2 ? L::ZZ : L::ZZZ);
+        return c ? v.c1 : v.c0;
+    }
+};
 
-// tree-sum of one XYZZ per thread across the block (blockDim.x must be a power of 2)
+// sum of the n = 2^k points of sh (coordinates of point i at (i*L + lane)*9, as
+// in k_msm_tree) by the block's lane groups, into point 0; one barrier per level
 template <class T>
-__device__ Xyzz<T> block_sum(Xyzz<T> v, Xyzz<T>* sh) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    for (int h = blockDim.x >> 1; h >= 1; h >>= 1) {
+ZK_DEV void tree_sum(uint32_t* sh, uint32_t n, const Coop<T>& k) {
+    constexpr uint32_t L = Coop<T>::LANES;
+    const uint32_t lane = threadIdx.x % L, grp = threadIdx.x / L, G = blockDim.x / L;
+    auto ld = [&](uint32_t i) {
+        F29 v;
+#pragma unroll
+        for (int l = 0; l < 9; l++) v.l[l] = sh[(i * L + lane) * 9 + l];
+        return v;
+    };
+#pragma unroll 1
+    for (uint32_t h = n / 2; h >= 1; h /= 2) {
         __syncthreads();
-        if (t < h) sh[t] = xyzz_add(sh[t], sh[t + h]);
+#pragma unroll 1
+        for (uint32_t i = grp; i < h; i += G) {
+            const F29 r = coop_add<T>(k, ld(i), ld(i + h));
+#pragma unroll
+            for (int l = 0; l < 9; l++) sh[(i * L + lane) * 9 + l] = r.l[l];
+        }
     }
     __syncthreads();
-    Xyzz<T> r = sh[0];
-    __syncthreads();
-    return r;
+}
+// point 0 of sh to point i of out, packed, by the first lane group
+template <class T>
+ZK_DEV void store_sum(const uint32_t* sh, void* out, size_t i) {
+    constexpr uint32_t L = Coop<T>::LANES;
+    if (threadIdx.x >= L) return;
+    const uint32_t lane = threadIdx.x;
+    F29 v;
+#pragma unroll
+    for (int l = 0; l < 9; l++) v.l[l] = sh[lane * 9 + l];
+    uint32_t w[8];
+    f29_pack(f29_reduce(v), w);   // X may be above 2^256
+    uint4* dst = reinterpret_cast<uint4*>(out) + (size_t)(Red<T>::WORDS / 4) * i + 2 * ((lane & 3) * (L / 4) + (lane >> 2));
+    dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
 }
 
-// one-wave workgroups with a small LDS tree (8 KiB for G1, 16 KiB for G2):
-// they must find CU slots while other streams' accumulations hold most of
-// the LDS, and with uniform scalars they have nothing to do
-constexpr int CHUNK_THREADS = 64;
-
-// one workgroup per chunk of an oversized bucket (grid-stride over the chunk list)
+// The chunked path of the oversized buckets: one wave per chunk, each lane
+// adding every 64th entry, then a tree over the 64 sums by lane groups; then one
+// workgroup per bucket adds its chunks' sums. Chunks are short (CHUNK entries, 8
+// per lane, but at most CHUNK_PARTS per bucket), since a bit-heavy witness has
+// one bucket with a third of the scalars and nothing else to fill the GPU:
+// 700001 points, 70 % of them bits, took 0.75 + 0.09 ms in the standard form with
+// 64 entries per lane, now 0.07 + 0.04 ms.
+// One-wave chunk workgroups with 9 KiB of LDS (G2 18): they must find CU slots
+// while other streams' accumulations hold most of the LDS, and with uniform
+// scalars they have nothing to do.
+constexpr int CHUNK_THREADS = 64, MERGE_THREADS = 256;
 template <class T>
 __global__ void __launch_bounds__(CHUNK_THREADS) k_msm_chunks(const uint32_t* __restrict__ entries,
                                                              const void* __restrict__ points29,
                                                              const uint32_t* __restrict__ counters,
                                                              const ChunkRec* __restrict__ chunks,
                                                              void* __restrict__ partials) {
-    __shared__ Xyzz<T> sh[CHUNK_THREADS];
+    constexpr int L = Coop<T>::LANES;
+    __shared__ uint32_t sh[CHUNK_THREADS * L * 9 > LaneSum<T>::LDS_WORDS ? CHUNK_THREADS * L * 9 : LaneSum<T>::LDS_WORDS];
+    const Coop<T> k(threadIdx.x % L);
     const uint32_t nch = counters[0];
     for (uint32_t ci = blockIdx.x; ci < nch; ci += gridDim.x) {
-        ChunkRec cr = chunks[ci];
-        Xyzz<T> acc = xyzz_inf<T>();
-        for (uint32_t e = threadIdx.x; e < cr.len; e += blockDim.x) {
-            uint32_t ref = entries[cr.start + e];
-            Aff<T> P = load_base<T>(points29, ref);
-            if (aff_is_inf(P)) continue;
-            if (ref >> 31) P.y = PointIO<T>::neg_y(P.y);
-            xyzz_madd(acc, P);
-        }
-        Xyzz<T> s = block_sum<T>(acc, sh);
-        if (threadIdx.x == 0) PointIO<T>::store_xyzz(partials, ci, s);
+        const ChunkRec cr = chunks[ci];
+        LaneSum<T> acc(sh);
+#pragma unroll 1
+        for (uint32_t e = threadIdx.x; e < cr.len; e += CHUNK_THREADS) acc.add(points29, entries[cr.start + e]);
+        F29 v[L];
+        const bool inf = acc.inf();
+#pragma unroll
+        for (int j = 0; j < L; j++) v[j] = inf ? F29{} : acc.coord(j & 3, j >> 2);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < L; j++)
+#pragma unroll
+            for (int l = 0; l < 9; l++) sh[(threadIdx.x * L + j) * 9 + l] = v[j].l[l];
+        tree_sum<T>(sh, CHUNK_THREADS, k);
+        store_sum<T>(sh, partials, ci);
+        __syncthreads();
     }
 }
 
 // one workgroup per oversized bucket: sum its chunk partials
 template <class T>
-__global__ void __launch_bounds__(CHUNK_THREADS) k_msm_merge(const uint32_t* __restrict__ counters, const LargeRec* __restrict__ large,
-                                                   const void* __restrict__ partials, uint32_t split,
-                                                   void* __restrict__ buckets) {
-    __shared__ Xyzz<T> sh[CHUNK_THREADS];
+__global__ void __launch_bounds__(MERGE_THREADS) k_msm_merge(const uint32_t* __restrict__ counters,
+                                                            const LargeRec* __restrict__ large,
+                                                            const void* __restrict__ partials, uint32_t split,
+                                                            void* __restrict__ buckets) {
+    constexpr int L = Coop<T>::LANES, G = MERGE_THREADS / L;
+    __shared__ uint32_t sh[G * L * 9];
+    const uint32_t lane = threadIdx.x % L, grp = threadIdx.x / L;
+    const Coop<T> k(lane);
+    const uint4* src = reinterpret_cast<const uint4*>(partials) + 2 * ((lane & 3) * (L / 4) + (lane >> 2));
     const uint32_t nl = counters[1];
     for (uint32_t li = blockIdx.x; li < nl; li += gridDim.x) {
-        LargeRec lr = large[li];
-        Xyzz<T> acc = xyzz_inf<T>();
-        for (uint32_t j = threadIdx.x; j < lr.count; j += blockDim.x)
-            acc = xyzz_add(acc, PointIO<T>::load_xyzz(partials, lr.first + j));
-        Xyzz<T> s = block_sum<T>(acc, sh);
-        if (threadIdx.x == 0) store_bucket<T>(buckets, (size_t)lr.bucket * split, s);
+        const LargeRec lr = large[li];
+        F29 v{};
+#pragma unroll 1
+        for (uint32_t j = grp; j < lr.count; j += G)
+            v = coop_add<T>(k, v, f29_load_packed(src + (size_t)(Red<T>::WORDS / 4) * (lr.first + j)));
+#pragma unroll
+        for (int l = 0; l < 9; l++) sh[(grp * L + lane) * 9 + l] = v.l[l];
+        tree_sum<T>(sh, G, k);
+        store_sum<T>(sh, buckets, (size_t)lr.bucket * split);
+        __syncthreads();
     }
 }
 
@@ -363,11 +406,11 @@ static void launch_pre_t(const MsmSort& sort, const void* d_points29, MsmScratch
     const MsmGeom g = msm_geom(sort.n, sort.g.c, g2, sort.g.merged);
     scr.ensure(g, sort.n_chunk_max, g2, split);
     scr.split = split;
-    k_msm_chunks<T><<<256, CHUNK_THREADS, 0, st>>>(sort.entries.as<uint32_t>(), d_points29,
+    k_msm_chunks<T><<<CHUNK_PARTS, CHUNK_THREADS, 0, st>>>(sort.entries.as<uint32_t>(), d_points29,
                                                    sort.counters.as<uint32_t>(), sort.chunks.as<ChunkRec>(),
                                                    scr.partials.p);
     ZK_HIP(hipGetLastError());
-    k_msm_merge<T><<<64, CHUNK_THREADS, 0, st>>>(sort.counters.as<uint32_t>(), sort.large.as<LargeRec>(), scr.partials.p,
+    k_msm_merge<T><<<16, MERGE_THREADS, 0, st>>>(sort.counters.as<uint32_t>(), sort.large.as<LargeRec>(), scr.partials.p,
                                          (uint32_t)split, scr.buckets.p);
     ZK_HIP(hipGetLastError());
 }
