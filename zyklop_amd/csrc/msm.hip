@@ -121,23 +121,6 @@ int msm_table_c(size_t n) {
     return best;
 }
 
-// ---------------------------------------------------------------- GLV split
-// Every scalar k_i becomes two half scalars (glv.hpp): half[i] = k1 for P_i and
-// half[n + i] = k2 for lambda*P_i, each a 127-bit magnitude with its sign in
-// bit 127 (4 x u32 LE).
-__global__ void k_glv_split(const uint32_t* __restrict__ sc, size_t n, uint4* __restrict__ half) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint4* p = reinterpret_cast<const uint4*>(sc) + 2 * i;
-    const uint4 a = p[0], b = p[1];
-    const uint64_t k[4] = {a.x | (uint64_t)a.y << 32, a.z | (uint64_t)a.w << 32, b.x | (uint64_t)b.y << 32,
-                           b.z | (uint64_t)b.w << 32};
-    uint64_t k1[2], k2[2];
-    glv::split(k, k1, k2);
-    half[i] = make_uint4((uint32_t)k1[0], (uint32_t)(k1[0] >> 32), (uint32_t)k1[1], (uint32_t)(k1[1] >> 32));
-    half[n + i] = make_uint4((uint32_t)k2[0], (uint32_t)(k2[0] >> 32), (uint32_t)k2[1], (uint32_t)(k2[1] >> 32));
-}
-
 // ---------------------------------------------------------------- digits
 // Signed digits of a half scalar, least significant window first, window w
 // being c - 1 bits wide for w < nlo and c bits above (128 bits in all):
@@ -150,8 +133,7 @@ struct DigitIter {
     uint32_t s[4];
     uint32_t carry, c, left;
     bool flip;
-    ZK_DEV void init(const uint32_t* hs, size_t i, int cc, int nlo) {
-        const uint4 a = reinterpret_cast<const uint4*>(hs)[i];
+    ZK_DEV void init(const uint4& a, int cc, int nlo) {
         s[0] = a.x; s[1] = a.y; s[2] = a.z; s[3] = a.w & 0x7fffffffu;
         flip = (a.w >> 31) != 0;
         carry = 0;
@@ -182,61 +164,85 @@ struct DigitIter {
 // Two-pass LDS radix sort of the flat bucket ids b = w*Kw + |digit| - 1 of all
 // nonzero digits (no global atomics; Kw = K, or 0 when all windows share one
 // set of buckets). Buckets are grouped by b >> s.
-// Pass A, per tile of scalars: an LDS histogram of groups goes to a count
-// matrix [group][tile]; a device scan of the matrix gives every tile its run
-// inside every group; the tile then writes (entry, b) pairs at run + LDS rank.
+// Pass A, per tile of scalars: the GLV split (glv.hpp) of every scalar k_i into
+// two half scalars, half[i] = k1 for P_i and half[n + i] = k2 for lambda*P_i,
+// each a 127-bit magnitude with its sign in bit 127, and an LDS histogram of
+// their digits' groups into a count matrix [group][tile]; a device scan of the
+// matrix gives every tile its run inside every group; the tile then writes
+// (entry, b) pairs at run + LDS rank.
 // Pass B, per group: LDS counts of its 2^s buckets give the bucket offsets,
 // then the entries go to offset + LDS rank.
-__global__ void __launch_bounds__(1024) k_sort_tile_hist(const uint32_t* __restrict__ sc, size_t n, size_t tile, int c,
+//
+// The first block also clears what later kernels of the sort count into
+// (SortZero): the matrix's last element, the load histograms, the chunk counters.
+struct SortZero {
+    uint32_t* end;
+    uint32_t* hist;
+    uint32_t nhist;
+    uint32_t* counters;
+};
+__global__ void __launch_bounds__(1024) k_sort_tile_hist(const uint4* __restrict__ sc, size_t n, size_t tile, int c,
                                                          int nlo, int W, uint32_t Kw, int s, uint32_t G, uint32_t nt,
-                                                         uint32_t* __restrict__ matrix) {
+                                                         uint32_t* __restrict__ matrix, uint4* __restrict__ half,
+                                                         SortZero z) {
     extern __shared__ uint32_t lh[];
     for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) lh[k] = 0;
+    if (blockIdx.x == 0) {
+        for (uint32_t k = threadIdx.x; k < z.nhist; k += blockDim.x) z.hist[k] = 0;
+        if (threadIdx.x < 16) z.counters[threadIdx.x] = 0;
+        if (threadIdx.x == 0) *z.end = 0;
+    }
     __syncthreads();
     const size_t i0 = (size_t)blockIdx.x * tile, i1 = i0 + tile < n ? i0 + tile : n;
     for (size_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        DigitIter it;
-        it.init(sc, i, c, nlo);
-        for (int w = 0; w < W; w++) {
-            bool ng;
-            uint32_t mag = it.next(ng);
-            if (mag) atomicAdd(&lh[((uint32_t)w * Kw + mag - 1) >> s], 1u);
+        const uint4 a = sc[2 * i], b = sc[2 * i + 1];
+        const uint64_t k[4] = {a.x | (uint64_t)a.y << 32, a.z | (uint64_t)a.w << 32, b.x | (uint64_t)b.y << 32,
+                               b.z | (uint64_t)b.w << 32};
+        uint64_t kh[2][2];
+        glv::split(k, kh[0], kh[1]);
+#pragma unroll 1
+        for (int h = 0; h < 2; h++) {
+            const uint64_t lo = h ? kh[1][0] : kh[0][0], hi = h ? kh[1][1] : kh[0][1];
+            const uint4 v = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+            half[h * n + i] = v;
+            DigitIter it;
+            it.init(v, c, nlo);
+            for (int w = 0; w < W; w++) {
+                bool ng;
+                uint32_t mag = it.next(ng);
+                if (mag) atomicAdd(&lh[((uint32_t)w * Kw + mag - 1) >> s], 1u);
+            }
         }
     }
     __syncthreads();
     for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) matrix[(size_t)k * nt + blockIdx.x] = lh[k];
 }
 
-// n here counts half scalars (2 per scalar); entry of half i in window w:
-// slot (i mod n/2) + w*sw (sw = n/2 for window tables, else 0), half
-// i >= n/2, sign
-__global__ void __launch_bounds__(1024) k_sort_tile_scatter(const uint32_t* __restrict__ sc, size_t n, size_t tile, int c,
+// entry of half h of scalar i in window w: slot i + w*sw (sw = n for window
+// tables, else 0), half, sign
+__global__ void __launch_bounds__(1024) k_sort_tile_scatter(const uint4* __restrict__ half, size_t n, size_t tile, int c,
                                                             int nlo, int W, uint32_t Kw, uint32_t sw, int s, uint32_t G,
                                                             uint32_t nt, const uint32_t* __restrict__ mscan,
                                                             const uint8_t* __restrict__ cls, uint2* __restrict__ pairs) {
-    extern __shared__ uint32_t lds[];
-    uint32_t* base = lds;       // this tile's run start in each group
-    uint32_t* rank = lds + G;   // next rank in each group
-    for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) {
-        base[k] = mscan[(size_t)k * nt + blockIdx.x];
-        rank[k] = 0;
-    }
+    extern __shared__ uint32_t lds[];   // where this tile's next pair of each group goes
+    for (uint32_t k = threadIdx.x; k < G; k += blockDim.x) lds[k] = mscan[(size_t)k * nt + blockIdx.x];
     __syncthreads();
     const size_t i0 = (size_t)blockIdx.x * tile, i1 = i0 + tile < n ? i0 + tile : n;
-    const uint32_t nh = (uint32_t)(n >> 1);
     for (size_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        DigitIter it;
-        it.init(sc, i, c, nlo);
-        const bool phi = (uint32_t)i >= nh;
-        const uint32_t ref0 = ((uint32_t)i - (phi ? nh : 0u)) | (phi ? 0x40000000u : 0u);
-        const uint32_t ctag = cls ? (uint32_t)cls[(uint32_t)i - (phi ? nh : 0u)] << 30 : 0u;
-        for (int w = 0; w < W; w++) {
-            bool ng;
-            uint32_t mag = it.next(ng);
-            if (mag) {
-                const uint32_t b = (uint32_t)w * Kw + mag - 1, g = b >> s;
-                const uint32_t pos = base[g] + atomicAdd(&rank[g], 1u);
-                pairs[pos] = make_uint2((ref0 + (uint32_t)w * sw) | (ng ? 0x80000000u : 0u), b | ctag);
+        const uint32_t ctag = cls ? (uint32_t)cls[i] << 30 : 0u;
+#pragma unroll 1
+        for (int h = 0; h < 2; h++) {
+            DigitIter it;
+            it.init(half[h * n + i], c, nlo);
+            const uint32_t ref0 = (uint32_t)i | (h ? 0x40000000u : 0u);
+            for (int w = 0; w < W; w++) {
+                bool ng;
+                uint32_t mag = it.next(ng);
+                if (mag) {
+                    const uint32_t b = (uint32_t)w * Kw + mag - 1;
+                    pairs[atomicAdd(&lds[b >> s], 1u)] =
+                        make_uint2((ref0 + (uint32_t)w * sw) | (ng ? 0x80000000u : 0u), b | ctag);
+                }
             }
         }
     }
@@ -424,26 +430,69 @@ __global__ void __launch_bounds__(1024) k_load_scatter(const uint32_t* __restric
     if (b < nb) out[lh[key] + rank - base] = b;
 }
 
+// chunk list entries of oversized bucket b (k_msm_chunks, k_msm_merge)
+__device__ inline void list_chunks(uint32_t b, const uint32_t* off, uint32_t* counters, ChunkRec* chunks, LargeRec* large) {
+    const uint32_t s0 = off[b], e0 = off[b + 1];
+    const uint32_t parts = min((e0 - s0 + CHUNK - 1) / CHUNK, CHUNK_PARTS);
+    const uint32_t len = (e0 - s0 + parts - 1) / parts, nch = (e0 - s0 + len - 1) / len;
+    const uint32_t first = atomicAdd(&counters[0], nch);
+    for (uint32_t j = 0; j < nch; j++) {
+        const uint32_t c0 = s0 + j * len;
+        chunks[first + j] = {b, c0, min(len, e0 - c0), 0u};
+    }
+    const uint32_t li = atomicAdd(&counters[1], 1u);
+    large[li] = {b, first, nch, 0u};
+}
+
 // Chunk lists of the oversized buckets (load key 0, first in the accumulation
 // order): one thread per oversized bucket, grid-stride; hist[0] is their count.
 __global__ void __launch_bounds__(256) k_chunk_list(const uint32_t* __restrict__ order, const uint32_t* __restrict__ off,
                                                     const uint32_t* __restrict__ hist, uint32_t* __restrict__ counters,
                                                     ChunkRec* __restrict__ chunks, LargeRec* __restrict__ large) {
     const uint32_t n_over = hist[0];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_over; i += gridDim.x * blockDim.x) {
-        const uint32_t b = order[i];
-        const uint32_t s0 = off[b], e0 = off[b + 1];
-        const uint32_t parts = min((e0 - s0 + CHUNK - 1) / CHUNK, CHUNK_PARTS);
-        const uint32_t len = (e0 - s0 + parts - 1) / parts, nch = (e0 - s0 + len - 1) / len;
-        const uint32_t first = atomicAdd(&counters[0], nch);
-        for (uint32_t j = 0; j < nch; j++) {
-            const uint32_t c0 = s0 + j * len;
-            chunks[first + j] = {b, c0, min(len, e0 - c0), 0u};
-        }
-        const uint32_t li = atomicAdd(&counters[1], 1u);
-        large[li] = {b, first, nch, 0u};
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_over; i += gridDim.x * blockDim.x)
+        list_chunks(order[i], off, counters, chunks, large);
+}
+
+// The three kernels above for few buckets, in one workgroup per order: the
+// histogram and its scan stay in LDS. The whole buckets' order (the last) also
+// lists the chunks.
+__global__ void __launch_bounds__(1024) k_order_small(const uint32_t* __restrict__ off, const uint32_t* __restrict__ cls_off,
+                                                      uint32_t nb, uint32_t lmax, int qs, uint32_t nkey,
+                                                      uint32_t* __restrict__ order_a, uint32_t* __restrict__ order_b,
+                                                      uint32_t* __restrict__ order, uint32_t* __restrict__ counters,
+                                                      ChunkRec* __restrict__ chunks, LargeRec* __restrict__ large) {
+    extern __shared__ uint32_t lh[];
+    __shared__ uint32_t wsum[16];
+    const int range = order_range(cls_off);
+    uint32_t* out = range == MSM_RANGE_A ? order_a : range == MSM_RANGE_B ? order_b : order;
+    for (uint32_t k = threadIdx.x; k < nkey; k += blockDim.x) lh[k] = 0;
+    __syncthreads();
+    for (uint32_t b = threadIdx.x; b < nb; b += blockDim.x)
+        atomicAdd(&lh[load_key(off, cls_off, range, b, lmax, qs, nkey)], 1u);
+    __syncthreads();
+    const uint32_t per = (nkey + blockDim.x - 1) / blockDim.x, k0 = threadIdx.x * per;
+    const uint32_t k1 = k0 + per < nkey ? k0 + per : nkey;
+    uint32_t sum = 0, total;
+    for (uint32_t k = k0; k < k1; k++) sum += lh[k];
+    uint32_t run = block_exclusive_scan(sum, wsum, &total);
+    for (uint32_t k = k0; k < k1; k++) {
+        const uint32_t v = lh[k];
+        lh[k] = run;
+        run += v;
+    }
+    __syncthreads();
+    for (uint32_t b = threadIdx.x; b < nb; b += blockDim.x) {
+        const uint32_t key = load_key(off, cls_off, range, b, lmax, qs, nkey);
+        out[atomicAdd(&lh[key], 1u)] = b;
+        if (key == 0 && range == MSM_RANGE_ALL) list_chunks(b, off, counters, chunks, large);
     }
 }
+
+// bucket sets up to here are ordered by one workgroup per order (k_order_small):
+// one launch of 4 us instead of four; at 2^15 its 32 rounds take longer than the
+// launches (8 proofs of 50021 constraints 6.12 against 6.24 ms)
+constexpr size_t ORDER_SMALL = 16384;
 
 // sizes of one digit sort over n scalars at window c (shared by reserve and run)
 struct SortShape {
@@ -454,7 +503,7 @@ struct SortShape {
     int sh, qs;
 };
 
-static SortShape sort_shape(size_t n, int c, bool merged) {
+static SortShape sort_shape(size_t n, int c, bool merged, size_t min_tile = 64) {
     ZK_REQUIRE(n < 0x40000000ull, ZK_E_ARG, "MSM size must be < 2^30");
     SortShape z;
     z.g = msm_geom(n, c, false, merged);
@@ -467,11 +516,16 @@ static SortShape sort_shape(size_t n, int c, bool merged) {
     z.sh = 7;
     while (((z.nb + (1ull << z.sh) - 1) >> z.sh) > 4096) z.sh++;
     z.G = (uint32_t)((z.nb + (1ull << z.sh) - 1) >> z.sh);
-    // tiles of pass A: multiples of 4096 scalars, at most 512 tiles (two
+    // tiles of pass A: up to 2^19 scalars, powers of two from 64 (one wave) to
+    // 2048 that make at most 256 tiles, since a tile's digits go through one
+    // CU's LDS atomics one after the other (1000 scalars, 22 windows: one tile 39
+    // + 40 us, 16 tiles 12 + 11); above, multiples of 2048, at most 512 tiles (two
     // workgroups per CU): longer runs per group and tile for the pair writes,
     // whose short runs wrote several times their bytes
-    z.tile = (size_t)4096 * std::max<size_t>(1, (z.n2 + 4096 * 512 - 1) / (4096 * 512));
-    z.nt = (uint32_t)std::max<size_t>(1, (z.n2 + z.tile - 1) / z.tile);
+    z.tile = min_tile;
+    while (z.tile < 2048 && z.tile * 256 < n) z.tile *= 2;
+    if (z.tile == 2048) z.tile *= std::max<size_t>(1, (n + 2048 * 512 - 1) / (2048 * 512));
+    z.nt = (uint32_t)std::max<size_t>(1, (n + z.tile - 1) / z.tile);
     z.mlen = (size_t)z.G * z.nt + 1;
     z.ne = std::max<size_t>(1, (size_t)z.g.W * z.n2);
     // accumulation order. Oversized threshold: 8x the mean bucket load
@@ -542,7 +596,7 @@ size_t MsmSort::count_reserve(size_t n_, int c, GrowCount& gc, bool merged, bool
 }
 
 void MsmSort::run(const void* d_scalars, size_t n_, int c, hipStream_t st, bool merged, const uint8_t* cls) {
-    const SortShape z = sort_shape(n_, c, merged);
+    const SortShape z = sort_shape(n_, c, merged, min_tile);
     sort_reserve(*this, z);
     if (cls) class_buffers(*this, z, [](DevBuf& b, size_t n) { b.ensure(n); });
     n = n_;
@@ -552,29 +606,31 @@ void MsmSort::run(const void* d_scalars, size_t n_, int c, hipStream_t st, bool 
     qs = z.qs;
     nkey = z.nkey;
     n_chunk_max = z.max_chunks;
-    const size_t n2 = z.n2, nb = z.nb, tile = z.tile, mlen = z.mlen;
+    const size_t nb = z.nb, tile = z.tile, mlen = z.mlen;
     const uint32_t G = z.G, nt = z.nt;
     const int sh = z.sh;
-    if (n) {
-        k_glv_split<<<cdiv(n, 256), 256, 0, st>>>((const uint32_t*)d_scalars, n, half.as<uint4>());
-        ZK_HIP(hipGetLastError());
-    }
-    const uint32_t* hs = half.as<uint32_t>();
     uint32_t* mat = matrix.as<uint32_t>();
     uint32_t* msc = mscan.as<uint32_t>();
+    // accumulation orders: the whole buckets', and with classes also those of
+    // the A and B parts, in one histogram, scan and scatter
+    const uint32_t nord = classes ? 3 : 1;
+    uint32_t* h = (classes ? okeys : lkeys).as<uint32_t>();
     if (n) {
-        k_sort_tile_hist<<<nt, 1024, G * 4, st>>>(hs, n2, tile, g.c, g.nlo, g.W, merged ? 0u : g.K, sh, G, nt, mat);
+        const unsigned threads = (unsigned)std::min<size_t>(1024, tile);
+        const SortZero zero{mat + mlen - 1, h, nord * nkey, counters.as<uint32_t>()};
+        k_sort_tile_hist<<<nt, threads, G * 4, st>>>((const uint4*)d_scalars, n, tile, g.c, g.nlo, g.W,
+                                                     merged ? 0u : g.K, sh, G, nt, mat, half.as<uint4>(), zero);
         ZK_HIP(hipGetLastError());
-        fill_u32(mat + mlen - 1, 0u, 1, st);
+        exclusive_scan(mat, msc, msc + mlen, mlen, st);
+        k_sort_tile_scatter<<<nt, threads, G * 4, st>>>(half.as<uint4>(), n, tile, g.c, g.nlo, g.W, merged ? 0u : g.K,
+                                                        merged ? (uint32_t)n : 0u, sh, G, nt, msc, cls,
+                                                        pairs.as<uint2>());
+        ZK_HIP(hipGetLastError());
     } else {
         fill_u32(mat, 0u, mlen, st);
-    }
-    exclusive_scan(mat, msc, msc + mlen, mlen, st);
-    if (n) {
-        k_sort_tile_scatter<<<nt, 1024, 2 * G * 4, st>>>(hs, n2, tile, g.c, g.nlo, g.W, merged ? 0u : g.K,
-                                                          merged ? (uint32_t)n : 0u, sh, G, nt, msc, cls,
-                                                          pairs.as<uint2>());
-        ZK_HIP(hipGetLastError());
+        fill_u32(h, 0u, nord * nkey, st);
+        fill_u32(counters.as<uint32_t>(), 0u, 16, st);
+        exclusive_scan(mat, msc, msc + mlen, mlen, st);
     }
     // stage for the heaviest group uniform scalars give, plus a margin
     // (group sizes are sums of many digits, so larger ones are rare and take
@@ -596,15 +652,17 @@ void MsmSort::run(const void* d_scalars, size_t n_, int c, hipStream_t st, bool 
                                                                 cls ? cls_off.as<uint32_t>() : nullptr);
     ZK_HIP(hipGetLastError());
     const uint32_t* off = offsets.as<uint32_t>();
-    uint32_t* hist = lkeys.as<uint32_t>();
-    const unsigned nblk_o = (unsigned)cdiv(nb, 1024);
     const uint32_t* co = classes ? cls_off.as<uint32_t>() : nullptr;
-    // accumulation orders: the whole buckets', and with classes also those of
-    // the A and B parts, in one histogram, scan and scatter
-    const uint32_t nord = classes ? 3 : 1;
-    uint32_t* h = classes ? okeys.as<uint32_t>() : hist;
+    if (nb <= ORDER_SMALL) {
+        k_order_small<<<dim3(1, nord), 1024, nkey * 4, st>>>(off, co, (uint32_t)nb, lmax, qs, nkey,
+                                                             order_a.as<uint32_t>(), order_b.as<uint32_t>(),
+                                                             order.as<uint32_t>(), counters.as<uint32_t>(),
+                                                             chunks.as<ChunkRec>(), large.as<LargeRec>());
+        ZK_HIP(hipGetLastError());
+        return;
+    }
+    const unsigned nblk_o = (unsigned)cdiv(nb, 1024);
     uint32_t* cur = h + nord * nkey;
-    fill_u32(h, 0u, nord * nkey, st);
     k_load_hist<<<dim3(nblk_o, nord), 1024, nkey * 4, st>>>(off, co, (uint32_t)nb, lmax, qs, nkey, h);
     ZK_HIP(hipGetLastError());
     exclusive_scan(h, cur, cur + nord * nkey, nord * nkey, st);
@@ -612,11 +670,10 @@ void MsmSort::run(const void* d_scalars, size_t n_, int c, hipStream_t st, bool 
                                                               order_a.as<uint32_t>(), order_b.as<uint32_t>(),
                                                               order.as<uint32_t>());
     ZK_HIP(hipGetLastError());
-    hist = h + (nord - 1) * nkey;   // the whole buckets' histogram: hist[0] oversized
-    // chunk lists of the oversized buckets, shared by every MSM over this sort
-    fill_u32(counters.as<uint32_t>(), 0u, 16, st);
-    k_chunk_list<<<64, 256, 0, st>>>(order.as<uint32_t>(), off, hist, counters.as<uint32_t>(), chunks.as<ChunkRec>(),
-                                     large.as<LargeRec>());
+    // chunk lists of the oversized buckets (hist[0] of the whole buckets' order),
+    // shared by every MSM over this sort
+    k_chunk_list<<<64, 256, 0, st>>>(order.as<uint32_t>(), off, h + (nord - 1) * nkey, counters.as<uint32_t>(),
+                                     chunks.as<ChunkRec>(), large.as<LargeRec>());
     ZK_HIP(hipGetLastError());
 }
 
@@ -777,22 +834,30 @@ zkh::Xyzz<zkh::Fp> msm_g1_noalloc(int device, const void* d_points, const void* 
         if (device >= 0 && device < NOALLOC_MAX_DEVICES) base = g_noalloc_ptr[device];
     }
     ZK_REQUIRE(base != nullptr, ZK_E_STATE, "fixed MSM scratch not set up on this device");
-    const SortShape z = sort_shape(n, window, false);
+    SortShape z = sort_shape(n, window, false);
     const MsmGeom& g = z.g;
     // the same buffers the allocating path sizes, laid out in the array; fewer
-    // threads per bucket where that makes them fit
+    // threads per bucket, then fewer tiles, where that makes them fit
     MsmSort sort;
     MsmScratch scr;
     DevBuf p29;
     size_t need = 0;
     auto count = [&](const DevBuf&, size_t b) { need = ((need + 255) & ~(size_t)255) + b; };
     int split = msm_alone_split(n, g.c, false);
-    for (;; split = split > 4 ? split / 2 : split - 1) {
+    for (;;) {
         need = 0;
         sort_buffers(sort, z, count);
         scratch_buffers(scr, g, z.max_chunks, false, split, count);
         count(p29, std::max<size_t>(n, 1) * PT29_BYTES);
-        if (need <= MSM_NOALLOC_SCRATCH_BYTES || split == 1) break;
+        if (need <= MSM_NOALLOC_SCRATCH_BYTES) break;
+        if (split > 1) {
+            split = split > 4 ? split / 2 : split - 1;
+        } else if (sort.min_tile < 2048) {
+            sort.min_tile = 2048;
+            z = sort_shape(n, window, false, sort.min_tile);
+        } else {
+            break;
+        }
     }
     ZK_REQUIRE(need <= MSM_NOALLOC_SCRATCH_BYTES, ZK_E_ARG,
                "MSM of " + std::to_string(n) + " points at window " + std::to_string(g.c) + " needs " +

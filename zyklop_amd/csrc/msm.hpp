@@ -109,6 +109,7 @@ struct MsmSort {
     // chunk lists of the oversized buckets (above lmax entries), built by run()
     DevBuf chunks, large, counters;
     size_t n_chunk_max = 0;
+    size_t min_tile = 64;         // scalars per tile at least (2^6 .. 2^11): more need less memory
     // sizes every buffer a sort of n scalars at window c needs (no launch),
     // with_classes: also cls_off, order_a, order_b and okeys; returns the
     // chunk-list capacity for MsmScratch::ensure

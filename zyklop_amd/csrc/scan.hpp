@@ -83,8 +83,32 @@ __global__ void k_scan_add(uint32_t* __restrict__ out, const uint32_t* __restric
     if (i < n) out[i] += tile_sums[i / SCAN_TILE];
 }
 
+// n <= SCAN_ONE: one workgroup, consecutive elements per thread
+constexpr size_t SCAN_ONE = 32768;
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_one(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                           uint32_t n) {
+    __shared__ uint32_t lds[16];
+    const uint32_t per = (n + SCAN_THREADS - 1) / SCAN_THREADS, i0 = threadIdx.x * per;
+    const uint32_t i1 = i0 + per < n ? i0 + per : n;
+    uint32_t s = 0, total;
+#pragma unroll 4
+    for (uint32_t i = i0; i < i1; i++) s += in[i];
+    uint32_t ex = block_exclusive_scan(s, lds, &total);
+#pragma unroll 4
+    for (uint32_t i = i0; i < i1; i++) {
+        const uint32_t v = in[i];
+        out[i] = ex;
+        ex += v;
+    }
+}
+
 // out[0..n) = exclusive scan of in[0..n); tmp needs >= cdiv(n, SCAN_TILE) u32.
 inline void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t* tmp, size_t n, hipStream_t st) {
+    if (n <= SCAN_ONE) {
+        k_scan_one<<<1, SCAN_THREADS, 0, st>>>(in, out, (uint32_t)n);
+        ZK_HIP(hipGetLastError());
+        return;
+    }
     unsigned tiles = cdiv(n, SCAN_TILE);
     ZK_REQUIRE(tiles <= (unsigned)SCAN_TILE, ZK_E_ARG, "scan too large");
     k_scan_tiles<<<tiles, SCAN_THREADS, 0, st>>>(in, out, tmp, n);
