@@ -161,7 +161,8 @@ int zk_set_batch_slots(zk_ctx* ctx, int n);
  * proof finished by zk_prove / zk_prove_device on ctx:
  *  [0] SpMV (+ witness copy) ms   [1] 3 x iNTT+coset ms   [2] 3 x NTT ms
  *  [3] h + sort(h) ms             [4] shared witness sort ms
- *  [5..9]  bucket-accumulation kernel ms for A, B1, C, B2, H
+ *  [5..9]  bucket-accumulation kernel ms for A, B1, C, B2, H (A, B1 and C run
+ *  in one launch, whose time each of them shows)
  *  [10..14] whole MSM (accumulation .. partials on host) ms, same order
  *  [15] digit entries of the witness sort  [16] of the h sort
  *  [17] window c (witness) [18] c (h) [19] windows W (witness) [20] W (h)

@@ -94,7 +94,7 @@ void check_scalars(const uint64_t* sc, size_t n) {
 }
 
 zk::ProveSlot& ctx_slot(zk_ctx* ctx) {
-    if (!ctx->impl.slot) ctx->impl.slot = std::make_unique<zk::ProveSlot>();
+    if (!ctx->impl.slot) ctx->impl.slot = std::make_unique<zk::ProveSlot>(ctx->impl);
     return *ctx->impl.slot;
 }
 
@@ -191,8 +191,7 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
     sort.run(d_scalars, n, window, st, merged, cls);
     ZK_HIP(hipEventRecord(ctx->ev1, st));
     const void* pts = slots29 ? slots29 : p29.p;
-    zk::msm_launch_pre(sort, pts, g2, scr, st, split > 0 ? split : zk::msm_alone_split(n, sort.g.c, g2));
-    zk::msm_launch_main(sort, g2, scr, part, st, pts, range);
+    zk::msm_launch(sort, g2, {pts, &scr, &part, range}, st, split > 0 ? split : zk::msm_alone_split(n, sort.g.c, g2));
     ZK_HIP(hipEventRecord(ctx->ev2, st));
     const size_t nb = (size_t)sort.g.Wr * sort.g.K;
     use.w->entries.ensure(4);
@@ -300,7 +299,7 @@ int zk_prove(zk_ctx* ctx, const zk_circuit* c, const uint64_t* witness, uint32_t
         std::lock_guard<std::mutex> lk(ctx->impl.mu);
         ZK_HIP(hipSetDevice(ctx->impl.device));
         zk::ProveSlot& sl = ctx_slot(ctx);
-        sl.enqueue(ctx->impl, *c->impl, witness, false, r, s, true);
+        sl.enqueue(ctx->impl, *c->impl, witness, false, r, s);
         sl.finish(out);
     });
 }
@@ -312,7 +311,7 @@ int zk_prove_device(zk_ctx* ctx, const zk_circuit* c, const void* d_witness, con
         std::lock_guard<std::mutex> lk(ctx->impl.mu);
         ZK_HIP(hipSetDevice(ctx->impl.device));
         zk::ProveSlot& sl = ctx_slot(ctx);
-        sl.enqueue(ctx->impl, *c->impl, (const uint64_t*)d_witness, true, r, s, true);
+        sl.enqueue(ctx->impl, *c->impl, (const uint64_t*)d_witness, true, r, s);
         sl.finish(out);
     });
 }
@@ -449,7 +448,7 @@ int zk_prove_files(zk_ctx* ctx, const char* zkey_path, const char* wtns_path, co
                    "witness has " + std::to_string(nw) + " entries, need " + std::to_string(c->n_vars));
         check_scalars(w.data(), c->n_vars);
         zk::ProveSlot& sl = ctx_slot(ctx);
-        sl.enqueue(ctx->impl, *c, w.data(), false, r, s, true);
+        sl.enqueue(ctx->impl, *c, w.data(), false, r, s);
         sl.finish(out);
     });
 }

@@ -782,27 +782,33 @@ void MsmScratch::count_ensure(const MsmGeom& g, size_t max_chunks, bool g2, int 
     scratch_buffers(*this, g, max_chunks, g2, split, [&](const DevBuf& b, size_t n) { gc.need(b, n); });
 }
 
-void msm_launch_pre(const MsmSort& sort, const void* d_points29, bool g2, MsmScratch& scr, hipStream_t st, int split) {
+static void check_jobs(const MsmSort& sort, const MsmJob* jobs, int count) {
+    ZK_REQUIRE(count >= 1 && count <= MSM_GROUP, ZK_E_INTERNAL, "MSM group size");
+    for (int j = 0; j < count; j++) {
+        ZK_REQUIRE(sort.n == 0 || jobs[j].pts29, ZK_E_INTERNAL, "MSM launch without the 29-bit copy of its points");
+        ZK_REQUIRE(jobs[j].range >= MSM_RANGE_ALL && jobs[j].range <= MSM_RANGE_B, ZK_E_INTERNAL, "unknown MSM entry range");
+    }
+}
+
+void msm_launch_pre(const MsmSort& sort, bool g2, const MsmJob* jobs, int count, hipStream_t st, int split) {
     ZK_REQUIRE(split >= 1 && split <= MSM_SPLIT_MAX, ZK_E_ARG, "bucket split out of range");
-    ZK_REQUIRE(sort.n == 0 || d_points29, ZK_E_INTERNAL, "MSM launch without the 29-bit copy of its points");
-    if (g2) msm_launch_pre_g2(sort, d_points29, scr, st, split);
-    else msm_launch_pre_g1(sort, d_points29, scr, st, split);
+    check_jobs(sort, jobs, count);
+    if (g2) msm_launch_pre_g2(sort, jobs, count, st, split);
+    else msm_launch_pre_g1(sort, jobs, count, st, split);
 }
 
-void msm_launch_main(const MsmSort& sort, bool g2, MsmScratch& scr, MsmPartials& out, hipStream_t st,
-                     const void* d_points29, int range) {
-    ZK_REQUIRE(sort.n == 0 || d_points29, ZK_E_INTERNAL, "MSM launch without the 29-bit copy of its points");
-    ZK_REQUIRE(scr.split >= 1, ZK_E_INTERNAL, "MSM accumulation queued before its chunked path");
-    ZK_REQUIRE(range >= MSM_RANGE_ALL && range <= MSM_RANGE_B, ZK_E_INTERNAL, "unknown MSM entry range");
-    if (!sort.classes) range = MSM_RANGE_ALL;
-    if (g2) msm_launch_main_g2(sort, scr, out, st, d_points29, range);
-    else msm_launch_main_g1(sort, scr, out, st, d_points29, range);
+void msm_launch_main(const MsmSort& sort, bool g2, const MsmJob* jobs, int count, hipStream_t st) {
+    check_jobs(sort, jobs, count);
+    for (int j = 0; j < count; j++)
+        ZK_REQUIRE(jobs[j].scr->split >= 1 && jobs[j].scr->split == jobs[0].scr->split, ZK_E_INTERNAL,
+                   "MSM accumulation queued before its chunked path");
+    if (g2) msm_launch_main_g2(sort, jobs, count, st);
+    else msm_launch_main_g1(sort, jobs, count, st);
 }
 
-void msm_launch(const MsmSort& sort, bool g2, MsmScratch& scr, MsmPartials& out, hipStream_t st,
-                const void* d_points29, int split) {
-    msm_launch_pre(sort, d_points29, g2, scr, st, split);
-    msm_launch_main(sort, g2, scr, out, st, d_points29);
+void msm_launch(const MsmSort& sort, bool g2, const MsmJob& job, hipStream_t st, int split) {
+    msm_launch_pre(sort, g2, &job, 1, st, split);
+    msm_launch_main(sort, g2, &job, 1, st);
 }
 
 // ---------------------------------------------------------------- fixed-scratch G1 MSM
@@ -879,7 +885,7 @@ zkh::Xyzz<zkh::Fp> msm_g1_noalloc(int device, const void* d_points, const void* 
     part.ext_bytes = sizeof g_noalloc_host;
     if (n) msm_points_to29(d_points, n, p29.p, false, st);
     sort.run(d_scalars, n, window, st);
-    msm_launch(sort, false, scr, part, st, p29.p, split);
+    msm_launch(sort, false, {p29.p, &scr, &part}, st, split);
     ZK_HIP(hipStreamSynchronize(st));
     return msm_finish_g1(part);
 }

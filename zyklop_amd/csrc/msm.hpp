@@ -178,9 +178,9 @@ struct MsmWorkspace {
     void release();     // frees the device buffers
 };
 
-// Launch bucket accumulation + GPU reduction against a finished sort; queue
-// the D2H of the partials into out.host on st. The caller synchronises st
-// before finish. d_points29: the base slots of msm_points_to29 (for a merged
+// Launch bucket accumulation + GPU reduction against a finished sort; its last
+// points arrive in out's host memory on st. The caller synchronises st before
+// finish. pts29: the base slots of msm_points_to29 (for a merged
 // sort, the W window tables of msm_points_table, table w at slot w*n); may be
 // null only for n = 0.
 // split: threads per bucket in the accumulation (1..MSM_SPLIT_MAX), each over
@@ -193,17 +193,23 @@ int msm_default_split(size_t n, int c, bool g2, bool merged = false);
 // of an MSM that has the GPU to itself (the MSM entry points over caller-owned
 // points)
 int msm_alone_split(size_t n, int c, bool g2);
-void msm_launch(const MsmSort& sort, bool g2, MsmScratch& scr, MsmPartials& out, hipStream_t st,
-                const void* d_points29, int split = 1);
+// One MSM over a sort. Several that share the sort and the curve go out in the
+// same launches (up to MSM_GROUP): a proof's A', B1' and C' MSMs are one
+// accumulation and one tree instead of three of each.
+constexpr int MSM_GROUP = 3;
+struct MsmJob {
+    const void* pts29;
+    MsmScratch* scr;
+    MsmPartials* out;
+    int range = MSM_RANGE_ALL;   // the part of every bucket it reads (a sort without classes: all of it)
+};
+void msm_launch(const MsmSort& sort, bool g2, const MsmJob& job, hipStream_t st, int split = 1);
 // msm_launch in two parts: the chunked path of the oversized buckets, then
-// the accumulation, reductions and the copy of the partials. Queueing every
+// the accumulation, reductions and the points for the host. Queueing every
 // MSM's first part before any accumulation keeps those short launches from
 // waiting behind the accumulations of other streams.
-void msm_launch_pre(const MsmSort& sort, const void* d_points29, bool g2, MsmScratch& scr, hipStream_t st, int split);
-// range: the part of every bucket this MSM reads (MsmRange; a sort without
-// classes reads all of it)
-void msm_launch_main(const MsmSort& sort, bool g2, MsmScratch& scr, MsmPartials& out, hipStream_t st,
-                     const void* d_points29, int range = MSM_RANGE_ALL);
+void msm_launch_pre(const MsmSort& sort, bool g2, const MsmJob* jobs, int count, hipStream_t st, int split);
+void msm_launch_main(const MsmSort& sort, bool g2, const MsmJob* jobs, int count, hipStream_t st);
 
 // n affine points (standard form, G1 64 B / G2 128 B each) -> n slots of the
 // 29-bit-limb form (G1 128 B, G2 256 B; layout in field29.hpp), each holding

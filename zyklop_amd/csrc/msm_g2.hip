@@ -12,17 +12,15 @@ namespace zk {
 // bucket accumulator live in LDS (field29.hpp AccLds) and are loaded where
 // used. One-wave blocks let the LDS share set the waves per CU.
 constexpr int ACC29Q_THREADS = 64;
-__global__ void __launch_bounds__(ACC29Q_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_msm_accum29q(const uint32_t* __restrict__ entries,
-                                                                 const uint32_t* __restrict__ offsets,
-                                                                 const uint32_t* __restrict__ order,
-                                                                 const uint32_t* __restrict__ cls_off, int range,
-                                                                 uint32_t nb, uint32_t split, uint32_t lmax,
-                                                                 const void* __restrict__ points29,
-                                                                 void* __restrict__ buckets) {
+__global__ void __launch_bounds__(ACC29Q_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_msm_accum29q(
+    const uint32_t* __restrict__ entries, const uint32_t* __restrict__ offsets, uint32_t nb, uint32_t split, uint32_t lmax,
+    MsmArgs args) {
+    const void* __restrict__ points29 = args.pts29[blockIdx.y];
+    void* __restrict__ buckets = args.buckets[blockIdx.y];
     __shared__ uint32_t lds[AccLds<ACC29Q_THREADS>::LDS_WORDS];
     uint32_t st, en, slot;
-    if (!acc_range<Fq2>(blockIdx.x * blockDim.x + threadIdx.x, nb, split, order, offsets, cls_off, range, lmax,
-                        buckets, st, en, slot))
+    if (!acc_range<Fq2>(blockIdx.x * blockDim.x + threadIdx.x, nb, split, args.order[blockIdx.y], offsets,
+                        args.cls_off[blockIdx.y], args.range[blockIdx.y], lmax, buckets, st, en, slot))
         return;
     AccLds<ACC29Q_THREADS> A{lds + threadIdx.x, {}};
     bool inf = true;
@@ -88,22 +86,17 @@ __global__ void k_points_table_q(const void* __restrict__ pts, uint32_t n, int W
 }
 
 template <>
-void launch_accum<Fq2>(const MsmSort& sort, uint32_t nb, int split, const void* d_points29, void* buckets, hipStream_t st,
-                       int range) {
-    const uint32_t nt = nb * (uint32_t)split;
-    k_msm_accum29q<<<cdiv(nt, ACC29Q_THREADS), ACC29Q_THREADS, 0, st>>>(
-        sort.entries.as<uint32_t>(), sort.offsets.as<uint32_t>(), msm_range_order(sort, range),
-        range != MSM_RANGE_ALL ? sort.cls_off.as<uint32_t>() : nullptr, range, nb, (uint32_t)split, sort.lmax,
-        d_points29, buckets);
+void launch_accum<Fq2>(const MsmSort& sort, uint32_t nb, int split, const MsmArgs& args, int count, hipStream_t st) {
+    k_msm_accum29q<<<dim3(cdiv((size_t)nb * split, ACC29Q_THREADS), count), ACC29Q_THREADS, 0, st>>>(
+        sort.entries.as<uint32_t>(), sort.offsets.as<uint32_t>(), nb, (uint32_t)split, sort.lmax, args);
 }
 
-void msm_launch_pre_g2(const MsmSort& sort, const void* d_points29, MsmScratch& scr, hipStream_t st, int split) {
-    launch_pre_t<Fq2>(sort, d_points29, scr, st, split);
+void msm_launch_pre_g2(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st, int split) {
+    launch_pre_t<Fq2>(sort, jobs, count, st, split);
 }
 
-void msm_launch_main_g2(const MsmSort& sort, MsmScratch& scr, MsmPartials& out, hipStream_t st, const void* d_points29,
-                        int range) {
-    launch_main_t<Fq2>(sort, d_points29, scr, out, st, range);
+void msm_launch_main_g2(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st) {
+    launch_main_t<Fq2>(sort, jobs, count, st);
 }
 
 void msm_points_to29_g2(const void* d_points, size_t n, void* d_out, hipStream_t st) {

@@ -25,6 +25,19 @@ template <class T> inline constexpr int TREE_LOG = 7;   // G1: 64 groups of 4 la
 template <> inline constexpr int TREE_LOG<Fq2> = 6;     // 32 groups of 8 lanes
 template <class T> inline constexpr int TREE_NODES = 1 << TREE_LOG<T>;
 
+// what the MSMs of one launch do not share (MsmJob), by blockIdx.y (the tree:
+// blockIdx.z)
+struct MsmArgs {
+    const void* pts29[MSM_GROUP];
+    const uint32_t* order[MSM_GROUP];
+    const uint32_t* cls_off[MSM_GROUP];   // null: whole buckets
+    int range[MSM_GROUP];
+    void* buckets[MSM_GROUP];
+    void* partials[MSM_GROUP];
+    const void* in[MSM_GROUP];            // of a reduction launch
+    void* out[MSM_GROUP];
+};
+
 struct ChunkRec { uint32_t bucket, start, len, pad; };
 struct LargeRec { uint32_t bucket, first, count, pad; };
 
@@ -221,11 +234,11 @@ ZK_DEV void store_sum(const uint32_t* sh, void* out, size_t i) {
 constexpr int CHUNK_THREADS = 64, MERGE_THREADS = 256;
 template <class T>
 __global__ void __launch_bounds__(CHUNK_THREADS) k_msm_chunks(const uint32_t* __restrict__ entries,
-                                                             const void* __restrict__ points29,
                                                              const uint32_t* __restrict__ counters,
-                                                             const ChunkRec* __restrict__ chunks,
-                                                             void* __restrict__ partials) {
+                                                             const ChunkRec* __restrict__ chunks, MsmArgs args) {
     constexpr int L = Coop<T>::LANES;
+    const void* __restrict__ points29 = args.pts29[blockIdx.y];
+    void* __restrict__ partials = args.partials[blockIdx.y];
     __shared__ uint32_t sh[CHUNK_THREADS * L * 9 > LaneSum<T>::LDS_WORDS ? CHUNK_THREADS * L * 9 : LaneSum<T>::LDS_WORDS];
     const Coop<T> k(threadIdx.x % L);
     const uint32_t nch = counters[0];
@@ -252,10 +265,11 @@ __global__ void __launch_bounds__(CHUNK_THREADS) k_msm_chunks(const uint32_t* __
 // one workgroup per oversized bucket: sum its chunk partials
 template <class T>
 __global__ void __launch_bounds__(MERGE_THREADS) k_msm_merge(const uint32_t* __restrict__ counters,
-                                                            const LargeRec* __restrict__ large,
-                                                            const void* __restrict__ partials, uint32_t split,
-                                                            void* __restrict__ buckets) {
+                                                            const LargeRec* __restrict__ large, uint32_t split,
+                                                            MsmArgs args) {
     constexpr int L = Coop<T>::LANES, G = MERGE_THREADS / L;
+    const void* __restrict__ partials = args.partials[blockIdx.y];
+    void* __restrict__ buckets = args.buckets[blockIdx.y];
     __shared__ uint32_t sh[G * L * 9];
     const uint32_t lane = threadIdx.x % L, grp = threadIdx.x / L;
     const Coop<T> k(lane);
@@ -286,9 +300,11 @@ __global__ void __launch_bounds__(MERGE_THREADS) k_msm_merge(const uint32_t* __r
 // the bucket's `split` slots from the accumulation. out: [W][R, T][K/L1], the
 // two channels of the tree's nodes.
 template <class T>
-__global__ void __launch_bounds__(128) k_msm_reduce1(const void* __restrict__ buckets, uint32_t K, int W, uint32_t L1,
-                                                     uint32_t split, void* __restrict__ out) {
+__global__ void __launch_bounds__(128) k_msm_reduce1(MsmArgs args, uint32_t K, int W, uint32_t L1,
+                                                     uint32_t split) {
     using P = Red<T>;
+    const void* __restrict__ buckets = args.in[blockIdx.y];
+    void* __restrict__ out = args.out[blockIdx.y];
     uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t nseg = K / L1;
     if (j >= (uint32_t)W * nseg) return;
@@ -329,10 +345,11 @@ __global__ void __launch_bounds__(128) k_msm_reduce1(const void* __restrict__ bu
 // suffix scan and a tree sum over one workgroup per 1024 segments that this
 // replaced took 0.43, 0.52, 0.56, 1.31 and 1.42 ms.
 template <class T>
-__global__ void __launch_bounds__(TREE_THREADS) k_msm_tree(const void* __restrict__ in, uint32_t N, uint32_t C,
-                                                           uint32_t parts, int plain, int q, int last, uint32_t Cout,
-                                                           void* __restrict__ out) {
+__global__ void __launch_bounds__(TREE_THREADS) k_msm_tree(MsmArgs args, uint32_t N, uint32_t C, uint32_t parts,
+                                                           int plain, int q, int last, uint32_t Cout) {
     constexpr int L = Coop<T>::LANES, G = TREE_THREADS / L;
+    const void* __restrict__ in = args.in[blockIdx.z];
+    void* __restrict__ out = args.out[blockIdx.z];
     __shared__ uint32_t sh[TREE_NODES<T> * L * 9];
     const uint32_t lane = threadIdx.x % L, grp = threadIdx.x / L;
     const Coop<T> k(lane);
@@ -401,17 +418,23 @@ __global__ void __launch_bounds__(TREE_THREADS) k_msm_tree(const void* __restric
 // wait behind other streams' accumulations while its own stream's
 // accumulation waits behind it.
 template <class T>
-static void launch_pre_t(const MsmSort& sort, const void* d_points29, MsmScratch& scr, hipStream_t st, int split) {
+static void launch_pre_t(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st, int split) {
     const bool g2 = std::is_same<T, Fq2>::value;
     const MsmGeom g = msm_geom(sort.n, sort.g.c, g2, sort.g.merged);
-    scr.ensure(g, sort.n_chunk_max, g2, split);
-    scr.split = split;
-    k_msm_chunks<T><<<CHUNK_PARTS, CHUNK_THREADS, 0, st>>>(sort.entries.as<uint32_t>(), d_points29,
-                                                   sort.counters.as<uint32_t>(), sort.chunks.as<ChunkRec>(),
-                                                   scr.partials.p);
+    MsmArgs args{};
+    for (int j = 0; j < count; j++) {
+        MsmScratch& scr = *jobs[j].scr;
+        scr.ensure(g, sort.n_chunk_max, g2, split);
+        scr.split = split;
+        args.pts29[j] = jobs[j].pts29;
+        args.buckets[j] = scr.buckets.p;
+        args.partials[j] = scr.partials.p;
+    }
+    k_msm_chunks<T><<<dim3(CHUNK_PARTS, count), CHUNK_THREADS, 0, st>>>(
+        sort.entries.as<uint32_t>(), sort.counters.as<uint32_t>(), sort.chunks.as<ChunkRec>(), args);
     ZK_HIP(hipGetLastError());
-    k_msm_merge<T><<<16, MERGE_THREADS, 0, st>>>(sort.counters.as<uint32_t>(), sort.large.as<LargeRec>(), scr.partials.p,
-                                         (uint32_t)split, scr.buckets.p);
+    k_msm_merge<T><<<dim3(16, count), MERGE_THREADS, 0, st>>>(sort.counters.as<uint32_t>(), sort.large.as<LargeRec>(),
+                                                              (uint32_t)split, args);
     ZK_HIP(hipGetLastError());
 }
 
@@ -423,70 +446,80 @@ inline const uint32_t* msm_range_order(const MsmSort& sort, int range) {
 
 // the bucket-accumulation kernel of curve T (msm_g1.hip / msm_g2.hip)
 template <class T>
-void launch_accum(const MsmSort& sort, uint32_t nb, int split, const void* d_points29, void* buckets, hipStream_t st,
-                  int range);
+void launch_accum(const MsmSort& sort, uint32_t nb, int split, const MsmArgs& args, int count, hipStream_t st);
 
 template <class T>
-static void launch_main_t(const MsmSort& sort, const void* d_points29, MsmScratch& scr, MsmPartials& out,
-                          hipStream_t st, int range) {
+static void launch_main_t(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st) {
     const bool g2 = std::is_same<T, Fq2>::value;
     const MsmGeom g = msm_geom(sort.n, sort.g.c, g2, sort.g.merged);
-    const int split = scr.split;
+    const int split = jobs[0].scr->split;
     const uint32_t nb = (uint32_t)((size_t)g.Wr * g.K);
-    if (scr.ev_acc0) ZK_HIP(hipEventRecord(scr.ev_acc0, st));
-    launch_accum<T>(sort, nb, split, d_points29, scr.buckets.p, st, range);
+    MsmArgs args{};
+    for (int j = 0; j < count; j++) {
+        const int range = sort.classes ? jobs[j].range : (int)MSM_RANGE_ALL;
+        args.pts29[j] = jobs[j].pts29;
+        args.order[j] = msm_range_order(sort, range);
+        args.cls_off[j] = range != MSM_RANGE_ALL ? sort.cls_off.as<uint32_t>() : nullptr;
+        args.range[j] = range;
+        args.buckets[j] = jobs[j].scr->buckets.p;
+        if (jobs[j].scr->ev_acc0) ZK_HIP(hipEventRecord(jobs[j].scr->ev_acc0, st));
+    }
+    launch_accum<T>(sort, nb, split, args, count, st);
     ZK_HIP(hipGetLastError());
-    if (scr.ev_acc1) ZK_HIP(hipEventRecord(scr.ev_acc1, st));
+    for (int j = 0; j < count; j++)
+        if (jobs[j].scr->ev_acc1) ZK_HIP(hipEventRecord(jobs[j].scr->ev_acc1, st));
     const MsmTree t = msm_tree(g, g2, split);
-    const void* in = scr.buckets.p;
+    const size_t bytes = (size_t)g.Wr * t.nout * (g2 ? 256 : 128);
+    for (int j = 0; j < count; j++) {
+        MsmPartials& out = *jobs[j].out;
+        out.g = g;
+        out.g2 = g2;
+        out.bit0 = ilog2(t.l1);
+        out.nout = t.nout;
+        if (out.ext) ZK_REQUIRE(out.ext_bytes >= bytes, ZK_E_INTERNAL, "MSM partials exceed the caller's host buffer");
+        else out.host.ensure(bytes);
+        args.in[j] = jobs[j].scr->buckets.p;
+    }
     if (t.l1 > 1) {
-        k_msm_reduce1<T><<<cdiv((size_t)g.Wr * (g.K / t.l1), 128), 128, 0, st>>>(scr.buckets.p, g.K, g.Wr, t.l1,
-                                                                                 (uint32_t)split, scr.seg.p);
+        for (int j = 0; j < count; j++) args.out[j] = jobs[j].scr->seg.p;
+        k_msm_reduce1<T><<<dim3(cdiv((size_t)g.Wr * (g.K / t.l1), 128), count), 128, 0, st>>>(args, g.K, g.Wr, t.l1,
+                                                                                            (uint32_t)split);
         ZK_HIP(hipGetLastError());
-        in = scr.seg.p;
+        for (int j = 0; j < count; j++) args.in[j] = args.out[j];
     }
     uint32_t N = t.nodes, C = t.l1 > 1 ? 2 : 1, parts = t.parts;
     int plain = t.plain;
-    DevBuf* dst[2] = {&scr.node0, &scr.node1};
     for (int lev = 0; lev < t.levels; lev++) {
-        const int q = t.q[lev];
+        const int q = t.q[lev], last = lev == t.levels - 1;
         const uint32_t Cout = C + (uint32_t)std::max(0, q - plain);
-        k_msm_tree<T><<<dim3(N >> q, (unsigned)g.Wr * C), TREE_THREADS, 0, st>>>(in, N, C, parts, plain, q,
-                                                                               lev == t.levels - 1, Cout,
-                                                                               dst[lev & 1]->p);
+        // the last launch writes pinned host memory itself: a copy would be a
+        // launch of its own at the end of every MSM
+        for (int j = 0; j < count; j++)
+            args.out[j] = last && !jobs[j].out->ext ? jobs[j].out->host.p
+                                                    : (lev & 1 ? jobs[j].scr->node1 : jobs[j].scr->node0).p;
+        k_msm_tree<T><<<dim3(N >> q, (unsigned)g.Wr * C, count), TREE_THREADS, 0, st>>>(args, N, C, parts, plain, q, last,
+                                                                                        Cout);
         ZK_HIP(hipGetLastError());
-        in = dst[lev & 1]->p;
+        for (int j = 0; j < count; j++) args.in[j] = args.out[j];
         N >>= q;
         C = Cout;
         parts = 1;
         plain = std::max(0, plain - q);
     }
-    const size_t bytes = (size_t)g.Wr * t.nout * (g2 ? 256 : 128);
-    out.g = g;
-    out.g2 = g2;
-    out.bit0 = ilog2(t.l1);
-    out.nout = t.nout;
-    void* to = out.ext;
-    if (to) {
-        ZK_REQUIRE(out.ext_bytes >= bytes, ZK_E_INTERNAL, "MSM partials exceed the caller's host buffer");
-    } else {
-        out.host.ensure(bytes);
-        to = out.host.p;
+    for (int j = 0; j < count; j++) {
+        if (jobs[j].out->ext) ZK_HIP(hipMemcpyAsync(jobs[j].out->ext, args.in[j], bytes, hipMemcpyDeviceToHost, st));
+        if (jobs[j].scr->ev_end) ZK_HIP(hipEventRecord(jobs[j].scr->ev_end, st));
     }
-    ZK_HIP(hipMemcpyAsync(to, in, bytes, hipMemcpyDeviceToHost, st));
-    if (scr.ev_end) ZK_HIP(hipEventRecord(scr.ev_end, st));
 }
 
 
 // per-curve entry points, defined in msm_g1.hip and msm_g2.hip
-void msm_launch_pre_g1(const MsmSort& sort, const void* d_points29, MsmScratch& scr, hipStream_t st, int split);
-void msm_launch_main_g1(const MsmSort& sort, MsmScratch& scr, MsmPartials& out, hipStream_t st, const void* d_points29,
-                        int range);
+void msm_launch_pre_g1(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st, int split);
+void msm_launch_main_g1(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st);
 void msm_points_to29_g1(const void* d_points, size_t n, void* d_out, hipStream_t st);
 void msm_points_table_g1(const void* d_points, size_t n, const MsmGeom& g, void* d_out, hipStream_t st);
-void msm_launch_pre_g2(const MsmSort& sort, const void* d_points29, MsmScratch& scr, hipStream_t st, int split);
-void msm_launch_main_g2(const MsmSort& sort, MsmScratch& scr, MsmPartials& out, hipStream_t st, const void* d_points29,
-                        int range);
+void msm_launch_pre_g2(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st, int split);
+void msm_launch_main_g2(const MsmSort& sort, const MsmJob* jobs, int count, hipStream_t st);
 void msm_points_to29_g2(const void* d_points, size_t n, void* d_out, hipStream_t st);
 void msm_points_table_g2(const void* d_points, size_t n, const MsmGeom& g, void* d_out, hipStream_t st);
 

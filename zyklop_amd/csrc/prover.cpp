@@ -26,7 +26,7 @@ Context::Context(int dev) : device(dev) {
     ZK_REQUIRE(dev >= 0 && dev < count, ZK_E_ARG, "no such HIP device: " + std::to_string(dev));
     ZK_HIP(hipSetDevice(dev));
     ZK_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    ZK_HIP(hipStreamCreateWithFlags(&aux_stream, hipStreamNonBlocking));
+    for (hipStream_t* p : {&prove1, &prove2, &aux_stream}) ZK_HIP(hipStreamCreateWithFlags(p, hipStreamNonBlocking));
     msm_noalloc_setup(dev);   // device address of the fixed MSM scratch, once per device
     // default window-table mode for circuits loaded on this context
     if (const char* e = getenv("ZK_WINDOW_TABLES")) {
@@ -41,7 +41,8 @@ Context::~Context() {
     slot.reset();
     ntt_plans.clear();
     if (stream) (void)hipStreamDestroy(stream);
-    if (aux_stream) (void)hipStreamDestroy(aux_stream);
+    for (hipStream_t p : {prove1, prove2, aux_stream})
+        if (p) (void)hipStreamDestroy(p);
 }
 
 NttPlan& Context::ntt_plan(int log_n) {
@@ -347,7 +348,13 @@ void circuit_write_zkey(const Circuit& c, const std::string& path) {
 
 // ------------------------------------------------------------------ proving
 ProveSlot::ProveSlot() {
-    for (hipStream_t* p : {&s0, &s1, &s2, &s3, &s4}) ZK_HIP(hipStreamCreateWithFlags(p, hipStreamNonBlocking));
+    for (hipStream_t* p : {&s0, &s1, &s2}) ZK_HIP(hipStreamCreateWithFlags(p, hipStreamNonBlocking));
+    create_events();
+}
+
+ProveSlot::ProveSlot(Context& ctx) : s0(ctx.stream), s1(ctx.prove1), s2(ctx.prove2), own_streams(false) { create_events(); }
+
+void ProveSlot::create_events() {
     ZK_HIP(hipEventCreateWithFlags(&ev_scal, hipEventDisableTiming));
     ZK_HIP(hipEventCreateWithFlags(&ev_done1, hipEventDisableTiming));
     for (auto& e : ev_join) ZK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -364,8 +371,11 @@ void ProveSlot::enable_timing() {
 ProveSlot::~ProveSlot() {
     for (auto& e : ev)
         if (e) (void)hipEventDestroy(e);
-    for (hipStream_t p : {s0, s1, s2, s3, s4})
-        if (p) { (void)hipStreamSynchronize(p); (void)hipStreamDestroy(p); }
+    for (hipStream_t p : {s0, s1, s2})
+        if (p) {
+            (void)hipStreamSynchronize(p);
+            if (own_streams) (void)hipStreamDestroy(p);
+        }
     if (ev_scal) (void)hipEventDestroy(ev_scal);
     if (ev_done1) (void)hipEventDestroy(ev_done1);
     if (ev_h) (void)hipEventDestroy(ev_h);
@@ -416,7 +426,7 @@ void ProveSlot::reserve(Context& ctx, const Circuit& c, bool host_witness) {
 }
 
 void ProveSlot::enqueue(Context& ctx, const Circuit& c, const uint64_t* witness, bool on_dev, const uint64_t r_[4],
-                        const uint64_t s_[4], bool alone) {
+                        const uint64_t s_[4]) {
     circ = &c;
     for (int i = 0; i < 4; i++) { r[i] = r_ ? r_[i] : 0; s[i] = s_ ? s_[i] : 0; }
     ZK_REQUIRE(Fr::is_canonical(r) && Fr::is_canonical(s), ZK_E_ARG, "blinding scalars must be canonical (< r)");
@@ -436,10 +446,10 @@ void ProveSlot::enqueue(Context& ctx, const Circuit& c, const uint64_t* witness,
     uint64_t ex[16];
     blinding_tail(r, s, ex);
     write_scalars4((char*)scal.p + nv * 32, ex, s0);
-    body(ctx, c, parts, alone);
+    body(ctx, c, parts);
 }
 
-void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out, bool alone) {
+void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out) {
     const size_t nS = (size_t)c.n_vars + 4, n = c.n;
     NttPlan& plan = ctx.ntt_plan(c.log_n);
     const MsmPlan pl = ctx.msm_plan(c);
@@ -447,19 +457,15 @@ void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out, bool alone
     window_h = pl.ch;
     const int sp_w1 = pl.sp_w1, sp_w2 = pl.sp_w2, sp_h = pl.sp_h;
     ZK_HIP(hipEventRecord(ev_scal, s0));
-    // witness MSMs first: the G2 one is the longest chain of the proof, so its
-    // sort and accumulation are queued before the H pipeline. One shared
-    // sort, then the four MSMs read the same sorted entries on their own
-    // streams (B2 s4, B1 s2, C s3). Two layouts for the sort and A:
-    //  - batches (several proofs in flight): sort and A on s1, so each MSM
-    //    has a stream and one MSM's latency-bound reduction overlaps
-    //    another's accumulation;
-    //  - a proof alone on the device: sort on s2, A after B1 on s2, and s1
-    //    left empty. With more streams than hardware queues s1 shares its
-    //    queue with s0 (creation order), and work on it holds the H
-    //    pipeline, the proof's longest chain, behind it (plain proofs
-    //    13.8 -> 13.4 ms; in batches the other slots fill that gap and the
-    //    extra MSM stream does better).
+    // One shared sort on s1; then A, B1 and C in the same launches on s1 and B2
+    // on s2 read its entries, while s0 runs the H pipeline. Order of the launches:
+    // the H pipeline's come between the sort and the MSMs, since H is the longest
+    // chain and a small proof waits for launches; then G2, the H MSM, and the
+    // three G1 MSMs last, whose one large accumulation fills the GPU to the end
+    // (2^14 constraints 665 us, 690 with the MSMs before the H pipeline; 500000
+    // constraints 4.40 ms against 4.66; G1 before H the same within the noise).
+    // One launch for the three G1 MSMs against three streams: 8 proofs of 50021
+    // constraints 6.14 -> 5.59 ms.
     //
     // With wire classes (Circuit::wire_cls) the A MSM and the B1, B2 MSMs
     // read only the entries of their finite bases. An infinite base in the
@@ -467,25 +473,18 @@ void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out, bool alone
     // lanes of the wave are adding; a quarter of the A' and of the B' bases
     // of the synthetic circuits are infinite (row i draws its wires uniformly
     // from the first ones, so late wires are rarely used).
-    alone_layout = alone;
-    hipStream_t s_sort = alone ? s2 : s1, s_a = alone ? s2 : s1;
     const uint8_t* cls = c.wire_cls.bytes ? c.wire_cls.as<uint8_t>() : nullptr;
-    ZK_HIP(hipStreamWaitEvent(s_sort, ev_scal, 0));
-    if (timed) ZK_HIP(hipEventRecord(ev[4], s_sort));
-    sortW.run(scal.p, nS, window_w, s_sort, pl.mw, cls);
-    ZK_HIP(hipEventRecord(ev_done1, s_sort));
-    if (timed) ZK_HIP(hipEventRecord(ev[5], s_sort));
-    for (hipStream_t p : {s1, s2, s3, s4})
-        if (p != s_sort) ZK_HIP(hipStreamWaitEvent(p, ev_done1, 0));
-    msm_launch_pre(sortW, c.B2_29.p, true, scrB2, s4, sp_w2);
-    msm_launch_pre(sortW, c.B1_29.p, false, scrB1, s2, sp_w1);
-    msm_launch_pre(sortW, c.C29.p, false, scrC, s3, sp_w1);
-    msm_launch_pre(sortW, c.A29.p, false, scrA, s_a, sp_w1);
-    msm_launch_main(sortW, true, scrB2, out.b2, s4, c.B2_29.p, MSM_RANGE_B);
-    if (!alone) msm_launch_main(sortW, false, scrA, out.a, s_a, c.A29.p, MSM_RANGE_A);
-    msm_launch_main(sortW, false, scrB1, out.b1, s2, c.B1_29.p, MSM_RANGE_B);
-    msm_launch_main(sortW, false, scrC, out.c, s3, c.C29.p);
-    if (alone) msm_launch_main(sortW, false, scrA, out.a, s_a, c.A29.p, MSM_RANGE_A);
+    ZK_HIP(hipStreamWaitEvent(s1, ev_scal, 0));
+    if (timed) ZK_HIP(hipEventRecord(ev[4], s1));
+    sortW.run(scal.p, nS, window_w, s1, pl.mw, cls);
+    ZK_HIP(hipEventRecord(ev_done1, s1));
+    if (timed) ZK_HIP(hipEventRecord(ev[5], s1));
+    ZK_HIP(hipStreamWaitEvent(s2, ev_done1, 0));
+    const MsmJob b2 = {c.B2_29.p, &scrB2, &out.b2, MSM_RANGE_B};
+    const MsmJob abc1[3] = {{c.A29.p, &scrA, &out.a, MSM_RANGE_A}, {c.B1_29.p, &scrB1, &out.b1, MSM_RANGE_B},
+                            {c.C29.p, &scrC, &out.c}};
+    msm_launch_pre(sortW, true, &b2, 1, s2, sp_w2);
+    msm_launch_pre(sortW, false, abc1, 3, s1, sp_w1);
     // H pipeline on s0
     spmv_abc(c.rowA.as<uint32_t>(), c.colA.as<uint32_t>(), c.valA.p, c.n_rowsA, c.rowB.as<uint32_t>(),
              c.colB.as<uint32_t>(), c.valB.p, c.n_rowsB, scal.p, n, aw.p, bw.p, cw.p, s0);
@@ -498,22 +497,24 @@ void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out, bool alone
     if (timed) ZK_HIP(hipEventRecord(ev[3], s0));
     h_final(aw.p, bw.p, cw.p, h.p, n, s0);
     sortH.run(h.p, n, window_h, s0, pl.mh);
-    msm_launch(sortH, false, scrH, out.h, s0, c.H29.p, sp_h);
+    msm_launch_main(sortW, true, &b2, 1, s2);
+    msm_launch(sortH, false, {c.H29.p, &scrH, &out.h}, s0, sp_h);
+    msm_launch_main(sortW, false, abc1, 3, s1);
     ZK_HIP(hipEventRecord(ev_h, s0));
-    hipStream_t br[4] = {s1, s2, s3, s4};
-    for (int k = 0; k < 4; k++) {
+    hipStream_t br[2] = {s1, s2};
+    for (int k = 0; k < 2; k++) {
         ZK_HIP(hipEventRecord(ev_join[k], br[k]));
         ZK_HIP(hipStreamWaitEvent(s0, ev_join[k], 0));
     }
 }
 
 void ProveSlot::drain() noexcept {
-    for (hipStream_t p : {s0, s1, s2, s3, s4})
+    for (hipStream_t p : {s0, s1, s2})
         if (p) (void)hipStreamSynchronize(p);
 }
 
 bool ProveSlot::device_done() const {
-    for (hipStream_t p : {s0, s1, s2, s3, s4}) {
+    for (hipStream_t p : {s0, s1, s2}) {
         hipError_t e = hipStreamQuery(p);
         if (e == hipErrorNotReady) return false;
         if (e != hipSuccess) ZK_HIP(e);
@@ -603,11 +604,10 @@ double assemble_proof(const ProofParts& p, const uint64_t r[4], const uint64_t s
 }
 
 void ProveSlot::finish(zk_proof* out) {
-    // A on s1 (ev_join[0]), or after B1 on s2 (ev_join[1]) in the layout of a
-    // proof alone; B1 s2, C s3, B2 s4, H s0
-    const hipEvent_t ready[5] = {alone_layout ? ev_join[1] : ev_join[0], ev_join[1], ev_join[2], ev_join[3], ev_h};
+    // A, B1 and C on s1, B2 on s2, H on s0
+    const hipEvent_t ready[5] = {ev_join[0], ev_join[0], ev_join[0], ev_join[1], ev_h};
     const double tail_ms = assemble_proof(parts, r, s, out, ready);
-    ZK_HIP(hipStreamSynchronize(s0));   // s1..s4 are joined into s0
+    ZK_HIP(hipStreamSynchronize(s0));   // s1, s2 are joined into s0
     if (timed) {
         collect_stats();
         stats[23] = tail_ms;
@@ -705,7 +705,7 @@ void BatchGraph::fill_params(const uint64_t* r, const uint64_t* s) {
 }
 
 // queue the whole batch: proof i on slot i % S; a slot's proofs are ordered by
-// its s0 (each proof's end joins s1..s4 into s0)
+// its s0 (each proof's end joins s1, s2 into s0)
 void BatchGraph::record(bool capture) {
     const size_t S = slots.size();
     ZK_HIP(hipEventRecord(ev_fork, origin));

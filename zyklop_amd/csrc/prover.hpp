@@ -86,11 +86,11 @@ double assemble_proof(const ProofParts& p, const uint64_t r[4], const uint64_t s
                       const hipEvent_t* ready = nullptr);
 
 struct ProveSlot {
-    // s0: H pipeline + H MSM; s1: witness sort + A; s2: B1; s3: C; s4: B2.
-    // Each proof forks s1..s4 from s0 and joins them back into s0 at its end.
-    hipStream_t s0 = nullptr, s1 = nullptr, s2 = nullptr, s3 = nullptr, s4 = nullptr;
-    hipEvent_t ev_scal = nullptr, ev_done1 = nullptr, ev_join[4] = {}, ev_h = nullptr;
-    bool alone_layout = false;   // the layout body() used for the queued proof
+    // s0: H pipeline + H MSM; s1: witness sort, then A, B1 and C together; s2:
+    // B2. Each proof forks s1, s2 from s0 and joins them back into s0 at its end.
+    hipStream_t s0 = nullptr, s1 = nullptr, s2 = nullptr;
+    bool own_streams = true;
+    hipEvent_t ev_scal = nullptr, ev_done1 = nullptr, ev_join[2] = {}, ev_h = nullptr;
     DevBuf scal, aw, bw, cw, t0, t1, t2, h, wtmp;
     HostBuf staging;                 // pinned copy of a host witness (async upload)
     MsmSort sortW, sortH;
@@ -105,15 +105,15 @@ struct ProveSlot {
     double stats[24] = {};
     void enable_timing();
     void collect_stats();
-    ProveSlot();
+    ProveSlot();                       // on streams of its own
+    explicit ProveSlot(Context& ctx);  // on the context's streams
     ~ProveSlot();
     ProveSlot(const ProveSlot&) = delete;
     ProveSlot& operator=(const ProveSlot&) = delete;
     // queue all device work for one proof; witness is host (canonical) or
-    // device; alone: no other proof shares the device (the stream layout for
-    // latency, see body)
+    // device
     void enqueue(Context& ctx, const Circuit& c, const uint64_t* witness, bool witness_on_device, const uint64_t r[4],
-                 const uint64_t s[4], bool alone = false);
+                 const uint64_t s[4]);
     // size every device buffer a proof of c needs in this slot
     void prepare(Context& ctx, const Circuit& c);
     // size every buffer a proof of c needs in this slot, sorts, MSM scratch
@@ -123,8 +123,8 @@ struct ProveSlot {
     void reserve(Context& ctx, const Circuit& c, bool host_witness);
     // the device work of one proof once scal holds [w | 1, r, s, -rs] (queued
     // on s0 before the call): everything up to the partials in out, ending
-    // with s1..s4 joined into s0. Stream-capturable after prepare().
-    void body(Context& ctx, const Circuit& c, ProofParts& out, bool alone = false);
+    // with s1, s2 joined into s0. Stream-capturable after prepare().
+    void body(Context& ctx, const Circuit& c, ProofParts& out);
     // wait for the device work and run the host tail
     void finish(zk_proof* out);
     // true when every stream of the slot has drained (non-blocking)
@@ -142,6 +142,7 @@ struct ProveSlot {
     size_t device_bytes() const;
 
   private:
+    void create_events();
     static size_t count_bytes(const Context& ctx, const Circuit& c, const ProveSlot* sl);
 };
 
@@ -157,7 +158,14 @@ struct MsmPlan {
 
 struct Context {
     int device = 0;
-    hipStream_t stream = nullptr;
+    // The runtime spreads a process's streams over GPU_MAX_HW_QUEUES hardware
+    // queues (4 by default) as they are created, and streams that share a queue
+    // run one after the other. So the three that a proof alone on the device
+    // needs side by side (stream, prove1, prove2) come first, in one go, and the
+    // one-shot slot uses the context's own stream: created later, its H pipeline
+    // shared a queue with the G1 MSMs and waited for them (2^14 constraints 820 us
+    // instead of 665, 200003 2.5 ms instead of 2.17).
+    hipStream_t stream = nullptr, prove1 = nullptr, prove2 = nullptr;
     std::mutex mu;
     // side work that needs no other context state (synthetic witness
     // generation): its own stream and lock, so it does not wait for provers

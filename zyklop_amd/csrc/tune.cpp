@@ -140,8 +140,7 @@ void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged
                 if ((size_t)g.Wr * g.K * s > ((size_t)1 << 21) && s > 1) continue;
                 ZK_HIP(hipEventRecord(tb.e0, st));
                 MsmScratch& scr = ms[m].g2 ? tb.g2 : tb.g1;
-                msm_launch_pre(tb.sort, ms[m].p29, ms[m].g2, scr, st, s);
-                msm_launch_main(tb.sort, ms[m].g2, scr, tb.part, st, ms[m].p29, ms[m].range);
+                msm_launch(tb.sort, ms[m].g2, {ms[m].p29, &scr, &tb.part, ms[m].range}, st, s);
                 ZK_HIP(hipEventRecord(tb.e1, st));
                 const float t = elapsed(tb);
                 if (it > 0) msm[m][s - 1] = (msm[m][s - 1] < 0 ? 0 : msm[m][s - 1]) + t / reps;
