@@ -57,13 +57,6 @@ ZK_DEV uint32_t f29_or(const F29& a) {
     return d;
 }
 
-namespace f29c {
-// 6p with every limb but the top one in [3 * 2^29 - 3, 2^31) (3 borrowed from
-// the next limb): 6p - a - 2b never borrows for normalized a + 2b < 6p
-constexpr uint32_t P6[9] = {0x72edefaau, 0x661a4445u, 0x6aafd3d7u, 0x70fed0e2u, 0x612318cdu,
-                            0x71238481u, 0x63e94783u, 0x7628e535u, 0x012259d3u};
-}  // namespace f29c
-
 // What differs between the curves. mul: the lane's component of x*y, x and y
 // normalized, y < 8p; the result is below p + (x*y + 8x*p)/169p (G1: without
 // the 8x*p). all: whether a lane flag holds in every component.
@@ -97,12 +90,6 @@ struct Coop<Fq2> {
     ZK_DEV uint32_t any(uint32_t f) const { return f | u32_xor4(f); }
     ZK_DEV uint32_t all(uint32_t f) const { return f & u32_xor4(f); }
 };
-
-// value 0 or p (a product's zero: products are below 2p)
-ZK_DEV uint32_t f29_zero_mod(const F29& a) {
-    if (a.l[0] != 0 && a.l[0] != f29c::P[0]) return 0u;
-    return f29_or(a) == 0 || f29_eq(a, f29c::P) ? 1u : 0u;
-}
 
 // Bounds kept by both operations, in units of p (mul's bound, worst cases of
 // G2): X < 7.4, Y < 2.8, ZZ and ZZZ < 2, limbs normalized; points of the
@@ -157,7 +144,7 @@ ZK_DEV F29 coop_add(const Coop<T>& k, const F29& a, const F29& b) {
     for (int i = 0; i < 9; i++) d.l[i] = r1x.l[i] + P2[i] - r1.l[i];
     const F29 D = f29_norm(d);                                 // P, R, -P, -R
     const F29 r2 = k.mul(f29_sel(k.m2, a, D), f29_sel(k.m2, b, D));   // PP, RR, ZZ1*ZZ2, ZZZ1*ZZZ2
-    const uint32_t zero = k.all(f29_zero_mod(r2));
+    const uint32_t zero = k.all(f29_zero_mod(r2) ? 1u : 0u);
     const F29 PP = f29_quad<0, 0, 0, 0>(r2);
     const F29 r3 = k.mul(f29_sel(k.m2, r2, f29_sel(k.m1, f29_quad<0, 0, 0, 0>(r1), D)), PP);   // PPP, Q, ZZ3, -
     const F29 PPP = f29_quad<0, 0, 0, 0>(r3), Q = f29_quad<1, 1, 1, 1>(r3), RR = f29_quad<1, 1, 1, 1>(r2);

@@ -38,13 +38,17 @@ constexpr uint32_t P[9] = {0x187cfd47u, 0x010460b6u, 0x1c72a34fu, 0x02d522d0u, 0
                            0x02db40c0u, 0x00a6e141u, 0x0e5c2634u, 0x0030644eu};
 constexpr uint32_t NP = 0x04866389u;
 // 2p and 4p with every limb but the top one in [2^29, 2^30) (borrowed from
-// the next limb), so that kp - b never borrows for normalized b < kp; 3 x 4p
+// the next limb), so that kp - b never borrows for normalized b < kp - 2^232; 3 x 4p
 constexpr uint32_t P2[9] = {0x30f9fa8eu, 0x2208c16cu, 0x38e5469du, 0x25aa45a0u, 0x2b0bb2efu,
                             0x25b68180u, 0x214dc281u, 0x3cb84c67u, 0x0060c89bu};
 constexpr uint32_t P4[9] = {0x21f3f51cu, 0x241182dau, 0x31ca8d3bu, 0x2b548b42u, 0x361765dfu,
                             0x2b6d0301u, 0x229b8503u, 0x397098cfu, 0x00c19138u};
 constexpr uint32_t P12[9] = {0x65dbdf54u, 0x6c34888eu, 0x955fa7b1u, 0x81fda1c6u, 0xa246319du,
                              0x82470903u, 0x67d28f09u, 0xac51ca6du, 0x0244b3a8u};
+// 6p with every limb but the top one in [3 * 2^29 - 3, 2^31) (3 borrowed from
+// the next limb): 6p - a - 2b never borrows for normalized a + 2b < 6p - 2^234
+constexpr uint32_t P6[9] = {0x72edefaau, 0x661a4445u, 0x6aafd3d7u, 0x70fed0e2u, 0x612318cdu,
+                            0x71238481u, 0x63e94783u, 0x7628e535u, 0x012259d3u};
 // 8p with every limb but the top one in [2^30, 2^31): 8p - a - b never
 // borrows for normalized a, b
 constexpr uint32_t P8[9] = {0x43e7ea38u, 0x482305b4u, 0x43951a76u, 0x56a91685u, 0x4c2ecbbeu,
@@ -90,9 +94,12 @@ struct F29ModP {
     static constexpr uint32_t NEG_INV = f29c::NP;
 };
 
+// The sums of products below take an addend c (limbs below 2^32, null: none) into
+// their upper columns, so that a*b/R' + c comes out normalized.
+
 // Montgomery product a*b/R' mod m (product scanning, one 64-bit accumulator)
 template <class M>
-ZK_DEV F29 f29_mul_mod(const F29& a, const F29& b) {
+ZK_DEV F29 f29_mul_mod(const F29& a, const F29& b, const F29* c = nullptr) {
     using namespace f29c;
     uint32_t m[9];
     F29 t;
@@ -113,6 +120,7 @@ ZK_DEV F29 f29_mul_mod(const F29& a, const F29& b) {
             m[k] = f29_qword<M::NEG_INV>((uint32_t)acc);
             acc += (uint64_t)m[k] * M::L[0];
         } else {
+            if (c) acc += c->l[k - 9];
             t.l[k - 9] = (uint32_t)acc & MASK;
         }
         acc >>= 29;
@@ -121,11 +129,11 @@ ZK_DEV F29 f29_mul_mod(const F29& a, const F29& b) {
         // Karatsuba products of Fp2) and runs out of registers
         asm volatile("" : "+v"(acc));
     }
-    t.l[8] = (uint32_t)acc;
+    t.l[8] = (uint32_t)acc + (c ? c->l[8] : 0u);
     return t;
 }
 
-ZK_DEV F29 f29_mul(const F29& a, const F29& b) { return f29_mul_mod<F29ModP>(a, b); }
+ZK_DEV F29 f29_mul(const F29& a, const F29& b, const F29* c = nullptr) { return f29_mul_mod<F29ModP>(a, b, c); }
 
 // Montgomery square a*a/R' mod p for normalized a: 45 partial products
 // (the off-diagonal a_i*a_j, i < j, taken once against 2*a_j, which stays
@@ -171,7 +179,7 @@ ZK_DEV F29 f29_sqr(const F29& a) {
 // result is below 2p. A difference a*b - c*d is the sum with c replaced by
 // f29_neg(c).
 template <int N>
-ZK_DEV F29 f29_mulsum(const F29 (&a)[N], const F29 (&b)[N]) {
+ZK_DEV F29 f29_mulsum(const F29 (&a)[N], const F29 (&b)[N], const F29* c = nullptr) {
     static_assert(N >= 1 && N <= 4, "column sums must stay below 2^64");
     using namespace f29c;
     uint32_t m[9];
@@ -195,12 +203,13 @@ ZK_DEV F29 f29_mulsum(const F29 (&a)[N], const F29 (&b)[N]) {
             m[k] = f29_qword((uint32_t)acc);
             acc += (uint64_t)m[k] * P[0];
         } else {
+            if (c) acc += c->l[k - 9];
             t.l[k - 9] = (uint32_t)acc & MASK;
         }
         acc >>= 29;
         asm volatile("" : "+v"(acc));
     }
-    t.l[8] = (uint32_t)acc;
+    t.l[8] = (uint32_t)acc + (c ? c->l[8] : 0u);
     return t;
 }
 
@@ -246,6 +255,13 @@ ZK_DEV bool f29_eq(const F29& a, const uint32_t (&c)[9]) {
     return d == 0;
 }
 
+ZK_DEV bool f29_is_zero(const F29& a) {
+    uint32_t d = 0;
+#pragma unroll
+    for (int i = 0; i < 9; i++) d |= a.l[i];
+    return d == 0;
+}
+
 // for normalized x = u + 4p - v (u, v < 2p): x = 0 mod p iff x is 3p, 4p or 5p
 ZK_DEV bool f29_sub4_is_zero(const F29& x) {
     using namespace f29c;
@@ -254,11 +270,26 @@ ZK_DEV bool f29_sub4_is_zero(const F29& x) {
     return f29_eq(x, P3N) || f29_eq(x, P4N) || f29_eq(x, P5N);
 }
 
-ZK_DEV bool f29_is_zero(const F29& a) {
-    uint32_t d = 0;
+// value 0 or p (the zeros among products, which stay below 2p)
+ZK_DEV bool f29_zero_mod(const F29& a) {
+    if (a.l[0] != 0 && a.l[0] != f29c::P[0]) return false;
+    return f29_is_zero(a) || f29_eq(a, f29c::P);
+}
+
+// k*p - b limb-wise, an addend or operand, for b as the constant allows
+template <int N>
+ZK_DEV F29 f29_from(const uint32_t (&kp)[N], const F29& b) {
+    F29 r;
 #pragma unroll
-    for (int i = 0; i < 9; i++) d |= a.l[i];
-    return d == 0;
+    for (int i = 0; i < 9; i++) r.l[i] = kp[i] - b.l[i];
+    return r;
+}
+// 6p - a - 2b limb-wise: the addend of X3 = R^2 - PPP - 2Q
+ZK_DEV F29 f29_x3_addend(const F29& a, const F29& b) {
+    F29 r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.l[i] = f29c::P6[i] - a.l[i] - 2 * b.l[i];
+    return r;
 }
 
 // -y for y < p: 2p - y normalized (value in (p, 2p])
@@ -341,8 +372,10 @@ struct Xyzz29 {
 // madd-2008-s, acc += (x2, y2) with x2 < p and y2 < 2p, normalized or the
 // unnormalized negation of a value below p (f29_neg_lazy2). The equal-x
 // cases (doubling, or the sum is infinity) are rare: the doubling goes through
-// the standard-form formulas.
-ZK_DEV void f29_madd(Xyzz29& A, const F29& x2, const F29& y2) {
+// the standard-form formulas, over the point read again by again(x, y), so that
+// its coordinates need no registers up to there.
+template <class Again>
+ZK_DEV void f29_madd(Xyzz29& A, const F29& x2, const F29& y2, Again again) {
     using namespace f29c;
     if (A.inf) {
         A.X = x2;
@@ -358,9 +391,11 @@ ZK_DEV void f29_madd(Xyzz29& A, const F29& x2, const F29& y2) {
     const F29 R_ = f29_norm(f29_sub4(S2, A.Y));
     if (f29_sub4_is_zero(P_)) {
         if (f29_sub4_is_zero(R_)) {
+            F29 x, y;
+            again(x, y);
             Aff<Fp> a;
-            a.x = f29_to_std(x2);
-            a.y = f29_to_std(y2);
+            a.x = f29_to_std(x);
+            a.y = f29_to_std(y);
             const Xyzz<Fp> d = xyzz_mdbl(a);
             A.X = f29_from_std(d.X);
             A.Y = f29_from_std(d.Y);
@@ -466,8 +501,8 @@ ZK_DEV Xyzz29 f29_xyzz_add(const Xyzz29& p, const Xyzz29& q) {
     return r;
 }
 
-// An XYZZ point of this form in 32 words: X, Y, ZZ, ZZZ packed (values < 2p
-// fit 256 bits). Infinity is stored with ZZ = 0, which no finite point has
+// An XYZZ point of this form in 32 words: X, Y, ZZ, ZZZ packed
+// (values < 2p fit 256 bits). Infinity is stored with ZZ = 0, which no finite point has
 // (its ZZ is a nonzero square mod p, so neither 0 nor p).
 ZK_DEV void xyzz29_pack(const Xyzz29& p, uint32_t w[32]) {
     f29_pack(p.X, w);
@@ -513,6 +548,11 @@ ZK_DEV void f29_load_point(const void* base, uint32_t ref, F29& x, F29& y) {
                      ((ref >> 28) & 4u);
     y = f29_load_packed(p);
     x = f29_load_packed(p + 2);
+}
+// the same with the digit's sign: y lies below 2p, unnormalized if negated
+ZK_DEV void f29_load_signed(const void* base, uint32_t ref, F29& x, F29& y) {
+    f29_load_point(base, ref, x, y);
+    if (ref >> 31) y = f29_neg_lazy2(y);
 }
 
 // ---------------------------------------------------------------- Fr (NTT)
@@ -594,25 +634,29 @@ struct F29q {
 // -b1 = 4p - b1 unnormalized (a column stays below 63 * 2^58); result N. Four products and two reductions
 // cost fewer instructions than Karatsuba's three products, three reductions
 // and the normalisations of its differences.
-ZK_DEV F29q f29q_mul(const F29q& a, const F29q& b) {
+// c: an addend per component.
+ZK_DEV F29q f29q_mul(const F29q& a, const F29q& b, const F29q* c = nullptr) {
     const F29 x[2] = {a.c0, a.c1};
     const F29 y0[2] = {b.c0, f29_neg_lazy4(b.c1)}, y1[2] = {b.c1, b.c0};
-    return {f29_mulsum<2>(x, y0), f29_mulsum<2>(x, y1)};
+    return {f29_mulsum<2>(x, y0, c ? &c->c0 : nullptr), f29_mulsum<2>(x, y1, c ? &c->c1 : nullptr)};
 }
 
-// a: components N. (a0+a1)(a0-a1) + (2 a0 a1) u; result N.
-ZK_DEV F29q f29q_sqr(const F29q& a) {
+// a: components normalized, below 3.2p. (a0+a1)(a0-a1) + (2 a0 a1) u, the
+// products below 46p^2; result below 1.3p (without the addend c).
+ZK_DEV F29q f29q_sqr(const F29q& a, const F29q* c = nullptr) {
     const F29 d = f29_norm(f29_sub4(a.c0, a.c1));
-    return {f29_mul(f29_add(a.c0, a.c1), d), f29_mul(f29_add(a.c0, a.c0), a.c1)};
+    return {f29_mul(f29_add(a.c0, a.c1), d, c ? &c->c0 : nullptr),
+            f29_mul(f29_add(a.c0, a.c0), a.c1, c ? &c->c1 : nullptr)};
 }
 
-// a - b component-wise for N inputs: reduced to N, or only normalized (< 6p)
-ZK_DEV F29q f29q_sub(const F29q& a, const F29q& b) {
-    return {f29_reduce(f29_norm(f29_sub4(a.c0, b.c0))), f29_reduce(f29_norm(f29_sub4(a.c1, b.c1)))};
-}
+// a - b + 4p component-wise for N inputs, normalized (< 6p)
 ZK_DEV F29q f29q_sub_nr(const F29q& a, const F29q& b) {
     return {f29_norm(f29_sub4(a.c0, b.c0)), f29_norm(f29_sub4(a.c1, b.c1))};
 }
+template <int N>
+ZK_DEV F29q f29q_from(const uint32_t (&kp)[N], const F29q& b) { return {f29_from(kp, b.c0), f29_from(kp, b.c1)}; }
+ZK_DEV F29q f29q_x3_addend(const F29q& a, const F29q& b) { return {f29_x3_addend(a.c0, b.c0), f29_x3_addend(a.c1, b.c1)}; }
+ZK_DEV bool f29q_zero_mod(const F29q& x) { return f29_zero_mod(x.c0) && f29_zero_mod(x.c1); }
 
 ZK_DEV F29q f29q_from_std(const Fq2& x) { return {f29_from_std(x.c0), f29_from_std(x.c1)}; }
 ZK_DEV Fq2 f29q_to_std(const F29q& v) { return {f29_to_std(v.c0), f29_to_std(v.c1)}; }
@@ -620,7 +664,6 @@ ZK_DEV Fq2 f29q_to_std(const F29q& v) { return {f29_to_std(v.c0), f29_to_std(v.c
 // ---- general XYZZ operations over Fp2 in this form (the G2 bucket
 // reduction); bounds as in f29q_madd
 ZK_DEV F29q f29q_reduce(const F29q& a) { return {f29_reduce(a.c0), f29_reduce(a.c1)}; }
-ZK_DEV bool f29q_sub_is_zero(const F29q& x) { return f29_sub4_is_zero(x.c0) && f29_sub4_is_zero(x.c1); }
 
 // T*A - B*C, each component one sum of four products with one reduction:
 // T normalized < 6p, A, B, C N; the negations are 4p - x unnormalized (two of
@@ -672,31 +715,24 @@ ZK_DEV Xyzz29q f29q_xyzz_dbl(const Xyzz29q& p) {
     return r;
 }
 
-// add-2008-s over Fp2
+// add-2008-s over Fp2, bounds as in f29q_madd: U, S < 1.1p, P, R in (0.9p, 3.2p)
 ZK_DEV Xyzz29q f29q_xyzz_add(const Xyzz29q& p, const Xyzz29q& q) {
     using namespace f29c;
     if (p.inf) return q;
     if (q.inf) return p;
-    const F29q U1 = f29q_mul(p.X, q.ZZ), U2 = f29q_mul(q.X, p.ZZ);
-    const F29q S1 = f29q_mul(p.Y, q.ZZZ), S2 = f29q_mul(q.Y, p.ZZZ);
-    const F29q Pn = f29q_sub_nr(U2, U1), Rn = f29q_sub_nr(S2, S1);
-    if (f29q_sub_is_zero(Pn)) {
-        if (f29q_sub_is_zero(Rn)) return f29q_xyzz_dbl(p);
+    const F29q U1 = f29q_mul(p.X, q.ZZ), nU1 = f29q_from(P2, U1);
+    const F29q S1 = f29q_mul(p.Y, q.ZZZ), nS1 = f29q_from(P2, S1);
+    const F29q P_ = f29q_mul(q.X, p.ZZ, &nU1), R_ = f29q_mul(q.Y, p.ZZZ, &nS1);
+    const F29q PP = f29q_sqr(P_);
+    if (f29q_zero_mod(PP)) {
+        if (f29q_zero_mod(f29q_sqr(R_))) return f29q_xyzz_dbl(p);
         return xyzz29q_inf();
     }
-    const F29q P_ = f29q_reduce(Pn), R_ = f29q_reduce(Rn);
-    const F29q PP = f29q_sqr(P_);
     const F29q PPP = f29q_mul(P_, PP);
     const F29q Q = f29q_mul(U1, PP);
-    const F29q RR = f29q_sqr(R_);
-    F29 x0, x1;
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        x0.l[i] = (P12[i] - PPP.c0.l[i] - 2 * Q.c0.l[i]) + RR.c0.l[i];
-        x1.l[i] = (P12[i] - PPP.c1.l[i] - 2 * Q.c1.l[i]) + RR.c1.l[i];
-    }
+    const F29q nX3 = f29q_x3_addend(PPP, Q);
     Xyzz29q r;
-    r.X = {f29_reduce(f29_norm(x0)), f29_reduce(f29_norm(x1))};
+    r.X = f29q_reduce(f29q_sqr(R_, &nX3));
     r.Y = f29q_mul_sub_mul(f29q_sub_nr(Q, r.X), R_, S1, PPP);
     r.ZZ = f29q_mul(f29q_mul(p.ZZ, q.ZZ), PP);
     r.ZZZ = f29q_mul(f29q_mul(p.ZZZ, q.ZZZ), PPP);
@@ -745,6 +781,10 @@ ZK_DEV void f29q_load_point(const void* base, uint32_t ref, F29q& x, F29q& y) {
     x.c0 = f29_load_packed(p + 4);
     x.c1 = f29_load_packed(p + 6);
 }
+ZK_DEV void f29q_load_signed(const void* base, uint32_t ref, F29q& x, F29q& y) {
+    f29q_load_point(base, ref, x, y);
+    if (ref >> 31) y = {f29_neg_lazy2(y.c0), f29_neg_lazy2(y.c1)};
+}
 
 // A G2 XYZZ accumulator: X, Y and ZZZ in LDS, 3 coordinates x 18 limbs laid
 // out [coordinate][limb][lane] over a block of NT threads (consecutive lanes
@@ -785,30 +825,41 @@ struct AccLds {
 
 // madd-2008-s over Fp2 on that accumulator, acc += (x2, y2) with components
 // of x2 < p and y2 < 2p, normalized or f29_neg_lazy2 of values below p; inf
-// tracks the empty/infinite sum. The
-// equal-x cases go through the standard-form formulas.
-template <int NT>
-ZK_DEV void f29q_madd(AccLds<NT>& A, bool& inf, const F29q& x2, const F29q& y2) {
+// tracks the empty/infinite sum. The equal-x cases go through the standard-form
+// formulas, over the point read again as in f29_madd; they show in PP = P^2 = 0
+// mod p.
+// Bounds in units of p: X < 1.01 (reduced), Y < 1.4, ZZ, ZZZ < 2. P = x2*ZZ + 2 -
+// X in (0.9, 3.1), R = y2*ZZZ + 2 - Y in (0.6, 3.2): small enough for f29q_sqr
+// as they are. PP < 1.3, PPP, Q < 1.2; R^2 + 6 - PPP - 2Q in (2.4, 7.3), reduced
+// to X3; T = Q + 4 - X3 < 5.2.
+template <int NT, class Again>
+ZK_DEV void f29q_madd(AccLds<NT>& A, bool& inf, const F29q& x2, const F29q& y2, Again again) {
     using namespace f29c;
     using L = AccLds<NT>;
     if (inf) {
         const F29q one = {f29_const(ONE), F29{}};
         A.st(L::X, x2);
-        A.st(L::Y, F29q{f29_norm(y2.c0), f29_norm(y2.c1)});
+        A.st(L::Y, F29q{f29_reduce(f29_norm(y2.c0)), f29_reduce(f29_norm(y2.c1))});
         A.st(L::ZZ, one);
         A.st(L::ZZZ, one);
         inf = false;
         return;
     }
-    const F29q U2 = f29q_mul(x2, A.ld(L::ZZ));
-    const F29q S2 = f29q_mul(y2, A.ld(L::ZZZ));
-    const F29q Pn = f29q_sub_nr(U2, A.ld(L::X));   // normalized, in (2p, 6p): zero test
-    const F29q Rn = f29q_sub_nr(S2, A.ld(L::Y));
-    if (f29_sub4_is_zero(Pn.c0) && f29_sub4_is_zero(Pn.c1)) {
-        if (f29_sub4_is_zero(Rn.c0) && f29_sub4_is_zero(Rn.c1)) {
+    F29q P_, R_;
+    {
+        const F29q nX = f29q_from(P2, A.ld(L::X));
+        P_ = f29q_mul(x2, A.ld(L::ZZ), &nX);
+        const F29q nY = f29q_from(P2, A.ld(L::Y));
+        R_ = f29q_mul(y2, A.ld(L::ZZZ), &nY);
+    }
+    const F29q PP = f29q_sqr(P_);
+    if (f29q_zero_mod(PP)) {
+        if (f29q_zero_mod(f29q_sqr(R_))) {
+            F29q x, y;
+            again(x, y);
             Aff<Fq2> a;
-            a.x = f29q_to_std(x2);
-            a.y = f29q_to_std(y2);
+            a.x = f29q_to_std(x);
+            a.y = f29q_to_std(y);
             const Xyzz<Fq2> d = xyzz_mdbl(a);
             A.st(L::X, f29q_from_std(d.X));
             A.st(L::Y, f29q_from_std(d.Y));
@@ -819,30 +870,17 @@ ZK_DEV void f29q_madd(AccLds<NT>& A, bool& inf, const F29q& x2, const F29q& y2) 
         }
         return;
     }
-    const F29q P_ = {f29_reduce(Pn.c0), f29_reduce(Pn.c1)};
-    const F29q PP = f29q_sqr(P_);
     const F29q PPP = f29q_mul(P_, PP);
     A.st(L::ZZ, f29q_mul(A.ld(L::ZZ), PP));
     A.st(L::ZZZ, f29q_mul(A.ld(L::ZZZ), PPP));
     const F29q Q = f29q_mul(A.ld(L::X), PP);
-    const F29q R_ = {f29_reduce(Rn.c0), f29_reduce(Rn.c1)};
-    F29q X3;
-    {
-        const F29q RR = f29q_sqr(R_);
-        F29 x0, x1;
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-            x0.l[i] = (P12[i] - PPP.c0.l[i] - 2 * Q.c0.l[i]) + RR.c0.l[i];
-            x1.l[i] = (P12[i] - PPP.c1.l[i] - 2 * Q.c1.l[i]) + RR.c1.l[i];
-        }
-        X3 = {f29_reduce(f29_norm(x0)), f29_reduce(f29_norm(x1))};
-    }
+    const F29q nX3 = f29q_x3_addend(PPP, Q);
+    const F29q X3 = f29q_reduce(f29q_sqr(R_, &nX3));
     A.st(L::X, X3);
-    // Y3 = (Q - X3)*R - Y1*PPP, each Fp2 component as one sum of four
-    // products with one reduction: T = Q - X3 < 6p, R, Y1, PPP < 2p and the
-    // negations 4p - x unnormalized (f29_neg_lazy4), so the products sum
-    // below 48p^2 and a column, two of whose four terms carry a negation,
-    // below 63 * 2^58
+    // Y3 = T*R - Y1*PPP, each Fp2 component as one sum of four products with one
+    // reduction; the negations are 4p - x unnormalized (f29_neg_lazy4), so the
+    // products sum below 46p^2 and a column, two of whose four terms carry a
+    // negation, below 63 * 2^58
     const F29q T = f29q_sub_nr(Q, X3);
     const F29q Y1 = A.ld(L::Y);
     const F29 nr1 = f29_neg_lazy4(R_.c1), ny0 = f29_neg_lazy4(Y1.c0), ny1 = f29_neg_lazy4(Y1.c1);

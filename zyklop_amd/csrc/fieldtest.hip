@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(64) k_point_probe(int op, uint32_t iters, uint
     for (uint32_t it = 0; it < iters; it++) {
 #pragma unroll 1
         for (int r = 0; r < 16; r++) {
-            if (op == 4) f29_madd(p, q.X, q.Y);
+            if (op == 4) f29_madd(p, q.X, q.Y, [&](F29& x, F29& y) { x = q.X; y = q.Y; });
             else p = f29_xyzz_add(p, q);
         }
     }

@@ -17,12 +17,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     Xyzz29 acc;
     acc.inf = true;
     for (uint32_t e = st; e < en; e++) {
-        uint32_t ref = entries[e];
+        const uint32_t ref = entries[e];
         F29 x, y;
         f29_load_point(points29, ref, x, y);
         if (f29_is_zero(x) && f29_is_zero(y)) continue;   // infinity
         if (ref >> 31) y = f29_neg_lazy2(y);   // f29_madd takes it unnormalized
-        f29_madd(acc, x, y);
+        f29_madd(acc, x, y, [&](F29& px, F29& py) { f29_load_signed(points29, ref, px, py); });
     }
     red_store<Fp>(buckets, slot, acc);
 }

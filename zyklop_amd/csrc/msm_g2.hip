@@ -11,6 +11,11 @@ namespace zk {
 // register file next to the mixed add, so three coordinates of each thread's
 // bucket accumulator live in LDS (field29.hpp AccLds) and are loaded where
 // used. One-wave blocks let the LDS share set the waves per CU.
+// Bound by instruction issue at 2 waves per SIMD (172 VGPRs): 2^20 points, 16.8 M
+// entries, 4.11 ms for the call, 4.34 with P and R reduced before they are squared
+// and the coordinates of a point held for the doubling (230 VGPRs). 3 waves per
+// SIMD (168 VGPRs, but LDS for 11 waves per CU) 4.66 ms; the next entry's point
+// loaded an addition ahead 4.10 ms, no faster in proofs.
 constexpr int ACC29Q_THREADS = 64;
 __global__ void __launch_bounds__(ACC29Q_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_msm_accum29q(
     const uint32_t* __restrict__ entries, const uint32_t* __restrict__ offsets, uint32_t nb, uint32_t split, uint32_t lmax,
@@ -25,12 +30,12 @@ __global__ void __launch_bounds__(ACC29Q_THREADS) __attribute__((amdgpu_waves_pe
     AccLds<ACC29Q_THREADS> A{lds + threadIdx.x, {}};
     bool inf = true;
     for (uint32_t e = st; e < en; e++) {
-        uint32_t ref = entries[e];
+        const uint32_t ref = entries[e];
         F29q x, y;
         f29q_load_point(points29, ref, x, y);
         if (f29_is_zero(x.c0) && f29_is_zero(x.c1) && f29_is_zero(y.c0) && f29_is_zero(y.c1)) continue;
         if (ref >> 31) y = {f29_neg_lazy2(y.c0), f29_neg_lazy2(y.c1)};   // f29q_madd takes it unnormalized
-        f29q_madd(A, inf, x, y);
+        f29q_madd(A, inf, x, y, [&](F29q& px, F29q& py) { f29q_load_signed(points29, ref, px, py); });
     }
     using L = AccLds<ACC29Q_THREADS>;
     red_store<Fq2>(buckets, slot, Xyzz29q{A.ld(L::X), A.ld(L::Y), A.ld(L::ZZ), A.ld(L::ZZZ), inf});

@@ -155,7 +155,7 @@ struct LaneSum<Fp> {
         F29 x, y;
         f29_load_point(pts, ref, x, y);
         if (f29_is_zero(x) && f29_is_zero(y)) return;   // infinity
-        f29_madd(a, x, ref >> 31 ? f29_neg_lazy2(y) : y);
+        f29_madd(a, x, ref >> 31 ? f29_neg_lazy2(y) : y, [&](F29& px, F29& py) { f29_load_signed(pts, ref, px, py); });
     }
     ZK_DEV bool inf() const { return a.inf; }
     ZK_DEV F29 coord(int q, int) const { return q == 0 ? a.X : q == 1 ? a.Y : q == 2 ? a.ZZ : a.ZZZ; }
@@ -171,7 +171,7 @@ struct LaneSum<Fq2> {
         f29q_load_point(pts, ref, x, y);
         if (f29_is_zero(x.c0) && f29_is_zero(x.c1) && f29_is_zero(y.c0) && f29_is_zero(y.c1)) return;
         if (ref >> 31) y = {f29_neg_lazy2(y.c0), f29_neg_lazy2(y.c1)};
-        f29q_madd(a, empty, x, y);
+        f29q_madd(a, empty, x, y, [&](F29q& px, F29q& py) { f29q_load_signed(pts, ref, px, py); });
     }
     ZK_DEV bool inf() const { return empty; }
     ZK_DEV F29 coord(int q, int c) const {
