@@ -495,6 +495,13 @@ void ProveSlot::body(Context& ctx, const Circuit& c, ProofParts& out) {
     if (timed) ZK_HIP(hipEventRecord(ev[2], s0));
     ntt_run(plan, tmp, abc, 3, false, nullptr, nullptr, s0);          // values at w_2n^(2j+1)
     if (timed) ZK_HIP(hipEventRecord(ev[3], s0));
+    // The accumulations start after the transforms: their waves stay for a
+    // millisecond and more and leave a transform's workgroups waiting (one pass of
+    // the 2^20-constraint proof 5.2 ms instead of 0.25), and with them the H MSM,
+    // which then ran alone at the end. Proof of 2^20 constraints 10.5 -> 10.2 ms,
+    // 200003 constraints 2.20 -> 2.16; waiting for the sort of h as well 10.4 and 2.25.
+    ZK_HIP(hipEventRecord(ev_h, s0));
+    for (hipStream_t p : {s1, s2}) ZK_HIP(hipStreamWaitEvent(p, ev_h, 0));
     h_final(aw.p, bw.p, cw.p, h.p, n, s0);
     sortH.run(h.p, n, window_h, s0, pl.mh);
     msm_launch_main(sortW, true, &b2, 1, s2);
