@@ -53,11 +53,29 @@ ZK_DEV void st29_lazy(void* base, size_t i, const F29& x) {
 ZK_DEV F29 settle29(const F29& x) { return fr29_reduce(f29_norm(x)); }
 
 // root i of the DFTs inside a unit, w_256^i in limbs, 12 words apart
+constexpr int ROOTS = 256;
+static_assert(NTT_THREADS == ROOTS, "k_ntt_quad: a root a thread");
 constexpr int ROOT_WORDS = 12;
 ZK_DEV F29 ld_root(const void* roots, uint32_t i) {
     const uint4* p = reinterpret_cast<const uint4*>(roots) + ROOT_WORDS / 4 * i;
     const uint4 a = p[0], b = p[1];
     return F29{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, reinterpret_cast<const uint32_t*>(p + 2)[0]}};
+}
+// The same in a workgroup's LDS, limb by limb: [9][ROOTS]. For k_ntt_quad, where
+// 13 gathers of scattered roots a lane kept the address unit busy beside the
+// twiddles and points: 2^22 points 506 -> 488 us, three arrays of 2^20 378 -> 374.
+// k_ntt_lane reads them from the cache: fewer roots a lane, and the copy comes
+// first in a launch that waits for nothing else (three arrays of 2^18 125 us
+// from LDS, 124 from the cache).
+ZK_DEV void st_root_lds(uint32_t* sh, uint32_t i, const F29& r) {
+#pragma unroll
+    for (int l = 0; l < 9; l++) sh[l * ROOTS + i] = r.l[l];
+}
+ZK_DEV F29 ld_root_lds(const uint32_t* sh, uint32_t i) {
+    F29 r;
+#pragma unroll
+    for (int l = 0; l < 9; l++) r.l[l] = sh[l * ROOTS + i];
+    return r;
 }
 
 // what a pass reads and writes: unit u of 2^q points. Passes 0..np-2, in place
@@ -207,11 +225,11 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_lane(NttPtrs ptrs, NttShape
 // instruction per limb for both points), then 1, 0 (DPP in a quad); 3, 2 only
 // in units of 2^7 points and more. The bits left over number the wave's units.
 // Bound by instruction issue: 5044 VALU instructions per lane for 2^8 points per
-// unit (3336 for 2^6), 60 % of them v_mad_u64_u32; the 2^22 transform is three
-// launches of 165, 165 and 110 us and its instructions alone take 0.38 ms. Four
-// waves per SIMD (five are the same, six spill 12 %). The radix-8 threads before
-// took four launches, 0.56 ms (call 617 -> 522 us); eight points per lane with
-// the same exchange held three waves per SIMD and 563 us.
+// unit (3336 for 2^6), 60 % of them v_mad_u64_u32, which alone take 0.38 ms of the
+// 2^22 transform. Four waves per SIMD (five are the same, six spill 12 %). The
+// radix-8 threads before took four launches (call 617 us, now 488); eight points
+// per lane with the same exchange held three waves per SIMD and 563 us. Products
+// with a stored b' = floor(b 2^261 / r) instead of Montgomery's: the same time.
 constexpr int quad_bit(int Q, int i) {   // lane bit of the i-th bit from the top of the unit's lane
     return Q == 8 ? 5 - i : Q == 7 ? (i < 2 ? 5 - i : i < 4 ? 3 - i : 3) : (i < 2 ? 5 - i : 3 - i);
 }
@@ -238,7 +256,7 @@ ZK_DEV void dft4(F29 (&x)[4], const F29& w4) {
 // step T of a unit of 2^Q points, the digit over what lies below it in the lane
 template <int Q, int T>
 struct QuadStep {
-    ZK_DEV static void run(F29 (&x)[4], uint32_t lane, const void* roots, const F29& w4) {
+    ZK_DEV static void run(F29 (&x)[4], uint32_t lane, const uint32_t* roots, const F29& w4) {
         constexpr int LEFT = Q - 2 * T;   // bits below this step's digit
         dft4(x, w4);
         if constexpr (LEFT > 0) {
@@ -246,7 +264,7 @@ struct QuadStep {
             x[0] = settle29(x[0]);
 #pragma unroll
             for (uint32_t k = 1; k < 4; k++)   // w_{2^(LEFT + 2)}^(rest * k)
-                x[k] = fr29_mul(x[k], ld_root(roots, (rest * k) << (8 - LEFT - 2)));
+                x[k] = fr29_mul(x[k], ld_root_lds(roots, (rest * k) << (8 - LEFT - 2)));
             if constexpr (LEFT == 1) {
                 lane_swap<quad_bit(Q, Q - 3)>(x[0], x[2]);
                 lane_swap<quad_bit(Q, Q - 3)>(x[1], x[3]);
@@ -267,6 +285,8 @@ struct QuadStep {
 template <int Q>
 __global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_ntt_quad(NttPtrs ptrs, NttShape z) {
     constexpr int LB = Q - 2;            // lane bits of a unit
+    __shared__ uint32_t roots[9 * ROOTS];
+    const F29 root = ld_root(z.roots, threadIdx.x);
     const uint32_t hw = threadIdx.x & 63;
     uint32_t lane = 0, used = 0, sub = 0;   // the unit's lane; the unit in the wave
 #pragma unroll
@@ -277,18 +297,20 @@ __global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int i = 0, k = 0; i < 6; i++)
         if (!(used >> i & 1u)) sub |= (hw >> i & 1u) << k++;
-    const size_t u = (((size_t)blockIdx.x * (NTT_THREADS / 64) + threadIdx.x / 64) << (6 - LB)) + sub;
-    if (u >= z.n >> Q) return;   // whole units
+    const size_t u = (((size_t)blockIdx.x * (NTT_THREADS / 64) + threadIdx.x / 64) << (6 - LB)) + sub, units = z.n >> Q;
     const void* in = ptrs.in[blockIdx.y];
-    const NttUnit t = ntt_unit<Q>(z, u);
+    const NttUnit t = ntt_unit<Q>(z, u < units ? u : units - 1);
     F29 x[4];
 #pragma unroll
     for (uint32_t i = 0; i < 4; i++) x[i] = ld29(in, t.in + (lane + (i << LB)) * t.in_step);
+    st_root_lds(roots, threadIdx.x, root);
+    __syncthreads();
+    if (u >= units) return;   // whole units
     if (z.pre) {
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) x[i] = fr29_mul(x[i], ld29(z.pre, t.in + (lane + (i << LB)) * t.in_step));
     }
-    QuadStep<Q, 1>::run(x, lane, z.roots, ld_root(z.roots, 64));
+    QuadStep<Q, 1>::run(x, lane, roots, ld_root_lds(roots, 64));
     // output of slot s: digits k_1.. from the lane's top bits, the last from the slot
     uint32_t k0 = 0;
 #pragma unroll
@@ -367,7 +389,7 @@ static int ntt_layout(int ln, int lr[NTT_MAX_PASSES]) {
 // Two points per lane below 2^20 points in all, where four leave less than four
 // waves per SIMD: three arrays of 2^18 125 against 130 us, one of 2^19 101
 // against 107, three of 2^17 89 against 103; from 2^20 on four are faster (three
-// of 2^20 395 against 415, one of 2^22 522 against 569).
+// of 2^20 374 against 415, one of 2^22 488 against 569).
 static bool ntt_two_points(int ln, size_t points) {
     return ln <= NTT_LANE_LOG || (ln <= 19 && points < ((size_t)1 << 20));   // 2^20 and up have 2^8 passes
 }
@@ -388,7 +410,7 @@ size_t NttPlan::bytes_for(int ln) {
     int lr_[NTT_MAX_PASSES];
     const int np_ = ntt_layout(ln, lr_);
     const size_t tot = ntt_tw_entries(ln, np_, lr_, nullptr);
-    return 2 * std::max<size_t>(tot, 1) * 32 + 2 * 256 * ROOT_WORDS * 4 + 4 * ((size_t)1 << ln) * 32;
+    return 2 * std::max<size_t>(tot, 1) * 32 + 2 * ROOTS * ROOT_WORDS * 4 + 4 * ((size_t)1 << ln) * 32;
 }
 
 void NttPlan::build(int ln, hipStream_t st) {
@@ -421,8 +443,8 @@ void NttPlan::build(int ln, hipStream_t st) {
     for (int d = 0; d < 2; d++) {
         const zkh::Fr g = d ? root_of_unity(8).inv() : root_of_unity(8);
         zkh::Fr f = s32;
-        limbs[d].assign(256 * ROOT_WORDS, 0);
-        for (int i = 0; i < 256; i++, f = f * g)
+        limbs[d].assign(ROOTS * ROOT_WORDS, 0);
+        for (int i = 0; i < ROOTS; i++, f = f * g)
             for (int l = 0; l < 9; l++) {
                 const int k = 29 * l / 64, sh = 29 * l % 64;
                 uint64_t v = f.v[k] >> sh;
@@ -430,8 +452,8 @@ void NttPlan::build(int ln, hipStream_t st) {
                 limbs[d][ROOT_WORDS * i + l] = (uint32_t)v & f29c::MASK;
             }
         DevBuf& dst = d ? roots_inv : roots_fwd;
-        dst.ensure(256 * ROOT_WORDS * 4);
-        ZK_HIP(hipMemcpyAsync(dst.p, limbs[d].data(), 256 * ROOT_WORDS * 4, hipMemcpyHostToDevice, st));
+        dst.ensure(ROOTS * ROOT_WORDS * 4);
+        ZK_HIP(hipMemcpyAsync(dst.p, limbs[d].data(), ROOTS * ROOT_WORDS * 4, hipMemcpyHostToDevice, st));
     }
     // pass twiddle tables w_M^(c k), layout [k][c], for passes 0..np-2
     const size_t tot = ntt_tw_entries(ln, np, lr, tw_off);
