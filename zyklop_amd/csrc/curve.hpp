@@ -93,10 +93,9 @@ ZK_DEV Xyzz<T> xyzz_mdbl(const Aff<T>& a) {
     return {X3, Y3, V, W};
 }
 
-// dbl-2008-s-1, a = 0 (inline form; the rare equal-points branch of the
-// additions uses it so that their operands never need an address)
+// dbl-2008-s-1, a = 0, out of line: one copy per kernel
 template <class T>
-ZK_DEV Xyzz<T> xyzz_dbl_i(const Xyzz<T>& p) {
+ZK_NOINL Xyzz<T> xyzz_dbl(const Xyzz<T>& p) {
     T U = add(p.Y, p.Y);
     T V = sqr(U);
     T W = mul(U, V);
@@ -108,9 +107,6 @@ ZK_DEV Xyzz<T> xyzz_dbl_i(const Xyzz<T>& p) {
     // doubling infinity keeps ZZ = 0
     return {X3, Y3, mul(V, p.ZZ), mul(W, p.ZZZ)};
 }
-// out-of-line form for code outside the hot loops (one copy per kernel)
-template <class T>
-ZK_NOINL Xyzz<T> xyzz_dbl(const Xyzz<T>& p) { return xyzz_dbl_i(p); }
 
 // madd-2008-s: acc += a (a affine, not infinity)
 template <class T>
@@ -139,77 +135,21 @@ ZK_DEV void xyzz_madd(Xyzz<T>& acc, const Aff<T>& a) {
     acc.ZZZ = mul(acc.ZZZ, PPP);
 }
 
-// add-2008-s: p + q, both XYZZ
-template <class T>
-ZK_DEV Xyzz<T> xyzz_add_i(const Xyzz<T>& p, const Xyzz<T>& q) {
-    if (xyzz_is_inf(p)) return q;
-    if (xyzz_is_inf(q)) return p;
-    T U1 = mul(p.X, q.ZZ);
-    T U2 = mul(q.X, p.ZZ);
-    T S1 = mul(p.Y, q.ZZZ);
-    T S2 = mul(q.Y, p.ZZZ);
-    T P = sub(U2, U1);
-    T R = sub(S2, S1);
-    if (is_zero(P)) {
-        if (is_zero(R)) return xyzz_dbl_i(p);
-        return xyzz_inf<T>();
-    }
-    T PP = sqr(P);
-    T PPP = mul(P, PP);
-    T Q = mul(U1, PP);
-    T X3 = sub(sub(sub(sqr(R), PPP), Q), Q);
-    T Y3 = sub(mul(R, sub(Q, X3)), mul(S1, PPP));
-    return {X3, Y3, mul(mul(p.ZZ, q.ZZ), PP), mul(mul(p.ZZZ, q.ZZZ), PPP)};
-}
-
-// out-of-line form for code outside the hot loops (one copy per kernel)
-template <class T>
-ZK_NOINL Xyzz<T> xyzz_add(const Xyzz<T>& p, const Xyzz<T>& q) { return xyzz_add_i(p, q); }
-
 // ---- global memory access ----
 // G1 affine point: 64 B = x (32 B) then y (32 B). G2: 128 B = x.c0, x.c1, y.c0, y.c1.
 template <class T> struct PointIO;
 
 template <>
 struct PointIO<Fp> {
-    static constexpr int AFF_BYTES = 64;
-    static constexpr int XYZZ_BYTES = 128;
     ZK_DEV static Aff<Fp> load_aff(const void* base, size_t i) {
         return {load<FpCfg>(base, 2 * i), load<FpCfg>(base, 2 * i + 1)};
     }
-    ZK_DEV static Xyzz<Fp> load_xyzz(const void* base, size_t i) {
-        return {load<FpCfg>(base, 4 * i), load<FpCfg>(base, 4 * i + 1), load<FpCfg>(base, 4 * i + 2),
-                load<FpCfg>(base, 4 * i + 3)};
-    }
-    ZK_DEV static void store_xyzz(void* base, size_t i, const Xyzz<Fp>& p) {
-        store<FpCfg>(base, 4 * i, p.X);
-        store<FpCfg>(base, 4 * i + 1, p.Y);
-        store<FpCfg>(base, 4 * i + 2, p.ZZ);
-        store<FpCfg>(base, 4 * i + 3, p.ZZZ);
-    }
-    ZK_DEV static Fp neg_y(const Fp& y) { return neg<FpCfg>(y); }
 };
 
 template <>
 struct PointIO<Fq2> {
-    static constexpr int AFF_BYTES = 128;
-    static constexpr int XYZZ_BYTES = 256;
     ZK_DEV static Fq2 ld2(const void* base, size_t i) { return {load<FpCfg>(base, 2 * i), load<FpCfg>(base, 2 * i + 1)}; }
-    ZK_DEV static void st2(void* base, size_t i, const Fq2& a) {
-        store<FpCfg>(base, 2 * i, a.c0);
-        store<FpCfg>(base, 2 * i + 1, a.c1);
-    }
     ZK_DEV static Aff<Fq2> load_aff(const void* base, size_t i) { return {ld2(base, 2 * i), ld2(base, 2 * i + 1)}; }
-    ZK_DEV static Xyzz<Fq2> load_xyzz(const void* base, size_t i) {
-        return {ld2(base, 4 * i), ld2(base, 4 * i + 1), ld2(base, 4 * i + 2), ld2(base, 4 * i + 3)};
-    }
-    ZK_DEV static void store_xyzz(void* base, size_t i, const Xyzz<Fq2>& p) {
-        st2(base, 4 * i, p.X);
-        st2(base, 4 * i + 1, p.Y);
-        st2(base, 4 * i + 2, p.ZZ);
-        st2(base, 4 * i + 3, p.ZZZ);
-    }
-    ZK_DEV static Fq2 neg_y(const Fq2& y) { return neg(y); }
 };
 
 }  // namespace zk

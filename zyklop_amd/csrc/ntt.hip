@@ -62,7 +62,7 @@ ZK_DEV F29 ld_root(const void* roots, uint32_t i) {
     return F29{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, reinterpret_cast<const uint32_t*>(p + 2)[0]}};
 }
 // The same in a workgroup's LDS, limb by limb: [9][ROOTS]. For k_ntt_quad, where
-// 13 gathers of scattered roots a lane kept the address unit busy beside the
+// ten gathers of scattered roots a lane kept the address unit busy beside the
 // twiddles and points: 2^22 points 506 -> 488 us, three arrays of 2^20 378 -> 374.
 // k_ntt_lane reads them from the cache: fewer roots a lane, and the copy comes
 // first in a launch that waits for nothing else (three arrays of 2^18 125 us
