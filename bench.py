@@ -55,14 +55,14 @@ CALIB_BYTES = 384 << 20                 # device copy before the probes (profile
 # of the sort's 14,737,409 entries the A' probe reads the 11,054,444 of wires
 # with a finite A' base, the B2' probe the 11,052,135 with finite B' bases
 
-HBM_BYTES_PER_ENTRY_G1 = (1.9644e9 + 0.1069e9) / 11054444
-HBM_BYTES_PER_ENTRY_G2 = (1.8688e9 + 0.0671e9) / 11052135
+HBM_BYTES_PER_ENTRY_G1 = (1.9750e9 + 0.1007e9) / 11054444
+HBM_BYTES_PER_ENTRY_G2 = (1.8237e9 + 0.0671e9) / 11052135
 ALGO_BYTES_PER_ENTRY_G1 = 68            # y and x (or beta*x) of the base, 32 B each packed, + the 4 B entry
 ALGO_BYTES_PER_ENTRY_G2 = 132           # the same over Fp2, + the 4 B entry
-# NTT of 2^22, per transform (three pass pairs + the last pass)
-HBM_BYTES_NTT_2P22 = {"forward": 1.2250e9, "inverse": 1.3579e9, "coset": 1.3621e9}
+# NTT of 2^22, per transform (three passes)
+HBM_BYTES_NTT_2P22 = {"forward": 0.9432e9, "inverse": 1.0775e9, "coset": 1.1087e9}
 # SpMV of the 2^20 circuit (k_spmv_abc)
-HBM_BYTES_SPMV_2P20 = 1.3459e9 + 0.2017e9
+HBM_BYTES_SPMV_2P20 = 1.3475e9 + 0.2017e9
 
 
 def log(msg):
@@ -358,13 +358,13 @@ def section_probes(args, zk, ctx, circ):
     gbs = {k: 64 * n / (v / 1e3) / 1e9 for k, v in ntt.items()}
     log(f"[bench] NTT 2^22 ms {ntt} -> GB/s {({k: round(v) for k, v in gbs.items()})}")
     roofline_ntt = {
-        "bound": "hbm", "kernel": "NTT 2^22 (three k_ntt_pass2 launches + k_ntt_final<4>), forward",
+        "bound": "hbm", "kernel": "NTT 2^22 (two k_ntt_quad<8> launches + k_ntt_quad<6>), forward",
         "achieved": round(gbs["forward"], 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
         "frac": round(gbs["forward"] / PEAK_HBM_GBS, 4), "traffic": int(HBM_BYTES_NTT_2P22["forward"]),
         "traffic_by_kind": {k: int(v) for k, v in HBM_BYTES_NTT_2P22.items()},
         "traffic_GBps": {k: round(HBM_BYTES_NTT_2P22[k] / (v / 1e3) / 1e9, 1) for k, v in ntt.items()},
-        "note": ("the passes are mostly instruction-bound (29-bit Fr products), the rest memory latency at 2 waves "
-                 "per SIMD, not HBM bandwidth: the profiler's traffic runs at about a quarter of the HBM peak"),
+        "note": ("the passes are mostly instruction-bound (29-bit Fr products), not HBM-bound: their issue slots alone "
+                 "take 0.38 ms, while the profiler's traffic runs at about a quarter of the HBM peak"),
         "avg_launch_ms": r3(ntt["forward"]), "algorithmic_bytes": 64 * n,
         "ms": {k: r3(v) for k, v in ntt.items()},
         "GBps": {k: round(v, 1) for k, v in gbs.items()},
