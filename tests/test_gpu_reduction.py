@@ -7,6 +7,7 @@ ones (infinity) and infinity on either side."""
 import numpy as np
 import pytest
 
+import oracle as O
 import zyklop_amd as zk
 from tests import pyref
 from tests.test_gpu_parity import mont_pts_g1, mont_pts_g2, oracle_msm_g1, oracle_msm_g2
@@ -91,3 +92,29 @@ def test_oversized_bucket_most_chunks(ctx):
     expect = mont_pts_g1([total])[0]
     got, inf = ctx.msm_g1(pts, vals)
     assert not inf and np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("m", [300, 2500, 8200, 17000])
+def test_parts_of_few_buckets_in_proofs(tmp_path, m):
+    """A proof over few buckets takes more parts per bucket than a tuning table
+    can name: the same proof as with one part and the trapdoor closed form's."""
+    c = zk.Context(0)
+    circ = c.synth_circuit(91, m, 8)
+    w = circ.witness(5)
+    r, s = zk.synth_blinding(6)
+    base = c.prove(circ, w, r, s).words()
+    counted, held, left = c.slot_bytes_check(circ)
+    assert counted == held and left == 0
+    c.autotune(circ)
+    path = tmp_path / "t.txt"
+    c.tune_save(path)
+    rows = [ln.split() for ln in path.read_text().splitlines() if not ln.startswith("#")]
+    path.write_text("".join(" ".join(row[:4]) + " 1 1\n" for row in rows))
+    one = zk.Context(0)
+    one.tune_load(path)
+    assert np.array_equal(one.prove(circ, w, r, s).words(), base)
+    one.close()
+    ref = O.Circuit(91, m, 8, with_crs=False)
+    assert np.array_equal(base, ref.prove_trapdoor(r, s, w=w))
+    circ.free()
+    c.close()

@@ -20,13 +20,28 @@ int msm_default_c(size_t n) {
     return c;
 }
 
+// parts per bucket, a power of two: at most `threads` in all, about two entries each
+static int msm_double_parts(size_t nb, size_t load, size_t threads) {
+    int s = 1;
+    while (s < MSM_SPLIT_MAX && nb * s * 2 <= threads && load >= (size_t)s * 4) s *= 2;
+    return s;
+}
+
 int msm_default_split(size_t n, int c, bool g2, bool merged) {
     const MsmGeom g = msm_geom(n, c, g2, merged);
     // two rounds of waves at 6 (G1) and 3 (G2) waves per SIMD, i.e. three
     // and two rounds at the 4 and 2 the accumulation kernels hold (128 VGPRs;
     // 228 VGPRs and LDS); the autotuner picks the splits of a circuit's sizes
     const size_t target = (size_t)1024 * 64 * 2 * (g2 ? 3 : 6);
-    const size_t nb = (size_t)g.Wr * g.K;
+    const size_t nb = (size_t)g.Wr * g.K, load = 2 * n * (size_t)g.W / nb;
+    // Few buckets: up to half a wave per SIMD for each of a proof's MSMs, while a
+    // part keeps about two entries, as below; the chain of entries per thread set
+    // the time. Proofs of 5000 constraints 531 -> 460 us, 8200 680 -> 510, 11000
+    // 748 -> 547; where it comes to 4 parts (2^13 buckets, 2^14 constraints) the
+    // same. A limit of 2^16 threads is the same, 2^17 slower (2^14 constraints
+    // 656 -> 758 us, 8 proofs of 50021 5.5 -> 6.1 ms).
+    const int s = msm_double_parts(nb, load, (size_t)1 << 15);
+    if (s >= 4) return s;
     return (int)std::max<size_t>(1, std::min<size_t>(3, target / nb));
 }
 
@@ -35,16 +50,16 @@ int msm_default_split(size_t n, int c, bool g2, bool merged) {
 // while every part keeps about two entries: the chain of entries per thread,
 // about 10 us each in a GPU that is not full, gets shorter, and more rounds of
 // waves even out their lengths. Each part costs one addition in the tree.
-// Against at most 3 threads per bucket (other limits in brackets): G1 1000 points 0.52 -> 0.33 ms, 20000 0.48 -> 0.37, 100000 0.61 -> 0.51
-// (2^17 0.61, 2^20 0.57), 400000 and more unchanged; G2 1000 1.10 -> 0.57,
-// 200003 1.88 -> 1.41 (2^18 1.62, 2^20 1.58). In proofs, where five MSMs share
+// Against at most 3 threads per bucket (other limits in brackets): G1 1000
+// points 0.52 -> 0.33 ms, 20000 0.48 -> 0.37, 100000 0.61 -> 0.51 (2^17 0.61,
+// 2^20 0.57), 400000 and more unchanged; G2 1000 1.10 -> 0.57, 200003 1.88 ->
+// 1.41 (2^18 1.62, 2^20 1.58). In proofs, where five MSMs share
 // the GPU, the extra additions cost more than they give (8 proofs of 50021
-// constraints 6.6 ms at 3 threads, 7.1 at 8, 8.4 at 16).
+// constraints 6.6 ms at 3 threads, 7.1 at 8, 8.4 at 16), but where buckets are few.
 int msm_alone_split(size_t n, int c, bool g2) {
     const MsmGeom g = msm_geom(n, c, g2);
     const size_t nb = (size_t)g.Wr * g.K, load = 2 * n * (size_t)g.W / nb;
-    int s = 1;
-    while (s < MSM_SPLIT_MAX && nb * s * 2 <= (1u << 19) && load >= (size_t)s * 4) s *= 2;
+    const int s = msm_double_parts(nb, load, (size_t)1 << 19);
     return s >= 4 ? s : msm_default_split(n, c, g2);
 }
 

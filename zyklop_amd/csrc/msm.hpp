@@ -187,8 +187,9 @@ struct MsmWorkspace {
 // a consecutive part of the bucket's entries; the reduction adds the parts.
 // More threads than buckets fill the GPU when the buckets are few.
 constexpr int MSM_SPLIT_MAX = 64;
-constexpr int MSM_SPLIT_TUNE = 4;   // largest split of a proof's MSMs (autotuner, tables)
-// of a proof's MSMs: about two rounds of resident waves on a 256-CU GPU
+constexpr int MSM_SPLIT_TUNE = 4;   // largest split the autotuner tries and its tables hold
+// of a proof's MSMs: about two rounds of resident waves on a 256-CU GPU at most
+// 3 parts, more for few buckets
 int msm_default_split(size_t n, int c, bool g2, bool merged = false);
 // of an MSM that has the GPU to itself (the MSM entry points over caller-owned
 // points)
