@@ -23,7 +23,7 @@ struct zk_server;
 struct zk_ctx {
     zk::Context impl;
     std::vector<std::unique_ptr<zk::ProveSlot>> batch_slots;
-    zk::MsmWorkspace msm_ws;   // of the MSM entry points, which hold impl.mu
+    zk::KeptWorkspace msm_ws;   // of the MSM entry points, which hold impl.mu
     // servers created on this context: destroying the context finishes and
     // detaches them first (their worker threads use the context)
     std::mutex servers_mu;
@@ -145,27 +145,6 @@ void put_result(const zkh::Xyzz<HT>& p, uint64_t* out, int* is_inf) {
     memcpy(out + lw, &a.y, 8 * lw);
 }
 
-// the context's workspace for one call, or one of the call's own while another
-// thread takes the context's back
-struct WorkspaceUse {
-    std::unique_ptr<zk::MsmWorkspace> own;
-    zk::MsmWorkspace* w;
-    hipStream_t st;
-    WorkspaceUse(zk::MsmWorkspace& kept, hipStream_t s) : w(&kept), st(s) {
-        if (kept.busy.exchange(true)) {
-            own = std::make_unique<zk::MsmWorkspace>();
-            w = own.get();
-            w->busy = true;
-        }
-    }
-    ~WorkspaceUse() {
-        // a call that failed may have left work queued on the buffers
-        if (std::uncaught_exceptions()) (void)hipStreamSynchronize(st);
-        if (w->bytes() > zk::MSM_KEEP_BYTES || std::uncaught_exceptions()) w->release();
-        w->busy = false;
-    }
-};
-
 // MSM over device points; slots29, when given, are the points' 29-bit slots
 // already made (a circuit's resident arrays, W window tables when merged)
 // cls / range: scalar classes and the part of every bucket to read, as a
@@ -176,7 +155,7 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
                 int range = zk::MSM_RANGE_ALL, int split = 0) {
     zk::Context& C = ctx->impl;
     hipStream_t st = C.stream;
-    WorkspaceUse use(ctx->msm_ws, st);
+    zk::WorkspaceUse use(ctx->msm_ws, st);
     zk::MsmSort& sort = use.w->sort;
     zk::MsmScratch& scr = use.w->scr;
     zk::MsmPartials& part = use.w->part;

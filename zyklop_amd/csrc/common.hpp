@@ -32,7 +32,7 @@ struct Error : std::runtime_error {
         if (!(cond)) throw ::zk::Error((code), (msg));      \
     } while (0)
 
-// Gives back the idle MSM workspaces that contexts keep (MsmWorkspace,
+// Gives back the idle MSM workspaces that contexts keep (KeptWorkspace,
 // msm.hpp): they count as free memory. Called where an allocation failed,
 // before it is tried again, and by free_device_bytes().
 void release_idle_workspaces();

@@ -1,5 +1,6 @@
 // Pippenger MSM kernels for G1/G2 on gfx950 (see msm.hpp for the design).
 #include <algorithm>
+#include <exception>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -746,17 +747,17 @@ size_t MsmScratch::bytes() const {
 
 // ---------------------------------------------------------------- workspaces
 static std::mutex g_ws_mu;
-static std::vector<MsmWorkspace*>& workspaces() {
-    static std::vector<MsmWorkspace*> v;
+static std::vector<KeptWorkspace*>& workspaces() {
+    static std::vector<KeptWorkspace*> v;
     return v;
 }
 
-MsmWorkspace::MsmWorkspace() {
+KeptWorkspace::KeptWorkspace() {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     workspaces().push_back(this);
 }
 
-MsmWorkspace::~MsmWorkspace() {
+KeptWorkspace::~KeptWorkspace() {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     auto& v = workspaces();
     v.erase(std::find(v.begin(), v.end(), this));
@@ -768,9 +769,27 @@ void MsmWorkspace::release() {
     p29.release();
 }
 
+WorkspaceUse::WorkspaceUse(KeptWorkspace& k, hipStream_t s) : w(&k), st(s) {
+    if (!k.busy.exchange(true)) {
+        kept = &k;
+        return;
+    }
+    own = std::make_unique<MsmWorkspace>();
+    w = own.get();
+}
+
+WorkspaceUse::~WorkspaceUse() {
+    // a call that failed may have left work queued on the buffers
+    const bool failed = std::uncaught_exceptions() > 0;
+    if (failed) (void)hipStreamSynchronize(st);
+    if (!kept) return;
+    if (failed || kept->bytes() > MSM_KEEP_BYTES) kept->release();
+    kept->busy = false;
+}
+
 void release_idle_workspaces() {
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    for (MsmWorkspace* w : workspaces()) {
+    for (KeptWorkspace* w : workspaces()) {
         if (w->busy.exchange(true)) continue;
         w->release();
         w->busy = false;

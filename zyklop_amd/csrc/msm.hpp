@@ -30,6 +30,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <memory>
 #include <vector>
 
 #include "common.hpp"
@@ -156,26 +157,43 @@ struct MsmScratch {
     size_t bytes() const;   // device bytes held
 };
 
-// What one MSM over caller-owned points works in, kept by a context from one
-// call to the next: allocating and freeing it took up to as long as the MSM (G1
-// calls of 2^22 points 8.5 -> 6.2 ms, of 700001 4.4 -> 1.9, of 1000 0.61 ->
-// 0.54; G2 of 200003 2.9 -> 1.9). A
-// context keeps at most MSM_KEEP_BYTES of device memory (enough for 2^22 G1
-// points); a larger workspace is freed when its call ends, an idle one when an
-// allocation of the library fails, when free memory is asked for, and with its
-// context. busy: in use by a call, or being released.
-constexpr size_t MSM_KEEP_BYTES = (size_t)2 << 30;
+// What one MSM over caller-owned points works in.
 struct MsmWorkspace {
     MsmSort sort;
     MsmScratch scr;
     MsmPartials part;
     DevBuf p29;         // the points' 29-bit slots
     HostBuf entries;    // the sort's entry count
-    std::atomic<bool> busy{false};
-    MsmWorkspace();
-    ~MsmWorkspace();
     size_t bytes() const { return sort.bytes() + scr.bytes() + p29.bytes; }
     void release();     // frees the device buffers
+};
+
+// A context's workspace, kept from one call to the next: allocating and freeing
+// it took up to as long as the MSM (G1 calls of 2^22 points 8.5 -> 6.2 ms, of
+// 700001 4.4 -> 1.9, of 1000 0.61 -> 0.54; G2 of 200003 2.9 -> 1.9). A context
+// keeps at most MSM_KEEP_BYTES of device memory (enough for 2^22 G1 points); a
+// larger workspace is freed when its call ends, an idle one when an allocation of
+// the library fails, when free memory is asked for, and with its context.
+// release_idle_workspaces() finds the kept ones, and only them. busy: in use by a
+// call, or being released; whoever sets it owns the buffers until it is cleared.
+constexpr size_t MSM_KEEP_BYTES = (size_t)2 << 30;
+struct KeptWorkspace : MsmWorkspace {
+    std::atomic<bool> busy{false};
+    KeptWorkspace();
+    ~KeptWorkspace();
+};
+
+// The kept workspace for one call, or while another thread takes it back one of
+// the call's own, which no other thread can reach.
+struct WorkspaceUse {
+    std::unique_ptr<MsmWorkspace> own;
+    KeptWorkspace* kept = nullptr;   // held by this call
+    MsmWorkspace* w;
+    hipStream_t st;
+    WorkspaceUse(KeptWorkspace& k, hipStream_t s);
+    ~WorkspaceUse();
+    WorkspaceUse(const WorkspaceUse&) = delete;
+    WorkspaceUse& operator=(const WorkspaceUse&) = delete;
 };
 
 // Launch bucket accumulation + GPU reduction against a finished sort; its last
