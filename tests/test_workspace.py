@@ -85,3 +85,29 @@ int main() {
 }
 """)
     assert out == "ok"
+
+
+def test_take_back_is_per_device(tmp_path):
+    """Memory needed on one device leaves the workspaces of another alone; idle
+    bytes count what a finished call left, not what a running one holds."""
+    out = run(tmp_path, r"""
+int main() {
+    zk::KeptWorkspace a(0), b(1);
+    char mark;
+    zk::KeptWorkspace* both[2] = {&a, &b};
+    for (int d = 0; d < 2; d++) {
+        zk::WorkspaceUse use(*both[d], nullptr);
+        use.w->p29.borrow(&mark, 100 + d);
+        if (zk::idle_workspace_bytes(d) != 0) return 2;
+    }
+    if (zk::idle_workspace_bytes(0) != 100 || zk::idle_workspace_bytes(1) != 101) return 3;
+    zk::release_idle_workspaces(1);
+    if (a.p29.p != &mark || b.p29.p) return 4;
+    if (zk::idle_workspace_bytes(0) != 100 || zk::idle_workspace_bytes(1) != 0) return 5;
+    zk::release_idle_workspaces();
+    if (a.p29.p || zk::idle_workspace_bytes() != 0) return 6;
+    printf("ok");
+    return 0;
+}
+""")
+    assert out == "ok"

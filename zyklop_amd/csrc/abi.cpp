@@ -32,7 +32,7 @@ struct zk_ctx {
     float last_ms[5] = {0, 0, 0, 0, 0};
     bool profiling = false;
     int batch_slots_n = 3;
-    explicit zk_ctx(int dev) : impl(dev) {
+    explicit zk_ctx(int dev) : impl(dev), msm_ws(dev) {
         ZK_HIP(hipEventCreate(&ev0));
         ZK_HIP(hipEventCreate(&ev1));
         ZK_HIP(hipEventCreate(&ev2));

@@ -32,24 +32,43 @@ struct Error : std::runtime_error {
         if (!(cond)) throw ::zk::Error((code), (msg));      \
     } while (0)
 
-// Gives back the idle MSM workspaces that contexts keep (KeptWorkspace,
-// msm.hpp): they count as free memory. Called where an allocation failed,
-// before it is tried again, and by free_device_bytes().
-void release_idle_workspaces();
+// Gives back the idle MSM workspaces that contexts on a device (-1: on any) keep
+// (KeptWorkspace, msm.hpp). Freeing waits for the device's work in flight, so it
+// is done only where their memory is needed: an allocation failed
+// (device_malloc), or bytes asked for are not free (device_bytes_fit).
+void release_idle_workspaces(int device = -1);
+// bytes that they hold
+size_t idle_workspace_bytes(int device = -1);
 
 // hipMalloc that takes back idle workspaces before it gives up
 inline hipError_t device_malloc(void** p, size_t n) {
     hipError_t e = hipMalloc(p, n);
     if (e != hipErrorOutOfMemory) return e;
     (void)hipGetLastError();
-    release_idle_workspaces();
+    int dev = -1;
+    (void)hipGetDevice(&dev);
+    release_idle_workspaces(dev);
     return hipMalloc(p, n);
 }
 
-// free and total bytes of the current device
-inline void free_device_bytes(size_t* free_b, size_t* total_b) {
-    release_idle_workspaces();
-    ZK_HIP(hipMemGetInfo(free_b, total_b));
+// free bytes of the current device, idle workspaces not counted
+inline size_t free_device_bytes() {
+    size_t free_b = 0, total_b = 0;
+    ZK_HIP(hipMemGetInfo(&free_b, &total_b));
+    return free_b;
+}
+
+// Whether `need` bytes are free on the current device, where free_b were at the
+// last look. Idle workspaces count as free: they are given back when that, and
+// only that, makes room.
+inline bool device_bytes_fit(size_t& free_b, size_t need) {
+    if (free_b >= need) return true;
+    int dev = -1;
+    ZK_HIP(hipGetDevice(&dev));
+    if (free_b + idle_workspace_bytes(dev) < need) return false;
+    release_idle_workspaces(dev);
+    free_b = free_device_bytes();
+    return free_b >= need;
 }
 
 // Device allocation: owning (hipMalloc), or borrowed from memory the caller

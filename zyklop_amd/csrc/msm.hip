@@ -752,7 +752,7 @@ static std::vector<KeptWorkspace*>& workspaces() {
     return v;
 }
 
-KeptWorkspace::KeptWorkspace() {
+KeptWorkspace::KeptWorkspace(int dev) : device(dev) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     workspaces().push_back(this);
 }
@@ -784,16 +784,26 @@ WorkspaceUse::~WorkspaceUse() {
     if (failed) (void)hipStreamSynchronize(st);
     if (!kept) return;
     if (failed || kept->bytes() > MSM_KEEP_BYTES) kept->release();
+    kept->held = kept->bytes();
     kept->busy = false;
 }
 
-void release_idle_workspaces() {
+void release_idle_workspaces(int device) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     for (KeptWorkspace* w : workspaces()) {
-        if (w->busy.exchange(true)) continue;
+        if ((device >= 0 && w->device != device) || w->busy.exchange(true)) continue;
         w->release();
+        w->held = 0;
         w->busy = false;
     }
+}
+
+size_t idle_workspace_bytes(int device) {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    size_t b = 0;
+    for (const KeptWorkspace* w : workspaces())
+        if ((device < 0 || w->device == device) && !w->busy) b += w->held;
+    return b;
 }
 
 template <class S, class F>

@@ -172,14 +172,16 @@ struct MsmWorkspace {
 // it took up to as long as the MSM (G1 calls of 2^22 points 8.5 -> 6.2 ms, of
 // 700001 4.4 -> 1.9, of 1000 0.61 -> 0.54; G2 of 200003 2.9 -> 1.9). A context
 // keeps at most MSM_KEEP_BYTES of device memory (enough for 2^22 G1 points); a
-// larger workspace is freed when its call ends, an idle one when an allocation of
-// the library fails, when free memory is asked for, and with its context.
-// release_idle_workspaces() finds the kept ones, and only them. busy: in use by a
-// call, or being released; whoever sets it owns the buffers until it is cleared.
+// larger workspace is freed when its call ends, an idle one when the library needs
+// its memory (common.hpp), and with its context. release_idle_workspaces() finds
+// the kept ones, and only them. busy: in use by a call, or being released; whoever
+// sets it owns the buffers until it is cleared. held: device bytes while idle.
 constexpr size_t MSM_KEEP_BYTES = (size_t)2 << 30;
 struct KeptWorkspace : MsmWorkspace {
+    const int device;
     std::atomic<bool> busy{false};
-    KeptWorkspace();
+    std::atomic<size_t> held{0};
+    explicit KeptWorkspace(int device = 0);
     ~KeptWorkspace();
 };
 

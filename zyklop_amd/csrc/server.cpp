@@ -50,7 +50,7 @@ uint64_t Server::admit_request(std::shared_ptr<ServerRequest> req, const Circuit
     if (s) memcpy(req->s, s, 32);
     ZK_REQUIRE(zkh::Fr::is_canonical(req->r) && zkh::Fr::is_canonical(req->s), ZK_E_ARG, "blinding must be canonical");
     size_t free_b = 0, total_b = 0;
-    free_device_bytes(&free_b, &total_b);
+    ZK_HIP(hipMemGetInfo(&free_b, &total_b));
     size_t need;
     {
         std::lock_guard<std::mutex> g(ctx_.mu);
@@ -96,16 +96,14 @@ int Server::prepare(const Circuit* const* cs, int count) {
         if (k == (int)slots_.size()) {
             size_t need = 0;
             for (const Circuit* c : order) need = std::max(need, ProveSlot::bytes_needed(ctx_, *c));
-            size_t free_b = 0, total_b = 0;
-            free_device_bytes(&free_b, &total_b);
-            if (k > 0 && free_b < need + reserve_) break;
+            size_t free_b = free_device_bytes();
+            if (k > 0 && !device_bytes_fit(free_b, need + reserve_)) break;
             slots_.push_back(std::make_unique<ProveSlot>());
             running_.push_back(nullptr);
         }
         for (const Circuit* c : order) {
-            size_t free_b = 0, total_b = 0;
-            free_device_bytes(&free_b, &total_b);
-            ZK_REQUIRE(free_b >= slots_[k]->grow_bytes(ctx_, *c) + reserve_, ZK_E_NOMEM,
+            size_t free_b = free_device_bytes();
+            ZK_REQUIRE(device_bytes_fit(free_b, slots_[k]->grow_bytes(ctx_, *c) + reserve_), ZK_E_NOMEM,
                        "not enough free device memory to prepare a slot above the reserve");
             slots_[k]->reserve(ctx_, *c, true);
         }
@@ -210,20 +208,19 @@ bool Server::try_admit(std::unique_lock<std::mutex>& lk) {
         for (size_t i = 0; i < slots_.size() && pick < 0; i++)
             if (!running_[i] && grow(i) == 0) pick = (int)i;
         if (pick < 0) {
-            size_t free_b = 0, total_b = 0;
-            free_device_bytes(&free_b, &total_b);
+            size_t free_b = free_device_bytes();
             size_t need;
             {
                 std::lock_guard<std::mutex> g(ctx_.mu);
                 need = ProveSlot::bytes_needed(ctx_, *req->circ);
             }
-            if ((int)slots_.size() < max_slots_ && free_b >= need + reserve_) {
+            if ((int)slots_.size() < max_slots_ && device_bytes_fit(free_b, need + reserve_)) {
                 slots_.push_back(std::make_unique<ProveSlot>());
                 running_.push_back(nullptr);
                 pick = (int)slots_.size() - 1;
             }
             for (size_t i = 0; i < slots_.size() && pick < 0; i++)
-                if (!running_[i] && free_b >= grow(i) + reserve_) pick = (int)i;
+                if (!running_[i] && device_bytes_fit(free_b, grow(i) + reserve_)) pick = (int)i;
         }
         if (pick < 0) break;  // wait for a slot or for memory
         queue_.erase(qi);
