@@ -111,3 +111,24 @@ int main() {
 }
 """)
     assert out == "ok"
+
+
+def test_context_may_outlive_the_librarys_statics(tmp_path):
+    """A program that frees its context in an exit handler it registered before
+    its first use of the library: the list of kept workspaces is still there
+    (freed memory is overwritten, so a list that is gone shows)."""
+    os.environ["MALLOC_PERTURB_"] = "165"
+    try:
+        out = run(tmp_path, r"""
+#include <cstdlib>
+static zk::KeptWorkspace *a, *b;
+int main() {
+    atexit([] { delete a; zk::release_idle_workspaces(); delete b; printf("ok"); });
+    a = new zk::KeptWorkspace;
+    b = new zk::KeptWorkspace;
+    return 0;
+}
+""")
+    finally:
+        del os.environ["MALLOC_PERTURB_"]
+    assert out == "ok"

@@ -747,9 +747,11 @@ size_t MsmScratch::bytes() const {
 
 // ---------------------------------------------------------------- workspaces
 static std::mutex g_ws_mu;
+// never destroyed: a program may free its contexts in exit handlers that run
+// after the library's own
 static std::vector<KeptWorkspace*>& workspaces() {
-    static std::vector<KeptWorkspace*> v;
-    return v;
+    static auto* v = new std::vector<KeptWorkspace*>;
+    return *v;
 }
 
 KeptWorkspace::KeptWorkspace(int dev) : device(dev) {
