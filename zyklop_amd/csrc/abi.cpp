@@ -149,19 +149,17 @@ void put_result(const zkh::Xyzz<HT>& p, uint64_t* out, int* is_inf) {
 // already made (a circuit's resident arrays, W window tables when merged)
 // cls / range: scalar classes and the part of every bucket to read, as a
 // proof's witness MSMs do (MsmSort::run, msm_launch_main); split: threads per
-// bucket, 0 for msm_default_split
-void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t n, int window, bool g2, uint64_t* out,
-                int* is_inf, const void* slots29 = nullptr, bool merged = false, const uint8_t* cls = nullptr,
-                int range = zk::MSM_RANGE_ALL, int split = 0) {
+// bucket
+void msm_run(zk_ctx* ctx, zk::MsmWorkspace& w, const void* d_points, const void* d_scalars, size_t n, int window, bool g2,
+             uint64_t* out, int* is_inf, const void* slots29, bool merged, const uint8_t* cls, int range, int split) {
     zk::Context& C = ctx->impl;
     hipStream_t st = C.stream;
-    zk::WorkspaceUse use(ctx->msm_ws, st);
-    zk::MsmSort& sort = use.w->sort;
-    zk::MsmScratch& scr = use.w->scr;
-    zk::MsmPartials& part = use.w->part;
+    zk::MsmSort& sort = w.sort;
+    zk::MsmScratch& scr = w.scr;
+    zk::MsmPartials& part = w.part;
     scr.enable_timing();
     // buckets are accumulated in the 29-bit-limb form: convert the points first
-    zk::DevBuf& p29 = use.w->p29;
+    zk::DevBuf& p29 = w.p29;
     if (n && !slots29) {
         p29.ensure(n * (g2 ? zk::PT29Q_BYTES : zk::PT29_BYTES));
         zk::msm_points_to29(d_points, n, p29.p, g2, st);
@@ -170,18 +168,18 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
     sort.run(d_scalars, n, window, st, merged, cls);
     ZK_HIP(hipEventRecord(ctx->ev1, st));
     const void* pts = slots29 ? slots29 : p29.p;
-    zk::msm_launch(sort, g2, {pts, &scr, &part, range}, st, split > 0 ? split : zk::msm_alone_split(n, sort.g.c, g2));
+    zk::msm_launch(sort, g2, {pts, &scr, &part, range}, st, split);
     ZK_HIP(hipEventRecord(ctx->ev2, st));
     const size_t nb = (size_t)sort.g.Wr * sort.g.K;
-    use.w->entries.ensure(4);
-    ZK_HIP(hipMemcpyAsync(use.w->entries.p, sort.offsets.as<uint32_t>() + nb, 4, hipMemcpyDeviceToHost, st));
+    w.entries.ensure(4);
+    ZK_HIP(hipMemcpyAsync(w.entries.p, sort.offsets.as<uint32_t>() + nb, 4, hipMemcpyDeviceToHost, st));
     ZK_HIP(hipStreamSynchronize(st));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[0], ctx->ev0, ctx->ev2));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[1], ctx->ev0, ctx->ev1));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[2], scr.ev_acc0, scr.ev_acc1));
     ZK_HIP(hipEventElapsedTime(&ctx->last_ms[4], scr.ev_acc1, scr.ev_end));
     // entries the accumulation read: the sort's, or the parts of the range
-    uint32_t entries = *use.w->entries.as<uint32_t>();
+    uint32_t entries = *w.entries.as<uint32_t>();
     if (sort.classes && range != zk::MSM_RANGE_ALL) {
         std::vector<uint32_t> off(nb + 1), co(3 * nb);
         ZK_HIP(hipMemcpy(off.data(), sort.offsets.p, 4 * (nb + 1), hipMemcpyDeviceToHost));
@@ -193,6 +191,27 @@ void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t
     ctx->last_ms[3] = (float)entries;
     if (g2) put_result(zk::msm_finish_g2(part), out, is_inf);
     else put_result(zk::msm_finish_g1(part), out, is_inf);
+}
+
+// msm_run in the context's workspace; split 0: msm_alone_split. Where device memory
+// is short, what an earlier call of another shape left in the workspace makes way,
+// and the parts of a bucket are msm_default_split's: a call must not be refused for
+// what its context keeps or for threads it only takes because it is alone.
+void msm_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t n, int window, bool g2, uint64_t* out,
+                int* is_inf, const void* slots29 = nullptr, bool merged = false, const uint8_t* cls = nullptr,
+                int range = zk::MSM_RANGE_ALL, int split = 0) {
+    zk::WorkspaceUse use(ctx->msm_ws, ctx->impl.stream);
+    const int alone = split > 0 ? split : zk::msm_alone_split(n, window, g2);
+    const bool kept = use.w->bytes() > 0;
+    try {
+        return msm_run(ctx, *use.w, d_points, d_scalars, n, window, g2, out, is_inf, slots29, merged, cls, range, alone);
+    } catch (const zk::Error& e) {
+        if (split <= 0) split = zk::msm_default_split(n, window, g2);
+        if (e.code != ZK_E_NOMEM || (!kept && split == alone)) throw;
+    }
+    ZK_HIP(hipStreamSynchronize(ctx->impl.stream));
+    use.w->release();
+    msm_run(ctx, *use.w, d_points, d_scalars, n, window, g2, out, is_inf, slots29, merged, cls, range, split);
 }
 
 void ntt_device(zk_ctx* ctx, void* const* in, void* const* out, int batch, int log_n, int kind) {
