@@ -262,7 +262,10 @@ int zk_dev_copy(zk_ctx* ctx, void* dst, const void* src, size_t bytes);
 int zk_ntt_device(zk_ctx* ctx, void* const* d_in, void* const* d_out, int batch, int log_n, int kind);
 /* The MSM entry points keep their device workspace on ctx from call to call, up
  * to 2 GiB (2^22 G1 points); it is freed with ctx, or earlier when the library
- * needs the memory. */
+ * needs the memory, or by zk_msm_free_workspace: for programs whose other
+ * allocators share the GPU. That call waits for a running one; the next MSM
+ * allocates again. */
+int zk_msm_free_workspace(zk_ctx* ctx);
 int zk_msm_g1_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t n, int window, uint64_t out[8],
                      int* is_inf);
 int zk_msm_g2_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t n, int window, uint64_t out[16],

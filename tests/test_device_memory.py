@@ -89,3 +89,28 @@ int main() {
 }
 """)
     assert out == "ok"
+
+
+def test_workspace_is_given_back_on_request(tmp_path):
+    """Memory that a context keeps can be had back by a program whose other
+    allocators share the device; the next call allocates again."""
+    out = run(tmp_path, r"""
+int main() {
+    static char pts[64], sc[64];
+    uint64_t out[8];
+    int inf = 0;
+    zk_ctx* c = nullptr;
+    if (zk_ctx_create(0, &c)) return 2;
+    const size_t base = host_hip::used;
+    for (int i = 0; i < 2; i++) {
+        if (zk_msm_g1_device(c, pts, sc, 5000, 0, out, &inf)) return 3;
+        if (host_hip::used == base) { printf("nothing kept"); return 0; }
+        if (zk_msm_free_workspace(c) || host_hip::used != base) { printf("not given back"); return 0; }
+    }
+    if (zk_msm_free_workspace(c) || zk_msm_free_workspace(nullptr) != ZK_E_ARG) return 4;
+    zk_ctx_destroy(c);
+    printf("ok");
+    return 0;
+}
+""")
+    assert out == "ok"

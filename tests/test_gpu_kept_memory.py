@@ -1,6 +1,7 @@
 """What becomes of the device memory of the workspace that a context keeps
 between MSM calls, seen from outside (free device bytes) and by results."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -89,3 +90,25 @@ def test_admission_takes_the_workspace_where_it_makes_room(kept):
     srv.close()
     assert np.array_equal(pr.words(), kept.ctx.prove(kept.small, w).words())
     assert kept.allocated_by_msm() > kept.held // 4
+
+
+def test_workspace_given_back_under_a_running_thread(kept):
+    """zk_msm_free_workspace gives the memory back; called over and over while
+    another thread runs MSMs on the same context it changes no result."""
+    before = free_bytes()
+    kept.ctx.free_msm_workspace()
+    assert free_bytes() - before > kept.held // 2
+    bad = []
+
+    def work():
+        for _ in range(20):
+            got = kept.msm()
+            if got[1] != kept.out[1] or not np.array_equal(got[0], kept.out[0]):
+                bad.append(got)
+
+    t = threading.Thread(target=work)
+    t.start()
+    while t.is_alive():
+        kept.ctx.free_msm_workspace()
+    t.join()
+    assert not bad

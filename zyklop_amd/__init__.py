@@ -112,6 +112,7 @@ ABI = {
     "zk_dev_copy": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_size_t]),
     "zk_ntt_device": (ctypes.c_int, [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.c_int, ctypes.c_int,
                                      ctypes.c_int]),
+    "zk_msm_free_workspace": (ctypes.c_int, [_vp]),
     "zk_msm_g1_device": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_size_t, ctypes.c_int, _u64p,
                                         ctypes.POINTER(ctypes.c_int)]),
     "zk_msm_g2_device": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_size_t, ctypes.c_int, _u64p,
@@ -297,6 +298,10 @@ class Context:
         inf = ctypes.c_int(0)
         _check(lib().zk_msm_g1_device(self.h, d_points, d_scalars, n, window, u64p(out), ctypes.byref(inf)))
         return out, bool(inf.value)
+
+    def free_msm_workspace(self):
+        """Free the device memory that MSM calls keep on the context for the next ones."""
+        _check(lib().zk_msm_free_workspace(self.h))
 
     def circuit_msm_device(self, circuit, which, d_scalars, window=0):
         """MSM over a circuit's resident base array (0 A', 1 B1', 2 B2' (G2), 3 C', 4 H) through

@@ -753,6 +753,15 @@ int zk_msm_g2(zk_ctx* ctx, const uint64_t* points, const uint64_t* scalars, size
     return msm_host(ctx, points, scalars, n, window, true, out, is_inf);
 }
 
+int zk_msm_free_workspace(zk_ctx* ctx) {
+    return guard([&] {
+        need(ctx != nullptr, "NULL ctx");
+        std::lock_guard<std::mutex> lk(ctx->impl.mu);
+        ZK_HIP(hipSetDevice(ctx->impl.device));
+        ctx->msm_ws.take_back();
+    });
+}
+
 int zk_msm_g1_device(zk_ctx* ctx, const void* d_points, const void* d_scalars, size_t n, int window, uint64_t out[8],
                      int* is_inf) {
     return guard([&] {

@@ -790,14 +790,17 @@ WorkspaceUse::~WorkspaceUse() {
     kept->busy = false;
 }
 
+void KeptWorkspace::take_back() {
+    if (busy.exchange(true)) return;
+    release();
+    held = 0;
+    busy = false;
+}
+
 void release_idle_workspaces(int device) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    for (KeptWorkspace* w : workspaces()) {
-        if ((device >= 0 && w->device != device) || w->busy.exchange(true)) continue;
-        w->release();
-        w->held = 0;
-        w->busy = false;
-    }
+    for (KeptWorkspace* w : workspaces())
+        if (device < 0 || w->device == device) w->take_back();
 }
 
 size_t idle_workspace_bytes(int device) {

@@ -173,7 +173,7 @@ struct MsmWorkspace {
 // 700001 4.4 -> 1.9, of 1000 0.61 -> 0.54; G2 of 200003 2.9 -> 1.9). A context
 // keeps at most MSM_KEEP_BYTES of device memory (enough for 2^22 G1 points); a
 // larger workspace is freed when its call ends, an idle one when the library needs
-// its memory (common.hpp), and with its context. release_idle_workspaces() finds
+// its memory (common.hpp), when the caller asks for it, and with its context. release_idle_workspaces() finds
 // the kept ones, and only them. busy: in use by a call, or being released; whoever
 // sets it owns the buffers until it is cleared. held: device bytes while idle.
 constexpr size_t MSM_KEEP_BYTES = (size_t)2 << 30;
@@ -183,6 +183,7 @@ struct KeptWorkspace : MsmWorkspace {
     std::atomic<size_t> held{0};
     explicit KeptWorkspace(int device = 0);
     ~KeptWorkspace();
+    void take_back();   // frees the buffers unless in use
 };
 
 // The kept workspace for one call, or while another thread takes it back one of
