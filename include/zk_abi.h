@@ -111,7 +111,8 @@ int zk_circuit_window_tables(zk_ctx* ctx, zk_circuit* c, int mode, int windows[2
  * compile-time constant, include/msm_g1.cuh:11). For circuit c it measures on
  * the device, over c's resident bases and uniform scalars, the digit sort plus
  * the MSMs that share it, for one window per window count in [11, 19] around
- * the size (at most ceil(log2 n) - 2) and every bucket split 1..4: kind 0 =
+ * the size (at most ceil(log2 n) - 2) and every bucket split 1..4 (only the
+ * default, recorded as 0, where that is larger): kind 0 =
  * the witness sort over n_vars + 4 scalars and the A', B1', C' (G1) and B2'
  * (G2) MSMs; kind 1 = the sort of h and the H MSM (n scalars). The fastest
  * window, with its G1 and G2 splits, is recorded per (kind, ceil log2 n) in

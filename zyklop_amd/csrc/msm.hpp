@@ -208,7 +208,7 @@ struct WorkspaceUse {
 // a consecutive part of the bucket's entries; the reduction adds the parts.
 // More threads than buckets fill the GPU when the buckets are few.
 constexpr int MSM_SPLIT_MAX = 64;
-constexpr int MSM_SPLIT_TUNE = 4;   // largest split the autotuner tries and its tables hold
+constexpr int MSM_SPLIT_TUNE = 4;   // largest split a tuning table holds; the autotuner tries these
 // of a proof's MSMs: about two rounds of resident waves on a 256-CU GPU at most
 // 3 parts, more for few buckets
 int msm_default_split(size_t n, int c, bool g2, bool merged = false);

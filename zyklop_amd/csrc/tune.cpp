@@ -8,7 +8,10 @@
 // on the context stream over the circuit's resident bases and uniform
 // scalars, timed with HIP events. A candidate's cost is the sort plus, per
 // MSM, its fastest split; the cheapest c is recorded for (kind, ceil log2 n)
-// with its G1 and G2 splits. Two kinds:
+// with its G1 and G2 splits. Where the buckets are so few that the default takes
+// more parts than are tried, the default stays (split 0): it was measured in whole
+// proofs (msm_default_split), and a tuned split of 4 lost what it gives (proofs of
+// 5000 constraints over window tables). Two kinds:
 //   kind 0: the witness sort over n_vars + 4 scalars and its four MSMs
 //           (A', B1', C' in G1, B2' in G2), the cost one proof pays for c_w;
 //   kind 1: the sort of h over n scalars and the H MSM (c_h).
@@ -112,7 +115,8 @@ float elapsed(TuneBufs& tb) {
 
 // Device ms at window c, mean over reps after one warm-up: the sort, and each
 // MSM of `kind` at each split 1..MSM_SPLIT_TUNE (msm[m][split-1]; splits that
-// would start more than 2^21 threads are skipped and left at -1).
+// would start more than 2^21 threads are skipped and left at -1), or at the
+// default split alone (msm[m][0]) where that is larger.
 void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged, const void* d_sc, size_t n,
                  int reps, TuneBufs& tb, float& sort_ms, float msm[4][MSM_SPLIT_TUNE]) {
     hipStream_t st = ctx.stream;
@@ -135,16 +139,19 @@ void time_window(Context& ctx, const Circuit& circ, int kind, int c, bool merged
         ZK_HIP(hipEventRecord(tb.e1, st));
         const float t_sort = elapsed(tb);
         if (it > 0) sort_ms += t_sort / reps;
-        for (int m = 0; m < nm; m++)
-            for (int s = 1; s <= MSM_SPLIT_TUNE; s++) {
+        for (int m = 0; m < nm; m++) {
+            const int dflt = msm_default_split(n, c, ms[m].g2, merged);
+            const bool beyond = dflt > MSM_SPLIT_TUNE;
+            for (int s = 1; s <= (beyond ? 1 : MSM_SPLIT_TUNE); s++) {
                 if ((size_t)g.Wr * g.K * s > ((size_t)1 << 21) && s > 1) continue;
                 ZK_HIP(hipEventRecord(tb.e0, st));
                 MsmScratch& scr = ms[m].g2 ? tb.g2 : tb.g1;
-                msm_launch(tb.sort, ms[m].g2, {ms[m].p29, &scr, &tb.part, ms[m].range}, st, s);
+                msm_launch(tb.sort, ms[m].g2, {ms[m].p29, &scr, &tb.part, ms[m].range}, st, beyond ? dflt : s);
                 ZK_HIP(hipEventRecord(tb.e1, st));
                 const float t = elapsed(tb);
                 if (it > 0) msm[m][s - 1] = (msm[m][s - 1] < 0 ? 0 : msm[m][s - 1]) + t / reps;
             }
+        }
     }
 }
 
@@ -205,6 +212,8 @@ void Context::autotune(const Circuit& circ, bool force, int reps, int chosen[2])
                 int g1 = sp[0];
                 if (kind == 0 && sp[1] == sp[2]) g1 = sp[1];
                 best = {c, g1, kind == 0 ? sp[3] : 1};
+                if (msm_default_split(n, c, false, tc != 0) > MSM_SPLIT_TUNE) best.split_g1 = 0;
+                if (msm_default_split(n, c, true, tc != 0) > MSM_SPLIT_TUNE) best.split_g2 = 0;
             }
         }
         tuned[key] = best;
