@@ -32,7 +32,7 @@ int msm_default_split(size_t n, int c, bool g2, bool merged) {
     const MsmGeom g = msm_geom(n, c, g2, merged);
     // two rounds of waves at 6 (G1) and 3 (G2) waves per SIMD, i.e. three
     // and two rounds at the 4 and 2 the accumulation kernels hold (128 VGPRs;
-    // 228 VGPRs and LDS); the autotuner picks the splits of a circuit's sizes
+    // 172 VGPRs and LDS); the autotuner picks the splits of a circuit's sizes
     const size_t target = (size_t)1024 * 64 * 2 * (g2 ? 3 : 6);
     const size_t nb = (size_t)g.Wr * g.K, load = 2 * n * (size_t)g.W / nb;
     // Few buckets: up to half a wave per SIMD for each of a proof's MSMs, while a

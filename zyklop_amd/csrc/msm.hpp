@@ -146,7 +146,6 @@ struct MsmPartials {
 struct MsmScratch {
     DevBuf buckets, seg, node0, node1, partials;
     int split = 0;     // threads per bucket of the queued MSM (set by msm_launch_pre)
-    size_t cap_buckets = 0;
     // optional events around the bucket-accumulation kernel (profiling)
     hipEvent_t ev_acc0 = nullptr, ev_acc1 = nullptr, ev_end = nullptr;
     void enable_timing();

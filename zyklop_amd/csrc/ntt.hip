@@ -109,7 +109,7 @@ ZK_DEV NttUnit ntt_unit(const NttShape& z, size_t u) {
     }
     return {row << Q, 1, u, z.n >> Q, 0};
 }
-// output k of a unit, x with limbs below 1.5 * 2^30 and value below 20r: scaled,
+// output k of a unit, x with limbs below 2.5 * 2^30 and value below 20r: scaled,
 // then stored. Apart, so that the scaling loads of all outputs come before any
 // store, which they could not pass.
 ZK_DEV F29 ntt_scale(const NttShape& z, const NttUnit& t, uint32_t k, const F29& x) {
@@ -225,8 +225,9 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_lane(NttPtrs ptrs, NttShape
 // instruction per limb for both points), then 1, 0 (DPP in a quad); 3, 2 only
 // in units of 2^7 points and more. The bits left over number the wave's units.
 // Bound by instruction issue: 5044 VALU instructions per lane for 2^8 points per
-// unit (3336 for 2^6), 60 % of them v_mad_u64_u32, which alone take 0.38 ms of the
-// 2^22 transform. Four waves per SIMD (five are the same, six spill 12 %). The
+// unit (3336 for 2^6), 60 % of them v_mad_u64_u32: 14.1 G lane instructions for the
+// 2^22 transform, 0.38 ms at the 37 T/s of its mix, 0.25 ms of them the multiplies
+// (34 T/s). Four waves per SIMD (five are the same, six spill 12 %). The
 // radix-8 threads before took four launches (call 617 us, now 488); eight points
 // per lane with the same exchange held three waves per SIMD and 563 us. Products
 // with a stored b' = floor(b 2^261 / r) instead of Montgomery's: the same time.

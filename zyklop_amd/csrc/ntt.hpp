@@ -5,10 +5,11 @@
 // Every pass transforms units of R_j points, column c of a block of M = R_j*S
 // points, in the registers of a group of lanes of one wave: radix-2 butterflies
 // with two points per lane (n up to about 2^19) or radix-4 with four, the points
-// moving between lanes by v_permlane*_swap and DPP, with no LDS and no barrier.
-// A pass then multiplies by the inter-pass twiddle w_M^(c k) from a precomputed
-// [k][c] table and stores, not made canonical between passes. Passes 0..p-2 run
-// in place; the last pass writes the digit-reversed (natural) order out of place.
+// moving between lanes by v_permlane*_swap and DPP instead of through LDS (only the
+// four-point kernel's roots are staged there). A pass then multiplies by the
+// inter-pass twiddle w_M^(c k) from a precomputed [k][c] table and stores, not made
+// canonical between passes. Passes 0..p-2 run in place; the last pass writes the
+// digit-reversed (natural) order out of place.
 // An optional element-wise table multiplies the input (first pass) or the output
 // (last pass): that is how the coset shift and n^-1 are fused instead of
 // separate element-wise passes (src/groth16.cu:914-921, 1066-1076).
